@@ -25,7 +25,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wno-unus
           "-Wno-unknown-pragmas"]
 DEVICE = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 SOURCES = ["sxc_kernels.hip", "sxc_kernels_r2.hip", "sxc_kernels_s32.hip", "sxc_kernels_occ.hip", "sxc_kernels_lean.hip",
-           "sxc_api.hip",
+           "sxc_scan_pure.hip", "sxc_scan_n.hip", "sxc_scan_general.hip", "sxc_api.hip",
            "sxc_server.hip", "sxc_static.hip", "sxc_tables.cpp", "sxc_kmatch.hip",
            # the master's side of the search (host C++): match sets, chaining, grid search
            "sxc_master_api.cpp", "host/sxc_master.cpp", "host/sxc_seqio.cpp"]

@@ -162,6 +162,8 @@ int launch_correlate(sxc_ctx* ctx, sxc_batch_dev& b) {
   a.cutoff_fast = b.prm.cutoff_fast;
   a.cands = b.cands.as<uint16_t>();
   a.ncand = b.ncand.as<int32_t>();
+  a.counts = b.counts.as<int32_t>();
+  a.stats = b.stats.as<int32_t>();
   a.xc_out = nullptr;
   if (!b.hb.tails.empty()) {
     a.tails = b.tails.as<sxc_tail_dev>();
@@ -172,7 +174,8 @@ int launch_correlate(sxc_ctx* ctx, sxc_batch_dev& b) {
   return SXC_OK;
 }
 
-int launch_pairs(sxc_ctx* ctx, sxc_batch_dev& b) {
+// fresh: the pair kernel has just cleared the counts (the scan may split small launches).
+int launch_pairs(sxc_ctx* ctx, sxc_batch_dev& b, bool fresh) {
   const int total = (int)b.hb.pairs.size() * b.prm.strands;
   sxc::ScanArgs a{};
   a.tab = ctx->d_tab;
@@ -199,7 +202,7 @@ int launch_pairs(sxc_ctx* ctx, sxc_batch_dev& b) {
     a.ptable = b.ptable;
     a.table_prob = b.prm.table_prob;
   }
-  HIPCHK(sxc::launch_scan(b.nb, a, total, b.s));
+  HIPCHK(sxc::launch_scan(b.nb, a, total, b.kinds, fresh, b.s));
   return SXC_OK;
 }
 
@@ -254,7 +257,7 @@ int batch_enqueue(sxc_ctx* ctx, sxc_batch_dev& b, bool events) {
   rc = launch_correlate(ctx, b);
   if (rc) return rc;
   if (events) HIPCHK(hipEventRecord(b.ev[2], s));
-  rc = launch_pairs(ctx, b);
+  rc = launch_pairs(ctx, b, true);
   if (rc) return rc;
   if (events) HIPCHK(hipEventRecord(b.ev[3], s));
   HIPCHK(sxc::launch_count_offsets(b.counts.as<int32_t>(), total, b.slot_cap, b.offsets.as<int64_t>(),
@@ -405,7 +408,7 @@ int batch_end(sxc_ctx* ctx, sxc_batch_dev& b) {
     b.slot_cap = maxc;
     int rc = batch_alloc(ctx, b);
     if (rc) return rc;
-    rc = launch_pairs(ctx, b);
+    rc = launch_pairs(ctx, b, false);
     if (rc) return rc;
     HIPCHK(sxc::launch_count_offsets(b.counts.as<int32_t>(), total, b.slot_cap, b.offsets.as<int64_t>(),
                                      b.total.as<int64_t>(), b.maxc.as<int32_t>(), s, b.nflag.as<int32_t>()));
@@ -450,6 +453,9 @@ int batch_prepare(sxc_batch_dev& b, const sxc_pair* pairs, int32_t n, const sxc_
   if (rc) return rc;
   std::string e = sxc::pack_batch(pairs, n, prm->N, b.hb, t_tail, q_tail);
   if (!e.empty()) return fail(SXC_ERR_ARG, e);
+  b.kinds = sxc::ScanKinds();
+  for (const sxc_pair_dev& p : b.hb.pairs)
+    ++b.kinds.pairs[sxc::scan_kind(b.hb.tchunks[(size_t)p.t_chunk].flags, b.hb.qchunks[(size_t)p.q_chunk].flags)];
   b.prm = *prm;
   b.nb = nb;
   b.slot_cap = 64;  // records per (pair, strand) a run first makes room for; grows on overflow
@@ -1240,7 +1246,9 @@ int sxc_matchup(sxc_ctx* ctx, const char* q, int32_t lq, const char* t, int32_t 
   a.keys = ctx->p4.as<uint64_t>();
   a.counts = d_misc + 1;
   a.cap = slot;
-  HIPCHK(sxc::launch_scan(nb, a, 1, s));
+  sxc::ScanKinds kinds;
+  kinds.pairs[sxc::scan_kind(hb.tchunks[0].flags, hb.qchunks[0].flags)] = 1;
+  HIPCHK(sxc::launch_scan(nb, a, 1, kinds, false, s));
   int32_t cnt = 0;
   HIPCHK(hipMemcpyAsync(&cnt, d_misc + 1, sizeof cnt, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));

@@ -10,6 +10,7 @@
 
 #include "../../include/sxc.h"
 #include "sxc_batch_host.h"
+#include "sxc_kernels.h"
 #include "sxc_types.h"
 
 namespace sxc {
@@ -62,6 +63,7 @@ struct sxc_batch_dev {
   DevBuf ent;    // host-computed window entropies of chunks with B/D/H/V letters
   DevBuf nflag;  // records the last scan flagged near min_prob (the counts kernel reads and clears it)
   sxc::HostBatch hb;
+  sxc::ScanKinds kinds;  // of hb.pairs
   sxc_params prm{};
   int nb = 0;
   int slot_cap = 64;

@@ -11,31 +11,6 @@
 
 namespace sxc {
 
-struct NoRegs {};
-
-// The pure-A/C/G/T scan kernel gets a register budget for as many of its 4-wave
-// workgroups per CU as its LDS plan admits, up to 8 waves per SIMD (measured on the 4096-pair
-// workload at N = 8192 with byte-parallel flags: 5 waves 1.05 ms, 6: 1.00 ms, 7: 0.94 ms,
-// 8: 0.93 ms; the spills the budget costs are cheaper than the latency the extra waves hide).
-template <int NB>
-constexpr int scan_waves() {
-  if constexpr (!ScanSmem<NB>::PURE) {
-    return 1;
-  } else {
-    constexpr int wg = 163840 / ScanSmem<NB>::BYTES;
-    return wg < 1 ? 1 : (wg > 8 ? 8 : wg);
-  }
-}
-static_assert(scan_waves<13 | 32>() == 8, "the pure scan's LDS plan at N = 8192 fits 8 workgroups per CU");
-
-template <int NB>
-__global__ __launch_bounds__(SCAN_NT) __attribute__((amdgpu_waves_per_eu(scan_waves<NB>()))) void k_scan(ScanArgs a) {
-  __shared__ __align__(16) char sm[ScanSmem<NB>::BYTES];
-  NoRegs r;
-  DevExec<NoRegs> ex{r};
-  scan_body<NB>(ex, sm, a, (int)blockIdx.x);
-}
-
 template <int NB>
 __global__ __launch_bounds__(Geo<NB>::NT) void k_peaks(const float* xc, double cutoff, uint16_t* cands,
                                                      int32_t* ncand) {
@@ -104,14 +79,16 @@ __global__ void k_prob(ProbArgs a) {
 
 // Exclusive scan of per-(pair, strand) kept counts (clipped to cap) -> offsets, total.
 // With nflag: total[1] receives the scan's count of records flagged near min_prob, and the
-// counter is cleared for the next scan.
+// counter is cleared for the next scan.  One workgroup, bound by latency: each thread sums a
+// contiguous share, the shares are scanned by lane shuffles within a wave and across the 16
+// waves through LDS.
 __global__ __launch_bounds__(1024) void k_scan_counts(const int32_t* counts, int n, int cap, int64_t* offsets,
                                                       int64_t* total, int32_t* max_count, int32_t* nflag) {
-  __shared__ int64_t part[1024];
-  __shared__ int mx[1024];
-  const int t = threadIdx.x;
+  __shared__ int64_t wsum[16];
+  __shared__ int wmax[16];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int per = (n + 1023) / 1024;
-  const int b = t * per, e = (b + per < n) ? b + per : n;
+  const int b = t * per < n ? t * per : n, e = (b + per < n) ? b + per : n;
   int64_t s = 0;
   int m = 0;
   for (int i = b; i < e; ++i) {
@@ -119,27 +96,30 @@ __global__ __launch_bounds__(1024) void k_scan_counts(const int32_t* counts, int
     s += c < cap ? c : cap;
     m = c > m ? c : m;
   }
-  part[t] = s;
-  mx[t] = m;
+  int64_t inc = s;  // inclusive over the wave's lanes
+  for (int d = 1; d < 64; d <<= 1) {
+    const int64_t v = __shfl_up(inc, d, 64);
+    const int v2 = __shfl_xor(m, d, 64);
+    if (lane >= d) inc += v;
+    m = v2 > m ? v2 : m;
+  }
+  if (lane == 63) {
+    wsum[wave] = inc;
+    wmax[wave] = m;
+  }
   __syncthreads();
-  if (t == 0) {
-    int64_t acc = 0;
+  int64_t acc = inc - s;
+  for (int w = 0; w < wave; ++w) acc += wsum[w];
+  if (t == 1023) {
+    *total = acc + s;
     int mm = 0;
-    for (int i = 0; i < 1024; ++i) {
-      const int64_t v = part[i];
-      part[i] = acc;
-      acc += v;
-      mm = mx[i] > mm ? mx[i] : mm;
-    }
-    *total = acc;
+    for (int w = 0; w < 16; ++w) mm = wmax[w] > mm ? wmax[w] : mm;
     *max_count = mm;
     if (nflag) {
       total[1] = *nflag;
       *nflag = 0;
     }
   }
-  __syncthreads();
-  int64_t acc = part[t];
   for (int i = b; i < e; ++i) {
     offsets[i] = acc;
     const int c = counts[i];
@@ -238,17 +218,24 @@ hipError_t launch_correlate(int geo, const PairArgs& a, int total, hipStream_t s
   return e ? e->correlate(a, total, s) : hipErrorInvalidValue;
 }
 
-hipError_t launch_scan(int nb, const ScanArgs& a, int total, hipStream_t s) {
-  // the pure-A/C/G/T kernel, its A/C/G/T/N variant and the general one over the same grid;
-  // each workgroup exits at once on the other kernels' pairs
-  const int grid = total * (a.split > 1 ? a.split : 1);
-#define CALL(X)                                                            \
-  hipLaunchKernelGGL(k_scan<(X) | 32>, dim3(grid), dim3(SCAN_NT), 0, s, a); \
-  hipLaunchKernelGGL(k_scan<(X) | 64>, dim3(grid), dim3(SCAN_NT), 0, s, a); \
-  hipLaunchKernelGGL(k_scan<X>, dim3(grid), dim3(SCAN_NT), 0, s, a)
-  SXC_NB_SWITCH(nb, CALL)
-#undef CALL
-  return hipGetLastError();
+// Workgroups per (pair, strand) of one kind's kernel: as many as it takes to put `fill`
+// workgroups on the device, at most 16 (the lags of a strand are taken 8 or 16 at a time).
+static int scan_split(int fill, int n) {
+  const int k = n > 0 ? fill / n : 1;
+  return k < 1 ? 1 : (k > 16 ? 16 : k);
+}
+
+hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& kinds, bool can_split, hipStream_t s) {
+  // one launch per kind that occurs, over the same grid; a workgroup exits at once on another
+  // kind's pair
+  for (int k = 0; k < 3; ++k) {
+    if (kinds.pairs[k] <= 0) continue;
+    ScanArgs b = a;
+    b.split = can_split ? scan_split(256 * SCAN_FILL[k], kinds.pairs[k] * a.strands) : 1;
+    const hipError_t e = (k == 0 ? launch_scan_pure : k == 1 ? launch_scan_n : launch_scan_general)(nb, b, total * b.split, s);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_peaks(int nb, const float* xc, double cutoff, uint16_t* cands, int32_t* ncand, hipStream_t s) {

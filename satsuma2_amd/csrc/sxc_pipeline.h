@@ -48,6 +48,7 @@ struct PairArgs {
   // and forward transforms (the spectra are those transforms' output, bit for bit)
   const float* qspectra;
   int32_t* counts;               // optional: set to 0 per (pair, strand) for a split scan
+  int32_t* stats;                // optional: {candidates, runs} per (pair, strand), runs set to 0 for it
 };
 
 struct SpecArgs {
@@ -770,6 +771,7 @@ SXC_HD inline void correlate_body(Ex& ex, char* sm, const PairArgs& a, int ps) {
     if (tid == 0) {
       a.ncand[ps] = n;
       if (a.counts) a.counts[ps] = 0;
+      if (a.stats) a.stats[2 * ps + 1] = 0;
     }
   });
 }

@@ -88,6 +88,7 @@ struct Slot {
   int64_t copied = 0;               // ordered records the launch itself copied to h_final
   int cap = kDefaultCap;            // records per (pair, strand) of the current launch
   int npairs = 0;
+  sxc::ScanKinds kinds;
   std::vector<Piece> pieces;
   SlotState state = FREE;
 };
@@ -105,7 +106,6 @@ struct sxc_server {
   // mean records per pair (sizes the prefix of records a launch copies back with its counts).
   int cap_hint = kDefaultCap;
   double records_per_pair = 0.;
-  int cus = 256;  // compute units of the device
   DevBuf seq, tch, qch, spectra, qspectra;
   DevBuf ent;  // window entropies of chunks with B/D/H/V letters (computed on the host)
   // host copies of the chunk bytes and tables: records flagged near min_prob are decided
@@ -183,11 +183,11 @@ int64_t slot_bytes_for(int P, int N, int cap) {
   return (int64_t)P * sizeof(sxc_pair_dev) + total * N * 2 + total * 4 + total * cap * (72 + 8 + 72) + total * 12 + 64;
 }
 
-// split: workgroups per (pair, strand) (counts must have been cleared by the pair kernel
-// when above 1).  order: also order the records into final_ (up to out_cap) and copy the
-// first of them to the host in the same pass, so a launch whose records fit needs no
-// second round trip.
-int launch_scan_slot(sxc_server* sv, Slot& sl, int split, bool order) {
+// fresh: the pair kernel has just cleared the counts, so small launches may split a (pair,
+// strand)'s lags over several workgroups.  order: also order the records into final_ (up to
+// out_cap) and copy the first of them to the host in the same pass, so a launch whose records
+// fit needs no second round trip.
+int launch_scan_slot(sxc_server* sv, Slot& sl, bool fresh, bool order) {
   // Room for cap records of every (pair, strand) of this launch.  The buffers only grow;
   // a launch may have more pairs than the one that last grew them.
   const size_t nrec = (size_t)2 * sl.npairs * sl.cap;
@@ -216,8 +216,7 @@ int launch_scan_slot(sxc_server* sv, Slot& sl, int split, bool order) {
   a.stats = nullptr;
   a.ptable = sv->ptable;
   a.table_prob = sv->prm.table_prob;
-  a.split = split;
-  HIPCHK(sxc::launch_scan(sv->nb, a, 2 * sl.npairs, sl.s));
+  HIPCHK(sxc::launch_scan(sv->nb, a, 2 * sl.npairs, sl.kinds, fresh, sl.s));
   const int total = 2 * sl.npairs;
   HIPCHK(sxc::launch_count_offsets(sl.counts.as<int32_t>(), total, sl.cap, sl.offsets.as<int64_t>(),
                                    sl.total.as<int64_t>(), sl.maxc.as<int32_t>(), sl.s));
@@ -245,6 +244,7 @@ int launch_scan_slot(sxc_server* sv, Slot& sl, int split, bool order) {
 int slot_fill(sxc_server* sv, Slot& sl) {
   sl.pieces.clear();
   sl.npairs = 0;
+  sl.kinds = sxc::ScanKinds();
   sl.cap = sv->cap_hint;
   while (sl.npairs < sv->P && !sv->pending.empty()) {
     Request* r = sv->pending.front();
@@ -264,6 +264,7 @@ int slot_fill(sxc_server* sv, Slot& sl) {
       d.q_record_len = qm.record_len;
       d.fast = b.fast ? 1 : 0;
       d.q_tail = -1;
+      ++sl.kinds.pairs[sxc::scan_kind(sv->h_tch[(size_t)ti].flags, sv->h_qch[(size_t)qi].flags)];
       ++pc.count;
       ++r->dispatched;
       // align_target order: query chunks outer, target chunks inner
@@ -300,10 +301,7 @@ int slot_fill(sxc_server* sv, Slot& sl) {
   a.qspectra = sv->qspec_bytes > 0 ? sv->qspectra.as<float>() : nullptr;
   a.counts = sl.counts.as<int32_t>();  // cleared per (pair, strand) for a split scan
   HIPCHK(sxc::launch_correlate(sv->geo_corr, a, 2 * sl.npairs, sl.s));
-  // A launch too small to fill the device splits each (pair, strand)'s lags over up to 4
-  // scan workgroups (3 resident per CU), which shortens its latency.
-  const int split = std::max(1, std::min(4, 3 * sv->cus / (2 * sl.npairs)));
-  int rc = launch_scan_slot(sv, sl, split, true);
+  int rc = launch_scan_slot(sv, sl, true, true);
   if (rc) return rc;
   sl.state = COUNTING;
   ++sv->st_launches;
@@ -325,7 +323,7 @@ int slot_pack(sxc_server* sv, Slot& sl) {
     // start with that much room (up to 1024 records per (pair, strand))
     sl.cap = *sl.h_maxc;
     sv->cap_hint = std::min(1024, std::max(sv->cap_hint, sl.cap));
-    return launch_scan_slot(sv, sl, 1, true);
+    return launch_scan_slot(sv, sl, false, true);
   }
   const int64_t n = sl.h_offsets[total];
   sv->records_per_pair = 0.9 * sv->records_per_pair + 0.1 * (double)n / std::max(1, sl.npairs);
@@ -494,7 +492,6 @@ int server_init(sxc_server* sv, const sxc_chunk_desc* targets, int32_t nt, const
   if (rc) return rc;
   bytes.resize(bytes.size() + 16, 0);
   sv->P = cfg && cfg->max_pairs_per_launch > 0 ? cfg->max_pairs_per_launch : 2048;
-  HIPCHK(hipDeviceGetAttribute(&sv->cus, hipDeviceAttributeMultiprocessorCount, sv->ctx->device));
   const int max_slots = cfg && cfg->max_slots > 0 ? cfg->max_slots : 3;
   size_t free_b = 0, total_b = 0;
   HIPCHK(hipMemGetInfo(&free_b, &total_b));

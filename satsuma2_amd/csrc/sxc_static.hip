@@ -185,6 +185,8 @@ extern "C" int sxc_align_pair_static(sxc_ctx* ctx, const sxc_pair* pair, const s
   a.cutoff_fast = prm->cutoff_fast;
   a.cands = (uint16_t*)(base + L.cands);
   a.ncand = (int32_t*)(base + L.ncand);
+  a.counts = (int32_t*)(base + L.counts);
+  a.stats = (int32_t*)(base + L.stats);
   HIPCHK(sxc::launch_correlate(ctx->geo_corr[nb], a, S, s));
   // the diagonal scan and the probability tail
   sxc::ScanArgs c{};
@@ -207,7 +209,9 @@ extern "C" int sxc_align_pair_static(sxc_ctx* ctx, const sxc_pair* pair, const s
   c.counts = (int32_t*)(base + L.counts);
   c.cap = SXC_STATIC_RECORDS;
   c.stats = (int32_t*)(base + L.stats);
-  HIPCHK(sxc::launch_scan(nb, c, S, s));
+  sxc::ScanKinds kinds;
+  kinds.pairs[sxc::scan_kind(tch.flags, qch.flags)] = 1;
+  HIPCHK(sxc::launch_scan(nb, c, S, kinds, true, s));
   HIPCHK(sxc::launch_count_offsets(c.counts, S, SXC_STATIC_RECORDS, (int64_t*)(base + L.offsets),
                                    (int64_t*)(base + L.total), (int32_t*)(base + L.maxc), s, c.nflag));
   HIPCHK(sxc::launch_order_records(c.counts, S, SXC_STATIC_RECORDS, (const int64_t*)(base + L.offsets), c.out,
