@@ -21,8 +21,6 @@ inline int scan_kind(int32_t tflags, int32_t qflags) {
 struct ScanKinds {
   int32_t pairs[3] = {0, 0, 0};
 };
-// Workgroups per CU that a kind's kernel needs before a strand is taken by one workgroup.
-constexpr int SCAN_FILL[3] = {4, 4, 3};
 // Scans the accepted lags of `total` (pair, strand)s.  can_split: counts (and the run counts of
 // stats) are zero, so that a launch too small to fill the device may share a strand's lags
 // between several workgroups.

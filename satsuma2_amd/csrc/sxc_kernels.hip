@@ -4,6 +4,8 @@
 // double arithmetic are never contracted into FMA; see sxc_fft.h).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "sxc_fft_kernels.h"
 #include "sxc_kernels.h"
 #include "sxc_pipeline.h"
@@ -218,11 +220,14 @@ hipError_t launch_correlate(int geo, const PairArgs& a, int total, hipStream_t s
   return e ? e->correlate(a, total, s) : hipErrorInvalidValue;
 }
 
-// Workgroups per (pair, strand) of one kind's kernel: as many as it takes to put `fill`
-// workgroups on the device, at most 16 (the lags of a strand are taken 8 or 16 at a time).
-static int scan_split(int fill, int n) {
-  const int k = n > 0 ? fill / n : 1;
-  return k < 1 ? 1 : (k > 16 ? 16 : k);
+// Workgroups per (pair, strand) for n of them.  A strand's lags are taken 8 or 16 at a time, and
+// every workgroup packs both chunks first, so a share pays only while compute units are idle:
+// up to 2048 workgroups in all (8 per CU), more than 4 per strand only below 512.  Measured
+// at N = 8192, us of the pure kernel with 1 / 2 / 4 / 8 / 16 workgroups per strand: 2 strands
+// 109 / - / - / - / 16, 128 strands - / 17 / 18 / 22 / 29, 740 strands 195 / 120 / - / - / -.
+static int scan_split(int n) {
+  const int k = n > 0 ? std::min({2048 / n, std::max(4, 512 / n), 16}) : 1;
+  return std::max(1, k);
 }
 
 hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& kinds, bool can_split, hipStream_t s) {
@@ -231,7 +236,7 @@ hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& ki
   for (int k = 0; k < 3; ++k) {
     if (kinds.pairs[k] <= 0) continue;
     ScanArgs b = a;
-    b.split = can_split ? scan_split(256 * SCAN_FILL[k], kinds.pairs[k] * a.strands) : 1;
+    b.split = can_split ? scan_split(kinds.pairs[k] * a.strands) : 1;
     const hipError_t e = (k == 0 ? launch_scan_pure : k == 1 ? launch_scan_n : launch_scan_general)(nb, b, total * b.split, s);
     if (e != hipSuccess) return e;
   }
