@@ -5,8 +5,9 @@
  * the query's with the target's and chains joined positions that continue along one
  * diagonal, with gaps of up to max_jump positions, into blocks of at least min_length
  * bases.  SatsumaSynteny2 runs it for K = 11, 13, ..., 31 (analysis/SatsumaSynteny2.cc:
- * 417-463) and reads its t_result files as the search's first matches.  Here the k-mer
- * tables are built, sorted, filtered and joined on the GPU; the chaining sweep, whose
+ * 417-463) and reads its t_result files as the search's first matches.  Here, for
+ * max_freq = 1 and max_jump up to 64, the whole run is on the GPU; with other parameters the
+ * k-mer tables are built, sorted, filtered and joined there and the chaining sweep, whose
  * output order follows the sorted positions, runs on the host.  Results equal the
  * reference's (t_result records, same order; the 7 padding bytes after `reverse`, which
  * the reference leaves uninitialized, are zero) for max_freq = 1, SatsumaSynteny2's
@@ -40,7 +41,7 @@ typedef struct {
   int64_t query_kept, target_kept;    /* after the frequency filter */
   int64_t joined;                     /* joined positions (kmatches) */
   int64_t blocks;                     /* reported t_result records */
-  double read_ms, device_ms, sweep_ms;
+  double read_ms, device_ms, sweep_ms;  /* sweep_ms: the host's chaining sweep (0 when on the GPU) */
 } sxc_kmatch_stats;
 
 typedef struct sxc_kmatch sxc_kmatch;

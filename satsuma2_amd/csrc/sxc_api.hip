@@ -830,6 +830,7 @@ void sxc_destroy(sxc_ctx* c) {
   for (sxc_batch_dev& b : c->scratch_nb) b.release();
   for (auto& kv : c->ptables) kv.second.release();
   for (DevBuf* b : {&c->p0, &c->p1, &c->p2, &c->p3, &c->p4, &c->p5, &c->p6}) b->release();
+  for (DevBuf& b : c->km) b.release();
   (void)hipFree(c->d_tab);
   (void)hipFree(c->d_osc);
   for (auto p : c->d_ent)

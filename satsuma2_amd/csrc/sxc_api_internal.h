@@ -99,6 +99,8 @@ struct sxc_batch_dev {
   }
 };
 
+#define SXC_KMATCH_BUFS 13
+
 struct sxc_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -111,6 +113,7 @@ struct sxc_ctx {
   sxc_batch_dev scratch;          // buffers reused by the one-shot entry points
   sxc_batch_dev scratch_nb[16];  // ... per length class when N is chosen per pair
   DevBuf p0, p1, p2, p3, p4, p5, p6;  // plain-API staging
+  DevBuf km[SXC_KMATCH_BUFS];         // KMatch's device buffers (at most 1 GiB between calls)
   std::map<double, DevBuf> ptables;   // ProbTable thresholds by target size (-prob_table)
   // FFT geometry code per log2 length for the pair kernel and the target-spectra kernel
   // (a plain log2 length: the default geometry; set by sxc_autotune / sxc_set_geometry)

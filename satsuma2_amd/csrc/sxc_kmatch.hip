@@ -1,5 +1,6 @@
-// sxc_kmatch.hip -- KMatch (kmatch/KMatch.cc) with its k-mer tables built, sorted,
-// filtered and joined on the GPU, and the chaining sweep on the host (include/sxc_kmatch.h).
+// sxc_kmatch.hip -- KMatch (kmatch/KMatch.cc) on the GPU (include/sxc_kmatch.h).  With max_freq = 1
+// the path of sxc_kmatch_unique.h runs; this file holds its host side and the general path, whose
+// k-mer tables are built, sorted, filtered and joined on the GPU and chained on the host.
 //
 // Per genome (KMatch::kmer_array_from_fasta, KMatch.cc:21-132): every position whose K
 // bases are all A/C/G/T (either case) gives its canonical k-mer -- the smaller of the
@@ -19,9 +20,12 @@
 // contain it (a group is longer than max_freq iff one such window has equal ends), so it
 // reads O(max_freq) neighbours instead of the group.
 #include <hip/hip_runtime.h>
+#include <stdlib.h>
 #include <string.h>
+#include <sys/mman.h>
 
 #include <chrono>
+#include <deque>
 #include <fstream>
 #include <memory>
 #include <rocprim/device/device_radix_sort.hpp>
@@ -31,6 +35,7 @@
 
 #include "../../include/sxc_kmatch.h"
 #include "sxc_api_internal.h"
+#include "sxc_kmatch_unique.h"
 
 using sxc::fail;
 
@@ -41,10 +46,13 @@ constexpr int kSpan = 16;                          // positions per lane
 constexpr int kChunk = 64 * kSpan;                 // positions per chunk (one wave)
 constexpr int kBlock = 256;
 
-// One genome's sequences as the table builder walks them.
+// One genome's sequences as the table builder walks them: in device memory they follow each
+// other, each preceded by one 'N'.
 struct Side {
-  std::string buf;                 // each sequence preceded by one 'N'
-  std::vector<int64_t> off;        // start of each sequence in buf
+  std::deque<std::string> owned;   // sequences read from a file
+  std::vector<const char*> seq;    // each sequence's bytes (owned, or the caller's)
+  int64_t len = 0;                 // bytes of the device buffer
+  std::vector<int64_t> off;        // start of each sequence in it
   std::vector<int64_t> index;      // its sequence index (headers seen when it was processed)
   std::vector<uint64_t> lengths;   // seqnames[].length, in processing order
   int64_t slots = 0;               // table size: sum of len + 1 - K
@@ -56,9 +64,9 @@ int add_sequence(Side* s, const char* p, int64_t len, int64_t index, int K, cons
     return fail(SXC_ERR_ARG, what + ": a record of " + std::to_string(len) + " bases is shorter than K - 1");
   s->slots += len + 1 - K;
   s->lengths.push_back((uint64_t)len);
-  s->buf.push_back('N');
-  s->off.push_back((int64_t)s->buf.size());
-  s->buf.append(p, (size_t)len);
+  s->off.push_back(s->len + 1);
+  s->len += 1 + len;
+  s->seq.push_back(p);
   s->index.push_back(index);
   return SXC_OK;
 }
@@ -74,10 +82,11 @@ int read_side(const char* path, int K, Side* s) {
   for (;;) {
     std::getline(f, line);
     if ((!line.empty() && line[0] == '>') || f.eof()) {
-      const int rc = add_sequence(s, seq.data(), (int64_t)seq.size(), index, K, path);
+      s->owned.push_back(std::move(seq));
+      const int rc = add_sequence(s, s->owned.back().data(), (int64_t)s->owned.back().size(), index, K, path);
       if (rc != SXC_OK) return rc;
       if (f.eof()) break;
-      seq.clear();
+      seq = std::string();
       ++index;
     } else {
       if (f.fail()) return fail(SXC_ERR_ARG, std::string("read error in ") + path);
@@ -268,6 +277,30 @@ struct Buffers {
     if (e_ != hipSuccess) return fail(SXC_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_));      \
   } while (0)
 
+// A genome's buffer into device memory at d.  Long sequences are copied from where they lie,
+// runs of short ones through `stage` (which has to live until the stream is synchronised).
+int upload(const Side& side, unsigned char* d, std::vector<std::string>& stage, hipStream_t s) {
+  constexpr int64_t kLong = 65536, kStage = 1 << 22;
+  KCHK(hipMemsetAsync(d, 'N', (size_t)side.len, s));
+  for (size_t k = 0; k < side.seq.size();) {
+    const int64_t n = (int64_t)side.lengths[k];
+    if (n >= kLong) {
+      KCHK(hipMemcpyAsync(d + side.off[k], side.seq[k], (size_t)n, hipMemcpyHostToDevice, s));
+      ++k;
+      continue;
+    }
+    const int64_t at = side.off[k];
+    std::string run;
+    for (; k < side.seq.size() && (int64_t)side.lengths[k] < kLong && (int64_t)run.size() < kStage; ++k) {
+      run.resize((size_t)(side.off[k] - at), 'N');
+      run.append(side.seq[k], (size_t)side.lengths[k]);
+    }
+    stage.push_back(std::move(run));
+    KCHK(hipMemcpyAsync(d + at, stage.back().data(), stage.back().size(), hipMemcpyHostToDevice, s));
+  }
+  return SXC_OK;
+}
+
 // exclusive scan of n uint64 values; returns the total in *total
 int scan(Buffers& B, const uint64_t* in, uint64_t* out, int64_t n, uint64_t* total, hipStream_t s) {
   if (n == 0) {
@@ -290,8 +323,8 @@ int scan(Buffers& B, const uint64_t* in, uint64_t* out, int64_t n, uint64_t* tot
 // One genome's table: built, sorted by k-mer, filtered; the sorted kept entries are left in
 // (*keys, *vals), *n of them.
 int build_table(Buffers& B, const Side& side, int K, int F, hipStream_t s, uint64_t** keys, int64_t** vals,
-                int64_t* n, int64_t* kept) {
-  const int64_t len = (int64_t)side.buf.size();
+                int64_t* n, int64_t* kept, std::vector<std::string>& stage) {
+  const int64_t len = side.len;
   const int64_t slots = side.slots;
   const int nseq = (int)side.off.size();
   *n = 0;
@@ -302,7 +335,8 @@ int build_table(Buffers& B, const Side& side, int K, int F, hipStream_t s, uint6
   KCHK(B.get(&dbuf, len));
   KCHK(B.get(&doff, nseq));
   KCHK(B.get(&didx, nseq));
-  KCHK(hipMemcpyAsync(dbuf, side.buf.data(), (size_t)len, hipMemcpyHostToDevice, s));
+  int rc = upload(side, dbuf, stage, s);
+  if (rc != SXC_OK) return rc;
   KCHK(hipMemcpyAsync(doff, side.off.data(), sizeof(int64_t) * nseq, hipMemcpyHostToDevice, s));
   KCHK(hipMemcpyAsync(didx, side.index.data(), sizeof(int64_t) * nseq, hipMemcpyHostToDevice, s));
   const int64_t chunks = (len + kChunk - 1) / kChunk;
@@ -313,7 +347,7 @@ int build_table(Buffers& B, const Side& side, int K, int F, hipStream_t s, uint6
                      nullptr, doff, didx, nseq, nullptr, nullptr);
   KCHK(hipGetLastError());
   uint64_t filled = 0;
-  int rc = scan(B, cnt, base, chunks, &filled, s);
+  rc = scan(B, cnt, base, chunks, &filled, s);
   if (rc != SXC_OK) return rc;
   if ((int64_t)filled > slots) return fail(SXC_ERR_ARG, "k-mer table overflow");  // cannot happen: one per slot
   uint64_t *k0, *k1;
@@ -353,8 +387,13 @@ int build_table(Buffers& B, const Side& side, int K, int F, hipStream_t s, uint6
 }  // namespace
 
 struct sxc_kmatch {
-  std::vector<sxc_result> out;
+  std::vector<sxc_result> out;        // the general path's records
+  sxc_result* raw = nullptr;          // or the unique path's, as they came from the device
+  int64_t n_raw = 0;
   sxc_kmatch_stats st{};
+  const sxc_result* data() const { return raw ? raw : out.data(); }
+  int64_t size() const { return raw ? n_raw : (int64_t)out.size(); }
+  ~sxc_kmatch() { free(raw); }
 };
 
 namespace {
@@ -417,16 +456,202 @@ void sweep(const std::vector<uint64_t>& q, const std::vector<int64_t>& t, const 
   (void)ts;
 }
 
+// Memory for records that come back from the device; large blocks ask for huge pages, whose first
+// touch costs a copy into fresh memory far less.  Given back with free().
+void* result_memory(size_t bytes) {
+  constexpr size_t kHuge = 2u << 20;
+  if (bytes < 2 * kHuge) return malloc(bytes);
+  const size_t n = (bytes + kHuge - 1) / kHuge * kHuge;
+  void* p = aligned_alloc(kHuge, n);
+  if (p) (void)madvise(p, n, MADV_HUGEPAGE);
+  return p;
+}
+
+// Device buffers of the unique path, kept by the context between calls.
+enum { KM_BUF, KM_KEYS, KM_KEYS2, KM_VALS, KM_VALS2, KM_TMP, KM_START, KM_DENSE, KM_SEEN, KM_JOINED, KM_LINKS, KM_SEQS,
+       KM_OUT };
+static_assert(KM_OUT < SXC_KMATCH_BUFS, "");
+
+// What the unique path takes: every k-mer at most once, gaps the neighbour searches can bridge
+// (SatsumaSynteny2 asks for K - 1 <= 30; both searches read up to max_jump entries), positions
+// in 31 bits.
+bool unique_path(const Side& qs, const Side& ts, const sxc_kmatch_params& p) {
+  return p.max_freq == 1 && p.max_jump <= 64 && qs.slots > 0 && ts.slots > 0 &&
+         qs.len + ts.len < (1ll << 31) - 65536;
+}
+
+// KMatch for max_freq = 1 on the device (sxc_kmatch_unique.h).  *done is false if a bucket held
+// more k-mers than its table takes; the general path then runs.
+int run_unique(sxc_ctx* ctx, const Side& qs, const Side& ts, const sxc_kmatch_params& p, sxc_kmatch* res, bool* done) {
+  using namespace sxc::km;
+  hipStream_t s = ctx->stream;
+  DevBuf* W = ctx->km;
+  std::vector<std::string> stage;
+  *done = false;
+  const int64_t len = qs.len + ts.len, slots = qs.slots + ts.slots;
+  const int nq = (int)qs.off.size(), nt = (int)ts.off.size();
+  // buckets of 200 .. 400 entries: half full tables
+  int bits = 1;
+  while (bits < 24 && (slots >> bits) > 400) ++bits;
+  const uint32_t buckets = 1u << bits;
+  const size_t heavy_max = (size_t)(slots / kHeavy) + 1;
+  constexpr int kHeavyGroups = 1024, kLook = 64, kWaves = kBucketGroups + kLook;
+  // sequence starts (in the joint buffer) and indices of both genomes, then the query's lengths
+  std::vector<int64_t> seqs;
+  seqs.insert(seqs.end(), qs.off.begin(), qs.off.end());
+  seqs.insert(seqs.end(), qs.index.begin(), qs.index.end());
+  for (int64_t o : ts.off) seqs.push_back(o + qs.len);
+  seqs.insert(seqs.end(), ts.index.begin(), ts.index.end());
+  for (uint64_t l : qs.lengths) seqs.push_back((int64_t)l);
+  KCHK(W[KM_BUF].ensure((size_t)((len + 15) / 16 * 16)));
+  KCHK(W[KM_SEQS].ensure(seqs.size() * sizeof(int64_t)));
+  KCHK(W[KM_KEYS].ensure((size_t)slots * sizeof(uint64_t)));
+  KCHK(W[KM_KEYS2].ensure((size_t)slots * sizeof(uint64_t)));
+  KCHK(W[KM_VALS].ensure((size_t)slots * sizeof(uint32_t)));
+  KCHK(W[KM_VALS2].ensure((size_t)slots * sizeof(uint32_t)));
+  KCHK(W[KM_DENSE].ensure((size_t)(qs.len + 16) * sizeof(uint32_t)));
+  // bucket starts, heavy list
+  KCHK(W[KM_START].ensure(((size_t)buckets + 1 + heavy_max) * sizeof(uint32_t)));
+  const uint32_t dense_groups = (uint32_t)((qs.len + kDense - 1) / kDense);
+  // control words, per-wave results, group counts; the heavy tables behind them
+  const size_t seen_bytes = 256 + (size_t)kWaves * 2 * (sizeof(uint64_t) + sizeof(uint32_t)) +
+                            (((size_t)dense_groups * sizeof(uint32_t) + 255) & ~(size_t)255);
+  KCHK(W[KM_SEEN].ensure(seen_bytes + heavy_max * kTable * (sizeof(uint64_t) + 2 * sizeof(uint32_t))));
+  unsigned char* dbuf = W[KM_BUF].as<unsigned char>();
+  uint64_t *k0 = W[KM_KEYS].as<uint64_t>(), *k1 = W[KM_KEYS2].as<uint64_t>();
+  uint32_t *v0 = W[KM_VALS].as<uint32_t>(), *v1 = W[KM_VALS2].as<uint32_t>();
+  uint32_t* dense = W[KM_DENSE].as<uint32_t>();
+  uint32_t *start = W[KM_START].as<uint32_t>(), *list = start + buckets + 1;
+  char* seen = W[KM_SEEN].as<char>();
+  Ctl* ctl = (Ctl*)seen;
+  static_assert(sizeof(Ctl) <= 256, "");
+  uint64_t* best = (uint64_t*)(seen + 256);
+  uint32_t* at = (uint32_t*)(best + 2 * kWaves);
+  uint32_t* groups = at + 2 * kWaves;
+  uint64_t* gkey = (uint64_t*)(seen + seen_bytes);
+  uint32_t* gpos = (uint32_t*)(gkey + heavy_max * kTable);
+  const int64_t* dseq = W[KM_SEQS].as<int64_t>();
+  const Seqs dq{dseq, dseq + nq, nq}, dt{dseq + 2 * nq, dseq + 2 * nq + nt, nt};
+  const uint64_t* dlen = (const uint64_t*)(dseq + 2 * nq + 2 * nt);
+  const uint32_t len_q = (uint32_t)qs.len;
+  Ctl host{};
+
+  KCHK(hipMemsetAsync(ctl, 0, sizeof(Ctl), s));
+  int rc = upload(qs, dbuf, stage, s);
+  if (rc == SXC_OK) rc = upload(ts, dbuf + qs.len, stage, s);
+  if (rc != SXC_OK) return rc;
+  KCHK(hipMemcpyAsync(W[KM_SEQS].p, seqs.data(), seqs.size() * sizeof(int64_t), hipMemcpyHostToDevice, s));
+  hipLaunchKernelGGL(k_unique_kmers, dim3((unsigned)((len + 4095) / 4096)), dim3(256), 0, s, dbuf, len, qs.len, p.K, k0,
+                     v0, ctl);
+  hipLaunchKernelGGL(k_unique_unfilled, dim3(1), dim3(1), 0, s, k0, v0, qs.slots, ts.slots, len_q, ctl);
+  KCHK(hipGetLastError());
+  KCHK(hipMemcpyAsync(&host, ctl, sizeof host, hipMemcpyDeviceToHost, s));
+  KCHK(hipStreamSynchronize(s));
+  const uint32_t n = (uint32_t)host.n;
+  if ((int64_t)host.n > slots) return fail(SXC_ERR_ARG, "k-mer table overflow");  // cannot happen: one per slot
+  if (n > 0) {
+    size_t bytes = 0;
+    KCHK(rocprim::radix_sort_pairs(nullptr, bytes, k0, k1, v0, v1, (size_t)n, 0, bits, s));
+    KCHK(W[KM_TMP].ensure(bytes));
+    KCHK(rocprim::radix_sort_pairs(W[KM_TMP].p, bytes, k0, k1, v0, v1, (size_t)n, 0, bits, s));
+    KCHK(hipMemsetAsync(dense, 0, (size_t)(qs.len + 16) * sizeof(uint32_t), s));
+    hipLaunchKernelGGL(k_bounds, dim3(n / 256 + 1), dim3(256), 0, s, k1, n, buckets, start);
+    hipLaunchKernelGGL(k_heavy_list, dim3((buckets + 255) / 256), dim3(256), 0, s, start, buckets, list, ctl);
+    hipLaunchKernelGGL(k_buckets, dim3(kBucketGroups), dim3(64), 0, s, k1, v1, start, buckets, len_q, dense, best, at, ctl);
+    // (these exit at once where no bucket is heavy)
+    hipLaunchKernelGGL(k_heavy_clear, dim3(kLook), dim3(256), 0, s, ctl, gkey, gpos);
+    hipLaunchKernelGGL(k_heavy_count, dim3(kHeavyGroups), dim3(256), 0, s, k1, v1, start, list, len_q, gkey, gpos, ctl);
+    hipLaunchKernelGGL(k_heavy_look, dim3(kLook), dim3(64), 0, s, len_q, gkey, gpos, dense, best + 2 * kBucketGroups,
+                       at + 2 * kBucketGroups, ctl);
+    hipLaunchKernelGGL(k_last, dim3(1), dim3(64), 0, s, best, at, kWaves, ctl);
+    hipLaunchKernelGGL(k_joined<false>, dim3(dense_groups), dim3(256), 0, s, dense, len_q, groups, dq, dt, nullptr,
+                       nullptr, nullptr, ctl);
+    hipLaunchKernelGGL(k_scan_groups, dim3(1), dim3(1024), 0, s, groups, (int)dense_groups, &ctl->joined);
+    KCHK(hipGetLastError());
+    KCHK(hipMemcpyAsync(&host, ctl, sizeof host, hipMemcpyDeviceToHost, s));
+    KCHK(hipStreamSynchronize(s));
+    if (host.overflow) return SXC_OK;
+  }
+  const uint32_t nj = (uint32_t)host.joined;
+  uint32_t nb = 0;
+  if (nj > 0) {
+    const uint32_t tiles = (nj + kTile - 1) / kTile;
+    const size_t m = ((size_t)nj + 15) / 16 * 16;
+    KCHK(W[KM_JOINED].ensure(m * (sizeof(uint64_t) + sizeof(int64_t) + 1)));
+    KCHK(W[KM_LINKS].ensure(m * (5 * sizeof(uint32_t) + 1) + (size_t)tiles * sizeof(uint32_t)));
+    uint64_t* jq = W[KM_JOINED].as<uint64_t>();
+    int64_t* jt = (int64_t*)(jq + m);
+    uint8_t* jr = (uint8_t*)(jt + m);
+    uint32_t *up = W[KM_LINKS].as<uint32_t>(), *first = up + m, *bf = first + m, *bl = bf + m, *bc = bl + m;
+    uint32_t* tile_count = bc + m;
+    uint8_t* extended = (uint8_t*)(tile_count + tiles);
+    KCHK(hipMemsetAsync(extended, 0, nj, s));
+    hipLaunchKernelGGL(k_joined<true>, dim3(dense_groups), dim3(256), 0, s, dense, len_q, groups, dq, dt, jq, jt, jr,
+                       ctl);
+    hipLaunchKernelGGL(k_link, dim3(tiles), dim3(kTile), 0, s, jq, jt, jr, nj, (int64_t)p.max_jump, up, extended);
+    hipLaunchKernelGGL(k_ends, dim3(tiles), dim3(256), 0, s, jq, up, extended, nj, p.K, p.min_length, first, tile_count);
+    hipLaunchKernelGGL(k_scan_groups, dim3(1), dim3(1024), 0, s, tile_count, (int)tiles, &ctl->blocks);
+    hipLaunchKernelGGL(k_blocks, dim3(tiles), dim3(256), 0, s, jq, first, nj, (int64_t)p.max_jump, tile_count, bf, bl, bc);
+    KCHK(hipGetLastError());
+    KCHK(hipMemcpyAsync(&host, ctl, sizeof host, hipMemcpyDeviceToHost, s));
+    KCHK(hipStreamSynchronize(s));
+    nb = (uint32_t)host.blocks;
+    if (nb > 0) {
+      KCHK(W[KM_OUT].ensure((size_t)nb * sizeof(sxc_result)));
+      const size_t bytes = (size_t)nb * sizeof(sxc_result);
+      res->raw = (sxc_result*)result_memory(bytes);
+      if (!res->raw) return fail(SXC_ERR_NOMEM, "sxc_kmatch: out of memory");
+      hipLaunchKernelGGL(k_records, dim3((nb + 255) / 256), dim3(256), 0, s, bf, bl, bc, nb, jq, jt, jr, p.K, dlen,
+                         (int)qs.lengths.size(), W[KM_OUT].as<sxc_result>());
+      KCHK(hipGetLastError());
+      KCHK(hipMemcpyAsync(res->raw, W[KM_OUT].p, (size_t)nb * sizeof(sxc_result), hipMemcpyDeviceToHost, s));
+      KCHK(hipStreamSynchronize(s));
+    }
+  }
+  res->n_raw = nb;
+  res->st.query_kept = (int64_t)host.kept[0];
+  res->st.target_kept = (int64_t)host.kept[1];
+  res->st.joined = nj;
+  *done = true;
+  return SXC_OK;
+}
+
+int run_general(sxc_ctx* ctx, const Side& qs, const Side& ts, const sxc_kmatch_params& p, sxc_kmatch* res);
+
 int run(sxc_ctx* ctx, const Side& qs, const Side& ts, const sxc_kmatch_params& p, double read_ms, sxc_kmatch** out) {
   std::lock_guard<std::mutex> lock(ctx->mu);
   KCHK(hipSetDevice(ctx->device));
-  hipStream_t s = ctx->stream;
   sxc_kmatch* res = new (std::nothrow) sxc_kmatch;
   if (!res) return fail(SXC_ERR_NOMEM, "sxc_kmatch: out of memory");
   std::unique_ptr<sxc_kmatch> hold(res);
   res->st.read_ms = read_ms;
   res->st.query_kmers = qs.slots;
   res->st.target_kmers = ts.slots;
+  bool done = false;
+  if (unique_path(qs, ts, p)) {
+    const auto t0 = std::chrono::steady_clock::now();
+    const int rc = run_unique(ctx, qs, ts, p, res, &done);
+    res->st.device_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    // the buffers stay for the next call while they are small beside the device's memory
+    size_t held = 0;
+    for (const DevBuf& b : ctx->km) held += b.cap;
+    if (held > ((size_t)1 << 30) || rc != SXC_OK)
+      for (DevBuf& b : ctx->km) b.release();
+    if (rc != SXC_OK) return rc;
+  }
+  if (!done) {
+    const int rc = run_general(ctx, qs, ts, p, res);
+    if (rc != SXC_OK) return rc;
+  }
+  res->st.blocks = res->size();
+  *out = hold.release();
+  return SXC_OK;
+}
+
+// Any max_freq and max_jump: tables sorted, filtered and joined on the device, chained on the host.
+int run_general(sxc_ctx* ctx, const Side& qs, const Side& ts, const sxc_kmatch_params& p, sxc_kmatch* res) {
+  hipStream_t s = ctx->stream;
+  std::vector<std::string> stage;
   hipEvent_t e0, e1;
   KCHK(hipEventCreate(&e0));
   KCHK(hipEventCreate(&e1));
@@ -438,9 +663,9 @@ int run(sxc_ctx* ctx, const Side& qs, const Side& ts, const sxc_kmatch_params& p
     KCHK(hipEventRecord(e0, s));
     uint64_t *qk = nullptr, *tk = nullptr;
     int64_t *qv = nullptr, *tv = nullptr, nq = 0, nt = 0;
-    int rc = build_table(B, qs, p.K, p.max_freq, s, &qk, &qv, &nq, &res->st.query_kept);
+    int rc = build_table(B, qs, p.K, p.max_freq, s, &qk, &qv, &nq, &res->st.query_kept, stage);
     if (rc != SXC_OK) return rc;
-    rc = build_table(B, ts, p.K, p.max_freq, s, &tk, &tv, &nt, &res->st.target_kept);
+    rc = build_table(B, ts, p.K, p.max_freq, s, &tk, &tv, &nt, &res->st.target_kept, stage);
     if (rc != SXC_OK) return rc;
     uint64_t nj = 0;
     uint64_t* base = nullptr;  // each query entry's first joined slot
@@ -504,8 +729,6 @@ int run(sxc_ctx* ctx, const Side& qs, const Side& ts, const sxc_kmatch_params& p
   const auto t0 = std::chrono::steady_clock::now();
   sweep(hq, ht, hr, p, qs, ts, &res->out);
   res->st.sweep_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-  res->st.blocks = (int64_t)res->out.size();
-  *out = hold.release();
   return SXC_OK;
 }
 
@@ -556,8 +779,8 @@ int sxc_kmatch_records(sxc_ctx* ctx, int32_t n_queries, const char* const* query
 
 int sxc_kmatch_results(const sxc_kmatch* k, sxc_result* out, int64_t cap, int64_t* n) {
   if (!k || !n || cap < 0 || (cap && !out)) return fail(SXC_ERR_ARG, "sxc_kmatch_results: bad arguments");
-  *n = (int64_t)k->out.size();
-  for (int64_t i = 0; i < *n && i < cap; ++i) out[i] = k->out[(size_t)i];
+  *n = k->size();
+  if (const int64_t m = *n < cap ? *n : cap) memcpy(out, k->data(), (size_t)m * sizeof(sxc_result));
   return *n > cap ? fail(SXC_ERR_CAPACITY, "sxc_kmatch_results: more records than cap") : SXC_OK;
 }
 
