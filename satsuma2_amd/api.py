@@ -16,6 +16,8 @@ from __future__ import annotations
 
 import ctypes as C
 from dataclasses import dataclass
+from itertools import chain
+from operator import attrgetter
 from typing import List, NamedTuple, Sequence
 
 import numpy as np
@@ -192,7 +194,33 @@ class ChunkPair:
     fast: int = 0
 
 
+# sxc_pair's layout, and the ChunkPair fields of its integers
+_PAIR_DTYPE = np.dtype({"names": [f for f, _ in Pair._fields_],
+                        "formats": ["<u8" if f in ("tseq", "qseq") else "<i4" for f, _ in Pair._fields_],
+                        "offsets": [getattr(Pair, f).offset for f, _ in Pair._fields_], "itemsize": C.sizeof(Pair)})
+_PAIR_INTS = ("t_chunk_start", "q_chunk_start", "t_record", "q_record", "q_record_len", "fast")
+
+
+def _pairs_table(pairs: Sequence[ChunkPair]):
+    """_pairs_array for many pairs, a column at a time."""
+    n = len(pairs)
+    keep = [[p.tseq for p in pairs], [p.qseq for p in pairs]]
+    tab = np.zeros(n, _PAIR_DTYPE)
+    for f, seqs in zip(("t", "q"), keep):
+        tab[f + "seq"] = np.frombuffer((C.c_char_p * n)(*seqs), np.uint64)
+        tab[f + "len"] = np.fromiter(map(len, seqs), np.int32, n)
+    ints = np.array(list(chain.from_iterable(map(attrgetter(*_PAIR_INTS), pairs)))).reshape(n, len(_PAIR_INTS))
+    if ints.dtype.kind not in "iub":
+        raise TypeError("a chunk pair's positions, records and flags are integers")
+    for k, f in enumerate(_PAIR_INTS):
+        tab[f] = ints[:, k]
+    tab["q_record_len"] = np.where(tab["q_record_len"] >= 0, tab["q_record_len"], tab["qlen"])
+    return (Pair * n).from_buffer(tab), keep
+
+
 def _pairs_array(pairs: Sequence[ChunkPair]):
+    if len(pairs) >= 32:
+        return _pairs_table(pairs)
     arr = (Pair * max(1, len(pairs)))()
     keep = []
     for k, p in enumerate(pairs):
