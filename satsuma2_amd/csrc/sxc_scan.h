@@ -42,6 +42,9 @@ struct ScanArgs {
   double min_prob;
   double target_total;
   double z_skip;             // runs with (m - x) / s / 1.414213562 >= z_skip have prob < min_prob
+  // shortest flagged stretch (ne - ns) a kept run can have, by the kernel that finds it (pure
+  // A/C/G/T, with N, general): keep_min_run.  0 or 1: every run reaches the tail.
+  int32_t min_run[3];
   // keep band (keep_band): runs with prob >= keep_lo are written; those with prob < flag_hi
   // are flagged SXC_REC_NEAR for the host to decide, and counted in *nflag (optional)
   double keep_lo;
@@ -69,6 +72,12 @@ inline void set_keep(ScanArgs& a, double min_prob, double target_total) {
   a.min_prob = min_prob;
   a.target_total = target_total;
   a.z_skip = keep_z_bound(min_prob, target_total);
+  // a window that rises to its threshold holds at most this much identity (in bases): 19
+  // identical bases; 4 M + K in [76, 79] quarters with N; a score in (1889, 1989] whose
+  // hundredths are rounded by at most half a point per position
+  a.min_run[0] = keep_min_run(a.z_skip, 19.);
+  a.min_run[1] = keep_min_run(a.z_skip, 79. / 4.);
+  a.min_run[2] = keep_min_run(a.z_skip, 19.89 + 46. * 0.005);
   keep_band(min_prob, target_total, &a.keep_lo, &a.flag_hi);
 }
 
@@ -462,7 +471,8 @@ SXC_HD inline void push_run(Ex& ex, char* sm, int c0, int rank, int ns, int ne) 
 // edge at ns and the first clear flag after it at ne (or npos, where the loop ends) into
 // the run [ns, ne) -- the runs DoOne opens and closes.
 template <int NB, class Ex, class Flush>
-SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, int c0, int c1, int gsz, Flush&& flush) {
+SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, int c0, int c1, int gsz, int min_run,
+                                     bool count, Flush&& flush) {
   using SS = ScanSmem<NB>;
   constexpr int H = SS::N / 2;
   constexpr int WPL = SS::WPL;
@@ -580,7 +590,7 @@ SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, in
   // All listed blocks at once; if their runs overflowed the queue, again in rounds of blocks
   // that fit it (a word holds at most 16 rising edges), the queue flushed after each round.
   const int nrb = misc[SM_NRB];
-  auto extract = [&](int x0, int x1) {
+  auto extract = [&](int x0, int x1, bool count_runs) {
     ex.each([&](int tid) {
       for (int x = x0 + tid; x < x1; x += SCAN_NT) {
         const int e = rlist[x];
@@ -594,6 +604,7 @@ SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, in
         while (rises) {
           const int r = __builtin_ctz(rises);
           rises &= rises - 1;
+          if (count_runs) ex.atomic_add_shared(&misc[SM_RUNS], 1);  // (one atomic per wave)
           const uint32_t clear = ~f & (~0u << r);  // bit r is set: the first clear bit is above it
           int ne;
           if (clear) {
@@ -603,6 +614,9 @@ SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, in
             while (w2 < W && row[w2] == ~0u) ++w2;
             ne = w2 < W ? 32 * w2 + __builtin_ctz(~row[w2]) : npos;
           }
+          // Too short to be kept (keep_min_run).  A run that starts at 46, where DoOne's test
+          // begins, may have been above the threshold before, so the bound does not hold for it.
+          if (ne - (32 * w + r) < min_run && 32 * w + r != 46) continue;
           const int at = ex.atomic_add_shared(&misc[SM_QN], 1);  // one atomic per wave
           if (at < SS::QCAP)
             queue[at] = (int)((unsigned)j | ((unsigned)(32 * w + r) << SS::RB) | ((unsigned)ne << (SS::RB + SS::NSB)));
@@ -611,7 +625,7 @@ SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, in
     });
     ex.sync();
   };
-  extract(0, nrb);
+  extract(0, nrb, count);
   const int qn = misc[SM_QN];
   if (qn <= SS::QCAP) {
     flush(qn);
@@ -622,7 +636,7 @@ SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, in
     });
     ex.sync();
     for (int x0 = 0; x0 < nrb; x0 += SS::QCAP / 16) {
-      extract(x0, (x0 + SS::QCAP / 16 < nrb) ? x0 + SS::QCAP / 16 : nrb);
+      extract(x0, (x0 + SS::QCAP / 16 < nrb) ? x0 + SS::QCAP / 16 : nrb, false);
       flush(misc[SM_QN]);
     }
   }
@@ -636,7 +650,7 @@ SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, in
 // recomputes the window at its segment start, records the runs that open and close inside
 // its segment, and a second phase closes runs that cross segment boundaries.
 template <int NB, class Ex>
-SXC_HD inline void scan_epoch_segments(Ex& ex, char* sm, const uint16_t* cands, int c0, int c1, int gsz) {
+SXC_HD inline void scan_epoch_segments(Ex& ex, char* sm, const uint16_t* cands, int c0, int c1, int gsz, int min_run) {
   using SS = ScanSmem<NB>;
   constexpr int INF = 0x7fffffff;
   constexpr int H = SS::N / 2;
@@ -646,7 +660,11 @@ SXC_HD inline void scan_epoch_segments(Ex& ex, char* sm, const uint16_t* cands, 
   int* misc = (int*)(sm + SS::MISC);
   int* summ = (int*)(sm + SS::SUMM);
   const int Lt = misc[SM_LT], Lq = misc[SM_LQ];
-  auto push = [&](int rank, int ns, int ne) { push_run<NB>(ex, sm, c0, rank, ns, ne); };
+  auto push = [&](int rank, int ns, int ne) {
+    ex.atomic_add_shared(&misc[SM_RUNS], 1);
+    if (ne - ns < min_run && ns != 46) return;  // too short to be kept (see scan_epoch_bitmap)
+    push_run<NB>(ex, sm, c0, rank, ns, ne);
+  };
   ex.each([&](int tid) {
     const int c = c0 + tid / gsz;
     const int l = tid % gsz;
@@ -951,7 +969,7 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
   // this workgroup's share of the lags (all of them unless the scan is split)
   const int lo = (int)((int64_t)ncand * part / split), hi = (int)((int64_t)ncand * (part + 1) / split);
   constexpr int CE = SS::CE;
-  int runs = 0;
+  const int min_run = a.mode == 0 && !a.ptable ? a.min_run[SS::HASN ? 1 : SS::PURE ? 0 : 2] : 0;
   // Queue entries before the current epoch, kept per thread: every thread must see the same
   // count, and the shared counter may already hold the next epoch's pushes of a faster wave.
   int queued = 0;
@@ -959,9 +977,8 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
     const int qstart = queued;
     const int e1 = (e0 + CE < hi) ? e0 + CE : hi;
     if constexpr (SS::BMRUNS) {
-      scan_epoch_bitmap<NB>(ex, sm, cands, e0, e1, SS::GSZ, [&](int n) {
+      scan_epoch_bitmap<NB>(ex, sm, cands, e0, e1, SS::GSZ, min_run, a.stats != nullptr, [&](int n) {
         drain<NB>(ex, sm, a, pr, cands, ps, n, e0);
-        runs += n;
         ex.each([&](int tid) {
           if (tid == 0) misc[SM_QN] = 0;
         });
@@ -969,23 +986,26 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
       });
       continue;
     }
-    scan_epoch_segments<NB>(ex, sm, cands, e0, e1, SS::GSZ);
+    const int runs0 = misc[SM_RUNS];  // no thread pushes before the next barrier
+    ex.sync();
+    scan_epoch_segments<NB>(ex, sm, cands, e0, e1, SS::GSZ, min_run);
     const int qn = misc[SM_QN];
     ex.sync();  // every thread has read the count before any thread pushes again
     queued = qn;
     if (qn > SS::QCAP) {
       // the epoch overflowed the queue: keep what came before it, redo its lags one by one
       drain<NB>(ex, sm, a, pr, cands, ps, qstart, e0);  // (compact queue: empty)
-      runs += qstart;
+      ex.each([&](int tid) {
+        if (tid == 0) misc[SM_RUNS] = runs0;  // its runs are counted again below
+      });
       for (int c = e0; c < e1; ++c) {
         ex.each([&](int tid) {
           if (tid == 0) misc[SM_QN] = 0;
         });
         ex.sync();
-        scan_epoch_segments<NB>(ex, sm, cands, c, c + 1, SCAN_NT);
+        scan_epoch_segments<NB>(ex, sm, cands, c, c + 1, SCAN_NT, min_run);
         const int n1 = misc[SM_QN];
         drain<NB>(ex, sm, a, pr, cands, ps, n1, c);
-        runs += n1;
       }
       ex.each([&](int tid) {
         if (tid == 0) misc[SM_QN] = 0;
@@ -994,7 +1014,6 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
       queued = 0;
     } else if (SS::COMPACT || qn > SS::QCAP / 2 || e1 == hi) {
       drain<NB>(ex, sm, a, pr, cands, ps, qn, e0);
-      runs += qn;
       ex.each([&](int tid) {
         if (tid == 0) misc[SM_QN] = 0;
       });
@@ -1008,11 +1027,11 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
         a.counts[ps] = misc[SM_KEPT];
         if (a.stats) {
           a.stats[2 * ps] = ncand;
-          a.stats[2 * ps + 1] = runs;
+          a.stats[2 * ps + 1] = misc[SM_RUNS];
         }
       } else if (a.stats) {
         if (part == 0) a.stats[2 * ps] = ncand;
-        ex.atomic_add_global(&a.stats[2 * ps + 1], runs);
+        ex.atomic_add_global(&a.stats[2 * ps + 1], misc[SM_RUNS]);
       }
     }
   });

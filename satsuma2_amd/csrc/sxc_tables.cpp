@@ -182,6 +182,25 @@ double keep_z_bound(double min_prob, double target_size) {
   return hi;
 }
 
+int keep_min_run(double z_skip, double rise) {
+  // The run covers len = R + 45 positions (R = ne - ns flagged ones): the 46 of its first
+  // window and R - 1 more, so it holds m <= rise + R - 1 identical bases.  The tail's expected
+  // identity is p = (g h + (1 - g)(1 - h)) / 2, g and h the two sides' G/C fractions.  With an
+  // identity of rho = m / len, the identical positions add the same a to both sides' G/C and the
+  // others anything, so p is least where the rest is all G/C on one side and all A/T on the
+  // other and 2 a = m: p >= rho / 2 - rho^2 / 4.  (A letter of several bases is a mixture of such
+  // positions.)  (m - p len) / sqrt(p (1 - p) len) grows with m and as p falls, so z is at its
+  // lowest with the most identity and the least p.
+  if (!(z_skip < 0.)) return 1;
+  for (int R = 1; R < 4096; ++R) {
+    const double len = R + 45., m = fmin(rise + R - 1., len), rho = m / len;
+    const double p = rho / 2. - rho * rho / 4.;
+    const double z = (p * len - m) / sqrt(p * (1. - p) * len) / 1.414213562;
+    if (z < z_skip + 1e-6) return R;
+  }
+  return 1;
+}
+
 // ProbTable::Setup (analysis/ProbTable.cc:15-52) with GetMatchProbabilityRaw (:143-163):
 // for expected identity i / 511 and length j, the identity where exp(-cdf * size) stops
 // being 0, by bisection to a width of 1e-8 (the reference tests the probability for non-zero,

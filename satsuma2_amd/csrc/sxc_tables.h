@@ -15,6 +15,9 @@ bool class_has_thirds(int c);
 int chunk_flags(const unsigned char* s, int len);
 // z above which a run's probability is certainly below min_prob (see sxc_scan.h tail).
 double keep_z_bound(double min_prob, double target_size);
+// The shortest flagged stretch (ne - ns of a run [ns, ne), ns > 46) whose run can reach a z below
+// z_skip when the window at its start holds at most `rise` identical bases; at least 1.
+int keep_min_run(double z_skip, double rise);
 // ProbTable thresholds for a target size: SXC_PT_ROWS x SXC_PT_LEN doubles (row 0 unused).
 void build_prob_table(double target_size, double* t);
 
