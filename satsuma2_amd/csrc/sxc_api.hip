@@ -1249,7 +1249,7 @@ int sxc_matchup(sxc_ctx* ctx, const char* q, int32_t lq, const char* t, int32_t 
   a.cap = slot;
   sxc::ScanKinds kinds;
   kinds.pairs[sxc::scan_kind(hb.tchunks[0].flags, hb.qchunks[0].flags)] = 1;
-  HIPCHK(sxc::launch_scan(nb, a, 1, kinds, false, s));
+  HIPCHK(sxc::launch_scan(nb, a, 1, kinds, true, s));  // launch_peaks cleared the count
   int32_t cnt = 0;
   HIPCHK(hipMemcpyAsync(&cnt, d_misc + 1, sizeof cnt, hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));

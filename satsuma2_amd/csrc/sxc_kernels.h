@@ -28,6 +28,7 @@ hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& ki
 hipError_t launch_scan_pure(int nb, const ScanArgs& a, int grid, hipStream_t s);
 hipError_t launch_scan_n(int nb, const ScanArgs& a, int grid, hipStream_t s);
 hipError_t launch_scan_general(int nb, const ScanArgs& a, int grid, hipStream_t s);
+// ncand receives the number of accepted lags and, behind it, a zero.
 hipError_t launch_peaks(int nb, const float* xc, double cutoff, uint16_t* cands, int32_t* ncand, hipStream_t s);
 hipError_t launch_spectra(int geo, const SpecArgs& a, hipStream_t s);
 hipError_t launch_encode(int nb, const EncodeArgs& a, int n, hipStream_t s);

@@ -20,6 +20,7 @@ __global__ __launch_bounds__(Geo<NB>::NT) void k_peaks(const float* xc, double c
   Regs<NB> r;
   DevExec<Regs<NB>> ex{r};
   peaks_body<NB>(ex, sm, xc, cutoff, cands, ncand);
+  if (threadIdx.x == 0) ncand[1] = 0;  // the run count of a scan that follows (it may be split)
 }
 
 // Plain-API kernels ----------------------------------------------------------------
@@ -51,19 +52,51 @@ __global__ __launch_bounds__(Geo<NB>::NT) void k_xcorr(XcorrArgs a) {
   for (int p = threadIdx.x; p < Geo<NB>::N; p += Geo<NB>::NT) a.xc[(size_t)k * Geo<NB>::N + p] = Y[pad(p)];
 }
 
-// GetMatchProbabilityEx + PrintMatch identity for given runs (one thread per run).
-__global__ void k_prob(ProbArgs a) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+// GetMatchProbabilityEx + PrintMatch identity for given runs (one thread per run).  The sums are
+// the reference's, base after base, so a thread is a chain of additions; what they wait for is
+// read 16 bases ahead, through tables in LDS, and a workgroup is one wave so that a few hundred
+// runs spread over the CUs.  (1600 runs of two 3001-bp chunks: 85 us with every base's four
+// dependent reads from memory in the chain.)
+__global__ __launch_bounds__(64) void k_prob(ProbArgs a) {
+  __shared__ double equal[SXC_NCLASS * SXC_NCLASS], gc[SXC_NCLASS];
+  __shared__ unsigned char cls[128];
+  const sxc_tables* tab = a.tab;
+  for (int i = threadIdx.x; i < SXC_NCLASS * SXC_NCLASS; i += 64) equal[i] = (&tab->equal[0][0])[i];
+  for (int i = threadIdx.x; i < SXC_NCLASS; i += 64) gc[i] = tab->gc[i];
+  for (int i = threadIdx.x; i < 128; i += 64) cls[i] = tab->cls[i];
+  __syncthreads();
+  const int k = blockIdx.x * 64 + threadIdx.x;
   if (k >= a.n) return;
   const int32_t* r = a.runs + 3 * k;
   const int st = r[0], sq = r[1], len = r[2];
-  const sxc_tables* tab = a.tab;
+  const unsigned char *t = a.t + st, *q = a.q + sq;
   double matches = 0, gct = 0, gcq = 0;
-  for (int i = 0; i < len; ++i) {
-    const int ca = tab->cls[a.t[st + i] & 127], cb = tab->cls[a.q[sq + i] & 127];
-    matches += tab->equal[ca][cb];
-    gct += tab->gc[ca];
-    gcq += tab->gc[cb];
+  int i = 0;
+  for (; i + 16 <= len; i += 16) {
+    unsigned char tb[16], qb[16];
+    static_for<0, 16>([&](auto K) {
+      tb[decltype(K)::value] = t[i + decltype(K)::value];
+      qb[decltype(K)::value] = q[i + decltype(K)::value];
+    });
+    double e[16], gt[16], gq[16];
+    static_for<0, 16>([&](auto K) {
+      constexpr int x = decltype(K)::value;
+      const int ca = cls[tb[x] & 127], cb = cls[qb[x] & 127];
+      e[x] = equal[ca * SXC_NCLASS + cb];
+      gt[x] = gc[ca];
+      gq[x] = gc[cb];
+    });
+    static_for<0, 16>([&](auto K) {
+      matches += e[decltype(K)::value];
+      gct += gt[decltype(K)::value];
+      gcq += gq[decltype(K)::value];
+    });
+  }
+  for (; i < len; ++i) {
+    const int ca = cls[t[i] & 127], cb = cls[q[i] & 127];
+    matches += equal[ca * SXC_NCLASS + cb];
+    gct += gc[ca];
+    gcq += gc[cb];
   }
   const double ident = matches / (double)len;
   const double gc_target = gct / (double)len;
@@ -148,13 +181,25 @@ __global__ __launch_bounds__(256) void k_finalize(const sxc_result_dev* slots, c
   }
 }
 
-// Orders MatchUp runs by (lag rank, run start): rank by counting smaller keys.
-__global__ __launch_bounds__(256) void k_order_runs(const int32_t* runs, const uint64_t* keys, int n, int32_t* out) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const uint64_t ke = keys[e];
+// Orders MatchUp runs by (lag rank, run start): rank by counting smaller keys, 1024 of which the
+// workgroup reads into LDS at a time (1600 runs: 90 us with every thread reading every key from
+// memory).
+__global__ __launch_bounds__(64) void k_order_runs(const int32_t* runs, const uint64_t* keys, int n, int32_t* out) {
+  __shared__ uint64_t part[1024];
+  const int e = blockIdx.x * 64 + threadIdx.x;
+  const uint64_t ke = e < n ? keys[e] : 0;
   int rank = 0;
-  for (int k = 0; k < n; ++k) rank += keys[k] < ke;
+  for (int k0 = 0; k0 < n; k0 += 1024) {
+    const int m = n - k0 < 1024 ? n - k0 : 1024;
+    __syncthreads();
+    for (int k = threadIdx.x; k < m; k += 64) part[k] = keys[k0 + k];
+    __syncthreads();
+    int k = 0;
+    for (; k + 8 <= m; k += 8)
+      static_for<0, 8>([&](auto K) { rank += part[k + decltype(K)::value] < ke; });
+    for (; k < m; ++k) rank += part[k] < ke;
+  }
+  if (e >= n) return;
   out[3 * rank] = runs[3 * e];
   out[3 * rank + 1] = runs[3 * e + 1];
   out[3 * rank + 2] = runs[3 * e + 2];
@@ -164,7 +209,7 @@ __global__ __launch_bounds__(256) void k_order_runs(const int32_t* runs, const u
 
 hipError_t launch_order_runs(const int32_t* runs, const uint64_t* keys, int n, int32_t* out, hipStream_t s) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_order_runs, dim3((n + 255) / 256), dim3(256), 0, s, runs, keys, n, out);
+  hipLaunchKernelGGL(k_order_runs, dim3((n + 63) / 64), dim3(64), 0, s, runs, keys, n, out);
   return hipGetLastError();
 }
 
@@ -271,7 +316,7 @@ hipError_t launch_xcorr(int nb, const XcorrArgs& a, int n, hipStream_t s) {
 
 hipError_t launch_prob(const ProbArgs& a, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_prob, dim3((a.n + 255) / 256), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(k_prob, dim3((a.n + 63) / 64), dim3(64), 0, s, a);
   return hipGetLastError();
 }
 
