@@ -24,7 +24,7 @@ ARCH = os.environ.get("SXC_OFFLOAD_ARCH", "gfx950")
 COMMON = ["-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Wall", "-Wno-unused-function",
           "-Wno-unknown-pragmas"]
 DEVICE = [f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-SOURCES = ["sxc_kernels.hip", "sxc_kernels_r2.hip", "sxc_kernels_s32.hip", "sxc_kernels_occ.hip", "sxc_kernels_lean.hip",
+SOURCES = ["sxc_kernels.hip", "sxc_kernels_r2.hip", "sxc_kernels_s32.hip", "sxc_kernels_occ.hip", "sxc_kernels_lean.hip", "sxc_kernels_parts.hip",
            "sxc_scan_pure.hip", "sxc_scan_n.hip", "sxc_scan_general.hip", "sxc_api.hip",
            "sxc_server.hip", "sxc_static.hip", "sxc_tables.cpp", "sxc_kmatch.hip",
            # the master's side of the search (host C++): match sets, chaining, grid search

@@ -130,6 +130,7 @@ int batch_alloc(sxc_ctx* ctx, sxc_batch_dev& b) {
   HIPCHK(b.stats.ensure((size_t)total * 2 * sizeof(int32_t)));
   HIPCHK(b.offsets.ensure((size_t)total * sizeof(int64_t)));
   HIPCHK(b.total.ensure(2 * sizeof(int64_t)));
+  if (total <= sxc::CHANNEL_SPLIT) HIPCHK(b.parts.ensure((size_t)total * 4 * b.prm.N * sizeof(float)));
   HIPCHK(b.maxc.ensure(sizeof(int32_t)));
   const void* had = b.nflag.p;
   HIPCHK(b.nflag.ensure(sizeof(int32_t)));
@@ -164,6 +165,7 @@ int launch_correlate(sxc_ctx* ctx, sxc_batch_dev& b) {
   a.ncand = b.ncand.as<int32_t>();
   a.counts = b.counts.as<int32_t>();
   a.stats = b.stats.as<int32_t>();
+  a.parts = total <= sxc::CHANNEL_SPLIT ? b.parts.as<float>() : nullptr;
   a.xc_out = nullptr;
   if (!b.hb.tails.empty()) {
     a.tails = b.tails.as<sxc_tail_dev>();
@@ -229,6 +231,7 @@ int launch_target_spectra(sxc_ctx* ctx, sxc_batch_dev& b) {
   sa.spectra = b.spectra.as<float>();
   sa.dst = b.which.as<int32_t>();
   sa.signals = nullptr;
+  sa.per_channel = sa.n <= sxc::CHANNEL_SPLIT;
   if (!b.hb.tails.empty()) {
     sa.chunk_tail = b.ttail.as<int32_t>();
     sa.tails = b.tails.as<sxc_tail_dev>();
@@ -277,7 +280,7 @@ uint64_t graph_signature(const sxc_ctx* ctx, const sxc_batch_dev& b) {
   auto mix = [&](uint64_t v) { h = (h ^ v) * 1099511628211ull; };
   for (const DevBuf* d : {&b.seq, &b.tch, &b.qch, &b.pairs, &b.spectra, &b.which, &b.slots, &b.keys, &b.counts,
                           &b.offsets, &b.total, &b.maxc, &b.final_, &b.stats, &b.cands, &b.ncand, &b.sch, &b.sstr,
-                          &b.tails, &b.segs, &b.ttail, &b.src_sig, &b.ent, &b.nflag})
+                          &b.tails, &b.segs, &b.ttail, &b.src_sig, &b.ent, &b.nflag, &b.parts})
     mix((uint64_t)(uintptr_t)d->p);
   mix((uint64_t)(uintptr_t)b.ptable);
   mix((uint64_t)(uintptr_t)b.h_ctl);
@@ -1188,9 +1191,12 @@ int sxc_xcorr(sxc_ctx* ctx, const float* tsig, const float* qsig, int32_t N, flo
   sa.spectra = ctx->p2.as<float>();
   sa.dst = ctx->p4.as<int32_t>() + 1;
   sa.signals = ctx->p0.as<float>();
+  sa.per_channel = 1;
   HIPCHK(sxc::launch_spectra(nb, sa, s));
-  sxc::XcorrArgs xa{ctx->d_tab, ctx->d_osc, ctx->p2.as<float>(), ctx->p1.as<float>(), ctx->p3.as<float>()};
-  HIPCHK(sxc::launch_xcorr(nb, xa, 1, s));
+  // (the target's signals are not needed any more: the channels' correlations take their place)
+  sxc::XcorrArgs xa{ctx->d_tab, ctx->d_osc, ctx->p2.as<float>(), ctx->p1.as<float>(), ctx->p3.as<float>(),
+                    ctx->p0.as<float>()};
+  HIPCHK(sxc::launch_xcorr(nb, xa, s));
   HIPCHK(hipMemcpyAsync(xc, ctx->p3.p, (size_t)N * sizeof(float), hipMemcpyDeviceToHost, s));
   HIPCHK(hipStreamSynchronize(s));
   return SXC_OK;

@@ -61,6 +61,7 @@ struct sxc_batch_dev {
   DevBuf seq, tch, qch, pairs, spectra, which, slots, keys, counts, offsets, total, maxc, final_, stats, cands, ncand;
   DevBuf sch, sstr, tails, segs, ttail, src_sig;  // signal tails
   DevBuf ent;    // host-computed window entropies of chunks with B/D/H/V letters
+  DevBuf parts;  // channel correlations of a small batch (sxc::CHANNEL_SPLIT)
   DevBuf nflag;  // records the last scan flagged near min_prob (the counts kernel reads and clears it)
   sxc::HostBatch hb;
   sxc::ScanKinds kinds;  // of hb.pairs
@@ -90,7 +91,7 @@ struct sxc_batch_dev {
     if (s) (void)hipStreamSynchronize(s);
     if (gexec) (void)hipGraphExecDestroy(gexec), gexec = nullptr;
     for (DevBuf* b : {&seq, &tch, &qch, &pairs, &spectra, &which, &slots, &keys, &counts, &offsets, &total, &maxc,
-                      &final_, &stats, &cands, &ncand, &sch, &sstr, &tails, &segs, &ttail, &src_sig, &ent, &nflag})
+                      &final_, &stats, &cands, &ncand, &sch, &sstr, &tails, &segs, &ttail, &src_sig, &ent, &nflag, &parts})
       b->release();
     for (hipEvent_t& e : ev)
       if (e) (void)hipEventDestroy(e), e = nullptr;

@@ -32,7 +32,12 @@ hipError_t launch_scan_general(int nb, const ScanArgs& a, int grid, hipStream_t 
 hipError_t launch_peaks(int nb, const float* xc, double cutoff, uint16_t* cands, int32_t* ncand, hipStream_t s);
 hipError_t launch_spectra(int geo, const SpecArgs& a, hipStream_t s);
 hipError_t launch_encode(int nb, const EncodeArgs& a, int n, hipStream_t s);
-hipError_t launch_xcorr(int nb, const XcorrArgs& a, int n, hipStream_t s);
+hipError_t launch_xcorr(int nb, const XcorrArgs& a, hipStream_t s);
+// Launches of at most this many (pair, strand)s, or chunks, take a workgroup per channel
+// (PairArgs.parts, SpecArgs.per_channel): up to two workgroups per CU.
+constexpr int CHANNEL_SPLIT = 128;
+hipError_t launch_correlate_parts(int nb, const PairArgs& a, int total, hipStream_t s);
+hipError_t launch_spectra_parts(int nb, const SpecArgs& a, hipStream_t s);
 hipError_t launch_prob(const ProbArgs& a, hipStream_t s);
 hipError_t launch_order_runs(const int32_t* runs, const uint64_t* keys, int n, int32_t* out, hipStream_t s);
 // Exclusive scan of the per-(pair, strand) record counts (clipped at cap) into offsets, their

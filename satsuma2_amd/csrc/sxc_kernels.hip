@@ -45,11 +45,18 @@ __global__ __launch_bounds__(Geo<NB>::NT) void k_xcorr(XcorrArgs a) {
   for (int i = threadIdx.x; i < SXC_LUT_LEN; i += Geo<NB>::NT) lut[i] = a.tab->lut[i];
   __syncthreads();
   const Twiddle tw{lut, a.osc};
-  const int k = blockIdx.x;
-  correlate<NB>(ex, sm, a.tab, tw, SeqView{nullptr, nullptr, 0, 0}, a.spectra + (size_t)k * 4 * Geo<NB>::N,
-                a.qsig + (size_t)k * 4 * Geo<NB>::N, TailRef{nullptr, 0, nullptr});
+  // a workgroup per channel; k_sum_channels adds them
+  const int ch = blockIdx.x;
+  correlate<NB>(ex, sm, a.tab, tw, SeqView{nullptr, nullptr, 0, 0}, a.spectra, a.qsig, TailRef{nullptr, 0, nullptr},
+                nullptr, ch, ch + 1);
   const float* Y = (const float*)(sm + SM::Y);
-  for (int p = threadIdx.x; p < Geo<NB>::N; p += Geo<NB>::NT) a.xc[(size_t)k * Geo<NB>::N + p] = Y[pad(p)];
+  for (int p = threadIdx.x; p < Geo<NB>::N; p += Geo<NB>::NT) a.parts[(size_t)ch * Geo<NB>::N + p] = Y[pad(p)];
+}
+
+// A split CrossCorrelate's second half (XcorrArgs.parts): xc = 0 + A + C + G + T.
+__global__ __launch_bounds__(256) void k_sum_channels(const float* parts, int N, float* xc) {
+  const int p = blockIdx.x * 256 + threadIdx.x;
+  if (p < N) xc[p] = (((0.f + parts[p]) + parts[N + p]) + parts[2 * N + p]) + parts[3 * N + p];
 }
 
 // GetMatchProbabilityEx + PrintMatch identity for given runs (one thread per run).  The sums are
@@ -261,6 +268,7 @@ int fft_geometries(int nb, int* out, int cap) {
 }
 
 hipError_t launch_correlate(int geo, const PairArgs& a, int total, hipStream_t s) {
+  if (a.parts) return launch_correlate_parts(geo_nb(geo), a, total, s);
   const FftEntry* e = fft_entry(geo);
   return e ? e->correlate(a, total, s) : hipErrorInvalidValue;
 }
@@ -296,6 +304,7 @@ hipError_t launch_peaks(int nb, const float* xc, double cutoff, uint16_t* cands,
 }
 
 hipError_t launch_spectra(int geo, const SpecArgs& a, hipStream_t s) {
+  if (a.per_channel) return launch_spectra_parts(geo_nb(geo), a, s);
   const FftEntry* e = fft_entry(geo);
   return e ? e->spectra(a, s) : hipErrorInvalidValue;
 }
@@ -307,10 +316,11 @@ hipError_t launch_encode(int nb, const EncodeArgs& a, int n, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_xcorr(int nb, const XcorrArgs& a, int n, hipStream_t s) {
-#define CALL(X) hipLaunchKernelGGL(k_xcorr<X>, dim3(n), dim3(Geo<X>::NT), 0, s, a)
+hipError_t launch_xcorr(int nb, const XcorrArgs& a, hipStream_t s) {
+#define CALL(X) hipLaunchKernelGGL(k_xcorr<X>, dim3(4), dim3(Geo<X>::NT), 0, s, a)
   SXC_NB_SWITCH(nb, CALL)
 #undef CALL
+  hipLaunchKernelGGL(k_sum_channels, dim3((1 << nb) / 256), dim3(256), 0, s, a.parts, 1 << nb, a.xc);
   return hipGetLastError();
 }
 

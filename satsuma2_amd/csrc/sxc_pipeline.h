@@ -49,6 +49,10 @@ struct PairArgs {
   const float* qspectra;
   int32_t* counts;               // optional: set to 0 per (pair, strand) for a split scan
   int32_t* stats;                // optional: {candidates, runs} per (pair, strand), runs set to 0 for it
+  // optional: 4*N floats per (pair, strand).  A workgroup then correlates one channel and leaves
+  // it here, and sum_peaks_body adds the four: for launches too small to fill the device, whose
+  // time is one workgroup's four channels in a row.
+  float* parts;
 };
 
 struct SpecArgs {
@@ -68,6 +72,7 @@ struct SpecArgs {
   const sxc_tail_seg_dev* segs;
   const float* src_sig;
   int32_t strand;            // 1: spectra of the reverse complement (resident query spectra)
+  int32_t per_channel;       // 1: a workgroup per channel (launches too small to fill the device)
 };
 
 struct EncodeArgs {
@@ -84,9 +89,10 @@ struct EncodeArgs {
 struct XcorrArgs {
   const sxc_tables* tab;
   const float* osc;
-  const float* spectra;      // 4*N target spectra per item
-  const float* qsig;         // 4*N query signals per item
-  float* xc;                 // N floats per item
+  const float* spectra;      // 4*N target spectra
+  const float* qsig;         // 4*N query signals
+  float* xc;                 // N floats
+  float* parts;              // 4*N floats: the channels' correlations
 };
 
 struct ProbArgs {
@@ -541,7 +547,7 @@ SXC_HD inline void encode_body(Ex& ex, char* sm, const EncodeArgs& a, int k) {
 
 // One workgroup per chunk: the four channel spectra (FFTReal layout) to global memory.
 template <int NB, class Ex>
-SXC_HD inline void spectra_body(Ex& ex, char* sm, const SpecArgs& a, int k) {
+SXC_HD inline void spectra_body(Ex& ex, char* sm, const SpecArgs& a, int k, int ch0 = 0, int ch1 = 4) {
   using SM = Smem<NB>;
   using G = Geo<NB>;
   const sxc_chunk ck = a.chunks[a.which[k]];
@@ -562,7 +568,7 @@ SXC_HD inline void spectra_body(Ex& ex, char* sm, const SpecArgs& a, int k) {
   const TailRef tail =
       tail_ref<NB>(a.tails, a.segs, a.src_sig, a.chunk_tail ? a.chunk_tail[a.which[k]] : -1);
   if (!a.signals) class_cache<NB>(ex, qs);
-  for (int ch = 0; ch < 4; ++ch) {
+  for (int ch = ch0; ch < ch1; ++ch) {
     const float* given = a.signals ? a.signals + ((size_t)k * 4 + ch) * G::N : nullptr;
     forward_channel<NB, true>(ex, sm, a.tab, tw, qs, ch, given, tail);
     ex.each([&](int tid) {
@@ -580,11 +586,12 @@ SXC_HD inline void spectra_body(Ex& ex, char* sm, const SpecArgs& a, int k) {
 // ---------------------------------------------------------------- correlate
 
 // xc = (((0 + A) + C) + G) + T of rescaled, fftshifted channel correlations, left in
-// natural order in Y.  Per-thread accumulators stay in registers across channels.
+// natural order in Y.  Per-thread accumulators stay in registers across channels.  Channels
+// [ch0, ch1) only, where a workgroup takes one of them.
 template <int NB, class Ex>
 SXC_HD inline void correlate(Ex& ex, char* sm, const sxc_tables* tab, const Twiddle& tw, const SeqView& qs,
                              const float* T4, const float* qsig4, const TailRef& tail,
-                             const float* qspec4 = nullptr) {
+                             const float* qspec4 = nullptr, int ch0 = 0, int ch1 = 4) {
   using SM = Smem<NB>;
   using G = Geo<NB>;
   float* Y = (float*)(sm + SM::Y);
@@ -596,11 +603,11 @@ SXC_HD inline void correlate(Ex& ex, char* sm, const sxc_tables* tab, const Twid
   if constexpr (pair_class_cache<NB>()) {
     if (!qspec4 && !qsig4) class_cache<NB>(ex, qs);
   }
-  for (int ch = 0; ch < 4; ++ch) {
+  for (int ch = ch0; ch < ch1; ++ch) {
     if (qspec4) {
       // the load below writes Y with another thread mapping than the previous channel's
       // inverse stage A read it: every thread must have read before any thread writes
-      if (ch > 0) ex.sync();
+      if (ch > ch0) ex.sync();
       const float* qch = qspec4 + (size_t)ch * G::N;
       ex.each([&](int tid) {
         float* yt = Y + pad(tid);
@@ -745,12 +752,33 @@ SXC_HD inline void peaks(Ex& ex, char* sm, double cutoff) {
   ex.sync();
 }
 
+// FindTop of the correlation in Y; the accepted lags (ascending) go to global memory for the
+// scan kernel.
+template <int NB, class Ex>
+SXC_HD inline void store_lags(Ex& ex, char* sm, const PairArgs& a, int ps, int fast) {
+  using SM = Smem<NB>;
+  using G = Geo<NB>;
+  peaks<NB>(ex, sm, fast ? a.cutoff_fast : a.cutoff);
+  const int* misc = (const int*)(sm + SM::MISC);
+  const uint16_t* cand = (const uint16_t*)(sm + SM::CAND);
+  const int n = misc[MISC_NCAND];
+  uint16_t* dst = a.cands + (size_t)ps * G::N;
+  ex.each([&](int tid) {
+    for (int i = tid; i < n; i += G::NT) dst[i] = cand[i];
+    if (tid == 0) {
+      a.ncand[ps] = n;
+      if (a.counts) a.counts[ps] = 0;
+      if (a.stats) a.stats[2 * ps + 1] = 0;
+    }
+  });
+}
+
 // ---------------------------------------------------------------- fused correlate body
 
 // One workgroup per (pair, strand): encode -> FFT -> product -> iFFT -> channel sum ->
 // FindTop; the accepted lags (ascending) go to global memory for the scan kernel.
 template <int NB, class Ex>
-SXC_HD inline void correlate_body(Ex& ex, char* sm, const PairArgs& a, int ps) {
+SXC_HD inline void correlate_body(Ex& ex, char* sm, const PairArgs& a, int ps, int ch0 = 0, int ch1 = 4) {
   using SM = Smem<NB>;
   using G = Geo<NB>;
   const int pair = ps / a.strands;
@@ -770,12 +798,20 @@ SXC_HD inline void correlate_body(Ex& ex, char* sm, const PairArgs& a, int ps) {
     ex.sync();
     correlate<NB>(ex, sm, a.tab, tw, SeqView{nullptr, nullptr, qc.len, 0}, a.spectra + (size_t)pr.t_chunk * 4 * G::N,
                   nullptr, TailRef{nullptr, 0, nullptr},
-                  a.qspectra + ((size_t)pr.q_chunk * 2 + strand) * 4 * G::N);
+                  a.qspectra + ((size_t)pr.q_chunk * 2 + strand) * 4 * G::N, ch0, ch1);
   } else {
     const SeqView qs = phase_prepare<NB>(ex, sm, a.tab, a.ent_lut, ent_row(a.ent_rows, qc, strand), a.seq + qc.off,
                                          qc.len, qc.flags & 1, strand);
     correlate<NB>(ex, sm, a.tab, tw, qs, a.spectra + (size_t)pr.t_chunk * 4 * G::N, nullptr,
-                  tail_ref<NB>(a.tails, a.segs, a.src_sig, pr.q_tail));
+                  tail_ref<NB>(a.tails, a.segs, a.src_sig, pr.q_tail), nullptr, ch0, ch1);
+  }
+  if (a.parts) {
+    const float* Y = (const float*)(sm + SM::Y);
+    float* out = a.parts + ((size_t)ps * 4 + ch0) * G::N;
+    ex.each([&](int tid) {
+      for (int p = tid; p < G::N; p += G::NT) out[p] = Y[pad(p)];
+    });
+    return;
   }
   if (a.xc_out) {
     const float* Y = (const float*)(sm + SM::Y);
@@ -783,19 +819,27 @@ SXC_HD inline void correlate_body(Ex& ex, char* sm, const PairArgs& a, int ps) {
       for (int p = tid; p < G::N; p += G::NT) a.xc_out[(size_t)ps * G::N + p] = Y[pad(p)];
     });
   }
-  peaks<NB>(ex, sm, pr.fast ? a.cutoff_fast : a.cutoff);
-  const int* misc = (const int*)(sm + SM::MISC);
-  const uint16_t* cand = (const uint16_t*)(sm + SM::CAND);
-  const int n = misc[MISC_NCAND];
-  uint16_t* dst = a.cands + (size_t)ps * G::N;
+  store_lags<NB>(ex, sm, a, ps, pr.fast);
+}
+
+// The second half of a split launch: a (pair, strand)'s four channels summed in their order (as
+// the accumulators of correlate are: 0 + A + C + G + T), then FindTop.
+template <int NB, class Ex>
+SXC_HD inline void sum_peaks_body(Ex& ex, char* sm, const PairArgs& a, int ps) {
+  using SM = Smem<NB>;
+  using G = Geo<NB>;
+  float* Y = (float*)(sm + SM::Y);
+  int* misc0 = (int*)(sm + SM::MISC);
+  const float* in = a.parts + (size_t)ps * 4 * G::N;
   ex.each([&](int tid) {
-    for (int i = tid; i < n; i += G::NT) dst[i] = cand[i];
-    if (tid == 0) {
-      a.ncand[ps] = n;
-      if (a.counts) a.counts[ps] = 0;
-      if (a.stats) a.stats[2 * ps + 1] = 0;
-    }
+    static_for<0, G::N / G::NT>([&](auto K) {
+      const int p = tid + decltype(K)::value * G::NT;
+      Y[pad(p)] = (((0.f + in[p]) + in[G::N + p]) + in[2 * G::N + p]) + in[3 * G::N + p];
+    });
+    if (tid < 16) misc0[tid] = 0;
   });
+  ex.sync();
+  store_lags<NB>(ex, sm, a, ps, a.pairs[ps / a.strands].fast);
 }
 
 // FindTop on a given xc (the first half of SeqAnalyzer::MatchUp, analysis/CrossCorr.cc:583-592).

@@ -79,6 +79,7 @@ struct Slot {
   hipStream_t s = nullptr;
   hipEvent_t ev_start = nullptr, ev_count = nullptr, ev_pack = nullptr;
   DevBuf pairs, cands, ncand, outs, keys, counts, offsets, total, maxc, final_;
+  DevBuf parts;                     // channel correlations of small launches, where the budget has room
   sxc_pair_dev* h_pairs = nullptr;  // pinned
   int64_t* h_offsets = nullptr;     // pinned, 2 * P + 1 (the last entry is the total)
   int32_t* h_maxc = nullptr;        // pinned
@@ -165,7 +166,7 @@ int slot_alloc(sxc_server* sv, Slot& sl) {
 
 void slot_free(Slot& sl) {
   for (DevBuf* b : {&sl.pairs, &sl.cands, &sl.ncand, &sl.outs, &sl.keys, &sl.counts, &sl.offsets, &sl.total,
-                    &sl.maxc, &sl.final_})
+                    &sl.maxc, &sl.final_, &sl.parts})
     b->release();
   if (sl.h_pairs) (void)hipHostFree(sl.h_pairs);
   if (sl.h_offsets) (void)hipHostFree(sl.h_offsets);
@@ -299,6 +300,7 @@ int slot_fill(sxc_server* sv, Slot& sl) {
   a.cands = sl.cands.as<uint16_t>();
   a.ncand = sl.ncand.as<int32_t>();
   a.qspectra = sv->qspec_bytes > 0 ? sv->qspectra.as<float>() : nullptr;
+  a.parts = 2 * sl.npairs <= sxc::CHANNEL_SPLIT ? sl.parts.as<float>() : nullptr;
   a.counts = sl.counts.as<int32_t>();  // cleared per (pair, strand) for a split scan
   HIPCHK(sxc::launch_correlate(sv->geo_corr, a, 2 * sl.npairs, sl.s));
   int rc = launch_scan_slot(sv, sl, true, true);
@@ -595,6 +597,10 @@ int server_init(sxc_server* sv, const sxc_chunk_desc* targets, int32_t nt, const
     rc = slot_alloc(sv, sl);
     if (rc) return rc;
   }
+  // small launches split their channels where what the budget leaves holds the slots' parts
+  const int64_t parts = (int64_t)sxc::CHANNEL_SPLIT * 4 * N * (int64_t)sizeof(float);
+  if (room - nslots * sv->slot_bytes >= nslots * parts)
+    for (Slot& sl : sv->slots) HIPCHK(sl.parts.ensure((size_t)parts));
   return SXC_OK;
 }
 
