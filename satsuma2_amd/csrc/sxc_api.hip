@@ -164,7 +164,6 @@ int launch_correlate(sxc_ctx* ctx, sxc_batch_dev& b) {
   a.cands = b.cands.as<uint16_t>();
   a.ncand = b.ncand.as<int32_t>();
   a.counts = b.counts.as<int32_t>();
-  a.stats = b.stats.as<int32_t>();
   a.parts = total <= sxc::CHANNEL_SPLIT ? b.parts.as<float>() : nullptr;
   a.xc_out = nullptr;
   if (!b.hb.tails.empty()) {
@@ -199,7 +198,7 @@ int launch_pairs(sxc_ctx* ctx, sxc_batch_dev& b, bool fresh) {
   a.keys = b.keys.as<uint64_t>();
   a.counts = b.counts.as<int32_t>();
   a.cap = b.slot_cap;
-  a.stats = b.stats.as<int32_t>();
+  a.stats = b.want_stats ? b.stats.as<int32_t>() : nullptr;
   if (b.prm.prob_table) {
     a.ptable = b.ptable;
     a.table_prob = b.prm.table_prob;
@@ -856,6 +855,7 @@ int sxc_align_batch(sxc_ctx* ctx, const sxc_pair* pairs, int32_t n, const sxc_pa
   for (Group& gr : gs) {
     gr.b = (prm->N != 0) ? &ctx->scratch : &ctx->scratch_nb[gr.nb];
     gr.b->use_graph = false;  // new inputs every call: launched kernel by kernel
+    gr.b->want_stats = false;  // only a resident batch is asked for them (sxc_batch_stats)
   }
   rc = groups_prepare(gs, pairs, n, prm, nullptr, nullptr);
   if (rc) return rc;

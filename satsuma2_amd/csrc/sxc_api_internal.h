@@ -83,6 +83,7 @@ struct sxc_batch_dev {
   // The run's launch sequence captured as a graph, replayed while the buffers it was
   // captured with (signature) stay in place.
   bool use_graph = true;
+  bool want_stats = true;   // count the scan's runs (sxc_batch_stats)
   bool last_graph = false;  // the last run replayed the graph
   int runs = 0;
   hipGraphExec_t gexec = nullptr;

@@ -21,9 +21,8 @@ inline int scan_kind(int32_t tflags, int32_t qflags) {
 struct ScanKinds {
   int32_t pairs[3] = {0, 0, 0};
 };
-// Scans the accepted lags of `total` (pair, strand)s.  can_split: counts (and the run counts of
-// stats) are zero, so that a launch too small to fill the device may share a strand's lags
-// between several workgroups.
+// Scans the accepted lags of `total` (pair, strand)s.  can_split: counts are zero, so that a
+// launch too small to fill the device may share a strand's lags between several workgroups.
 hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& kinds, bool can_split, hipStream_t s);
 hipError_t launch_scan_pure(int nb, const ScanArgs& a, int grid, hipStream_t s);
 hipError_t launch_scan_n(int nb, const ScanArgs& a, int grid, hipStream_t s);

@@ -19,7 +19,7 @@ __global__ __launch_bounds__(Geo<NB>::NT) void k_correlate_part(PairArgs a) {
   Regs<NB> r;
   DevExec<Regs<NB>> ex{r};
   const int b = (int)blockIdx.x;
-  correlate_body<NB>(ex, sm, a, b >> 2, b & 3, (b & 3) + 1);
+  correlate_body<NB, true>(ex, sm, a, b >> 2, b & 3, (b & 3) + 1);
 }
 
 template <int NB>

@@ -48,7 +48,6 @@ struct PairArgs {
   // and forward transforms (the spectra are those transforms' output, bit for bit)
   const float* qspectra;
   int32_t* counts;               // optional: set to 0 per (pair, strand) for a split scan
-  int32_t* stats;                // optional: {candidates, runs} per (pair, strand), runs set to 0 for it
   // optional: 4*N floats per (pair, strand).  A workgroup then correlates one channel and leaves
   // it here, and sum_peaks_body adds the four: for launches too small to fill the device, whose
   // time is one workgroup's four channels in a row.
@@ -128,8 +127,9 @@ struct Smem {
   static constexpr int OFF = ENV + 8 * NENV;                   // double[4] channel means
   static constexpr int DSUM = OFF + 32;                        // double[4] sequential sums
   static constexpr int MISC = DSUM + 32;                       // int32[16]
-  static constexpr int CODEC = MISC + 64;                      // double[18][4]; DNA_X - off[X] after prepare
-  static constexpr int CLS = CODEC + 8 * 4 * SXC_NCLASS;       // uchar[128] byte -> class
+  static constexpr int CODEC = MISC + 64;                      // double[18][4]; DNA_X - off[X] after prepare;
+                                                               // a last row of zeros (CLASS_PAST)
+  static constexpr int CLS = CODEC + 8 * 4 * (SXC_NCLASS + 1); // uchar[128] byte -> class
   static constexpr int QUART = CLS + 128;                      // uchar[18][4], read a row at a time
   static_assert(QUART % 4 == 0, "quarter rows are read as words");
   static constexpr int RCT = QUART + 4 * SXC_NCLASS;           // uchar[128] byte -> class of its complement
@@ -154,6 +154,9 @@ SXC_HD inline const float* twiddle_table(const char* sm, const sxc_tables* tab) 
   }
 }
 
+
+// The class cache's entry for positions past the chunk's end: their signal is e * 0 = 0.
+constexpr unsigned CLASS_PAST = SXC_NCLASS;
 
 enum { MISC_L = 0, MISC_THIRDS = 1, MISC_NCAND = 2, MISC_KEPT = 3, MISC_Q4 = 4 /* 4 ints */, MISC_RUNS = 8 };
 
@@ -246,6 +249,11 @@ SXC_HD inline SeqView phase_prepare(Ex& ex, char* sm, const sxc_tables* tab, con
         q[i] = strand ? tab->cls[tab->rc[src[L - 1 - i] & 127] & 127] : tab->cls[src[i] & 127];
     }
     if (tid < 16) misc[tid] = 0;
+    if (tid < 4) codec[4 * CLASS_PAST + tid] = 0.;
+    // entropy weights are 1 in chunks below 1024 (analysis/CrossCorr.cc:39-44); windows past the
+    // chunk hold no position that counts
+    float* ew = (float*)(sm + SM::ENT);
+    for (int w = tid; w < SM::NWIN; w += G::NT) ew[w] = L < 1024 ? 1.f : 0.f;
   });
   ex.sync();
   SeqView qs;
@@ -440,7 +448,7 @@ SXC_HD inline void class_cache(Ex& ex, const SeqView& qs) {
       uint32_t w = 0;
       static_for<0, 4>([&](auto B) {
         const int p = stageA_pos<NB>(g, 4 * decltype(W)::value + decltype(B)::value);
-        if (p < qs.L) w |= (uint32_t)qs[p] << (8 * decltype(B)::value);
+        w |= (p < qs.L ? (uint32_t)qs[p] : CLASS_PAST) << (8 * decltype(B)::value);
       });
       rg.cls[decltype(W)::value] = w;
     });
@@ -503,7 +511,37 @@ SXC_HD inline void forward_channel(Ex& ex, char* sm, const sxc_tables* tab, cons
     if (g >= G::GROUPS) return;
     const Regs<NB>& rg = ex.template reg<Regs<NB>>(g);
     float v[G::SA];
-    if constexpr (CACHED) {
+    if (CACHED && !given && !tail.n) {
+      // Slot r of group g is position stageA_hi(r) + bitrev(g), its class in the cache, its window
+      // weight one read at a constant offset, and odd slots lie past N/2, where most chunks have
+      // ended.  Testing every position against the chunk's end, in both halves, and looking the
+      // weight up by position took 0.817 against 0.730 ms per 4096 pairs at N = 8192 and 0.272
+      // against 0.237 ms for their target spectra.  (Without the cache, at N >= 16384 in the pair
+      // kernel, the old form is the faster one: 0.71 against 0.86 ms at 32768, where it spills.)
+      constexpr int WSH = G::LOG - 9;  // log2 of the window, N / 512
+      const int low = (int)bitrev((unsigned)g, G::LOG - G::LSA);
+      const float* ent = (const float*)(sm + SM::ENT) + (low >> WSH);
+      const double* diff = (const double*)(sm + SM::CODEC) + ch;
+      auto slots = [&](auto HALF) {
+        static_for<0, G::SA / 4>([&](auto W) {
+          uint32_t w = 0;
+          if constexpr (CACHED) w = fresh(rg.cls[decltype(W)::value]);
+          static_for<0, 2>([&](auto B) {
+            constexpr int r = 4 * decltype(W)::value + 2 * decltype(B)::value + decltype(HALF)::value;
+            const int p = stageA_hi<NB>(r) + low;
+            const unsigned c = CACHED ? (w >> (8 * (r % 4))) & 255u : p < qs.L ? qs[p] : CLASS_PAST;
+            const double e = (double)ent[stageA_hi<NB>(r) >> WSH];
+            v[r] = (float)(e * diff[4 * c]);
+          });
+        });
+      };
+      slots(std::integral_constant<int, 0>{});
+      if (qs.L > G::H) {
+        slots(std::integral_constant<int, 1>{});
+      } else {
+        static_for<0, G::SA / 2>([&](auto I) { v[2 * decltype(I)::value + 1] = 0.f; });
+      }
+    } else if constexpr (CACHED) {
       static_for<0, G::SA / 4>([&](auto W) {
         const uint32_t w = fresh(rg.cls[decltype(W)::value]);
         static_for<0, 4>([&](auto B) {
@@ -768,7 +806,6 @@ SXC_HD inline void store_lags(Ex& ex, char* sm, const PairArgs& a, int ps, int f
     if (tid == 0) {
       a.ncand[ps] = n;
       if (a.counts) a.counts[ps] = 0;
-      if (a.stats) a.stats[2 * ps + 1] = 0;
     }
   });
 }
@@ -777,7 +814,8 @@ SXC_HD inline void store_lags(Ex& ex, char* sm, const PairArgs& a, int ps, int f
 
 // One workgroup per (pair, strand): encode -> FFT -> product -> iFFT -> channel sum ->
 // FindTop; the accepted lags (ascending) go to global memory for the scan kernel.
-template <int NB, class Ex>
+// PART: only channels [ch0, ch1), left in a.parts.
+template <int NB, bool PART = false, class Ex>
 SXC_HD inline void correlate_body(Ex& ex, char* sm, const PairArgs& a, int ps, int ch0 = 0, int ch1 = 4) {
   using SM = Smem<NB>;
   using G = Geo<NB>;
@@ -805,7 +843,7 @@ SXC_HD inline void correlate_body(Ex& ex, char* sm, const PairArgs& a, int ps, i
     correlate<NB>(ex, sm, a.tab, tw, qs, a.spectra + (size_t)pr.t_chunk * 4 * G::N, nullptr,
                   tail_ref<NB>(a.tails, a.segs, a.src_sig, pr.q_tail), nullptr, ch0, ch1);
   }
-  if (a.parts) {
+  if constexpr (PART) {
     const float* Y = (const float*)(sm + SM::Y);
     float* out = a.parts + ((size_t)ps * 4 + ch0) * G::N;
     ex.each([&](int tid) {

@@ -186,7 +186,6 @@ extern "C" int sxc_align_pair_static(sxc_ctx* ctx, const sxc_pair* pair, const s
   a.cands = (uint16_t*)(base + L.cands);
   a.ncand = (int32_t*)(base + L.ncand);
   a.counts = (int32_t*)(base + L.counts);
-  a.stats = (int32_t*)(base + L.stats);
   HIPCHK(sxc::launch_correlate(ctx->geo_corr[nb], a, S, s));
   // the diagonal scan and the probability tail
   sxc::ScanArgs c{};
@@ -208,7 +207,6 @@ extern "C" int sxc_align_pair_static(sxc_ctx* ctx, const sxc_pair* pair, const s
   c.keys = (uint64_t*)(base + L.keys);
   c.counts = (int32_t*)(base + L.counts);
   c.cap = SXC_STATIC_RECORDS;
-  c.stats = (int32_t*)(base + L.stats);
   sxc::ScanKinds kinds;
   kinds.pairs[sxc::scan_kind(tch.flags, qch.flags)] = 1;
   HIPCHK(sxc::launch_scan(nb, c, S, kinds, true, s));
