@@ -3,10 +3,13 @@
 // One workgroup per (pair, strand).  SeqAnalyzer::DoOne (OPTIM_DOONE,
 // analysis/CrossCorr.cc:667-724) slides a 46-wide window of integer scores
 // (int)(100 * DNA_EqualAmb + 0.5) along the diagonal of each lag FindTop accepted and
-// opens a run while the window sum exceeds 1889.  Lags are taken in epochs of 8 or 16.
-// Pairs of pure A/C/G/T chunks (scan_epoch_bitmap): threads take whole 32-position blocks of
-// a lag, keep the window's flags in an LDS bitmap, and a second pass turns each rising edge
-// into a run.  Other pairs (scan_epoch_segments): a lag's diagonal is split into contiguous
+// opens a run while the window sum exceeds 1889.
+// Pairs of pure A/C/G/T chunks (scan_sliced): a thread moves 32 blocks of a lag by one position
+// per operation, one block in each bit of a word, and names the blocks whose runs may be kept;
+// those are scanned again position by position.  Other pairs take their lags in epochs of 8 or
+// 16.  A/C/G/T/N (scan_epoch_bitmap): threads take whole 32-position blocks of a lag, keep the
+// window's flags in an LDS bitmap, and a second pass turns each rising edge into a run.  The
+// rest (scan_epoch_segments): a lag's diagonal is split into contiguous
 // segments, one per thread; each thread recomputes the window at its segment start,
 // records the runs that open and close inside its segment, and a second phase closes runs
 // that cross segment boundaries.  Runs go to an LDS queue; the queue is drained by all
@@ -18,9 +21,12 @@
 // Queue capacity: the segment scans' queue holds every run one lag can produce (runs need
 // a below-threshold gap, so at most npos/2 + 1 per lag, npos <= N/2), and an epoch of
 // several lags that overflows is discarded and redone one lag at a time; the bitmap scan
-// re-extracts an overflowing epoch's runs in rounds that each fit its queue.
+// re-extracts an overflowing epoch's runs in rounds that each fit its queue, and the sliced scan
+// scans slices whose blocks overflow it again, as many as always fit.
 #pragma once
 #include <math.h>
+
+#include <type_traits>
 
 #include "sxc_fft.h"
 #include "sxc_tables.h"
@@ -91,10 +97,9 @@ constexpr int SXC_MIN_QUARTERS = SXC_WIN_THRESHOLD / 25 + 1;
 static_assert(25 * SXC_MIN_QUARTERS > SXC_WIN_THRESHOLD && 25 * (SXC_MIN_QUARTERS - 1) <= SXC_WIN_THRESHOLD, "");
 
 // NB: log2 N in bits 0-4; bit 5 selects the kernel for pairs whose two chunks are pure
-// A/C/G/T, whose LDS plan holds only the packed bases, the run queue and the counters (the
-// accepted lags are read from global memory), so twice as many of its workgroups share a
-// CU; bit 6 the same kernel for pairs of A/C/G/T/N chunks with an N (HASN: N masks beside
-// the packed bases).  The general kernel takes every other pair.  Each exits at once on the
+// A/C/G/T (SLICED); bit 6 the one for pairs of A/C/G/T/N chunks with an N (HASN), whose LDS plan
+// holds the packed bases, the N masks, the run queue and the counters (the accepted lags are read
+// from global memory).  The general kernel takes every other pair.  Each exits at once on the
 // others' pairs.
 template <int NB>
 struct ScanSmem {
@@ -102,24 +107,28 @@ struct ScanSmem {
   static constexpr bool HASN = (NB & 64) != 0;
   static constexpr bool PURE = (NB & 96) != 0;
   static constexpr int N = 1 << LOG;
+  // The pure kernel (SLICED) scans 32 blocks of a lag in the bits of a word (scan_sliced) and needs
+  // no bitmap: bit planes of the bases instead of the packed words, the staged lags, the queue
+  // of blocks and a run count per thread.
+  static constexpr bool SLICED = PURE && !HASN;
   // The segment scans' queue holds every run one lag can produce (npos / 2 + 1, npos <= N / 2);
   // the bitmap scan flushes its queue whenever it would overflow (896 entries keep its LDS
   // plan at N = 8192 within 20 KB, 8 workgroups per CU).
-  static constexpr int QCAP = (PURE ? 896 : N / 4 + 64);
-  static constexpr int PKW = N / 16 + 4;                // 2-bit packed words (+3 words of read-ahead)
+  static constexpr int QCAP = (SLICED ? (N / 16 < 1024 ? 1024 : N / 16) : PURE ? 896 : N / 4 + 64);
+  static constexpr int PKW = SLICED ? 0 : N / 16 + 4;   // 2-bit packed words (+3 words of read-ahead)
   static constexpr int TCODE = 0;                       // uchar[N] (general kernel)
   static constexpr int QCODE = TCODE + (PURE ? 0 : N);  // uchar[N] (general kernel)
-  static constexpr int TPK = QCODE + (PURE ? 0 : N);    // uint32[PKW]: 16 bases per word (pure A/C/G/T only)
+  static constexpr int TPK = QCODE + (PURE ? 0 : N);    // uint32[PKW]: 16 bases per word (HASN)
   static constexpr int QPK = TPK + 4 * PKW;             // uint32[PKW]
-  // The pure kernel (BMRUNS) keeps each epoch's flags in a bitmap of WPL words per lag and
+  // The kernel with N (BMRUNS) keeps each epoch's flags in a bitmap of WPL words per lag and
   // turns its rising edges into runs afterwards; the general kernel scans contiguous
   // segments per thread and stitches runs across them.  BMRUNS, and the general kernel from
   // N = 16384, take one epoch at a time (drained after every epoch) in
   // 4-byte queue entries {lag - first lag of the epoch (RB bits), ns (NSB = LOG - 1), ne
   // (LOG)}; otherwise 16-lag epochs accumulate in 8-byte entries {lag rank, ns | ne << 16}
   // until the queue is half full.
-  static constexpr bool BMRUNS = PURE;
-  static constexpr bool COMPACT = BMRUNS || LOG >= 14;
+  static constexpr bool BMRUNS = HASN;
+  static constexpr bool COMPACT = PURE || LOG >= 14;
   static constexpr int CE = LOG >= 14 ? 8 : 16;         // lags per epoch
   static constexpr int GSZ = SCAN_NT / CE;              // threads per lag in an epoch
   static constexpr int NSB = LOG - 1;                   // ns < N / 2
@@ -133,7 +142,14 @@ struct ScanSmem {
   static constexpr int SUMM = QUEUE + QE * QCAP;        // int2[SCAN_NT] (segments)
   static constexpr int BITMAP = SUMM;                   // uint32[CE][WPL] (BMRUNS)
   static constexpr int RLIST = BITMAP + 4 * CE * WPL;   // uint16[CE * WPL]: blocks with a rising edge (BMRUNS)
-  static constexpr int EQUAL = SUMM + (BMRUNS ? 6 * CE * WPL : 8 * SCAN_NT);  // double[18][18]
+  static constexpr int PLW = N / 32 + 2 + 34;           // plane words: blocks -2 .. of a scan that runs past the end
+  static constexpr int TPL = (SUMM + 7) & ~7;           // uint32[PLW][2]: low and high bits of 32 bases (SLICED)
+  static constexpr int QPL = TPL + 8 * PLW;
+  static constexpr int RPL = QUEUE;                     // uint32[N/32][2]: the query, reversed (before the scan)
+  static constexpr int LAGS = QPL + 8 * PLW;            // uint16[SLICE_LAGS]
+  static constexpr int RUNS = LAGS + 2 * 512;           // int32[SCAN_NT]
+  static constexpr int RANGE = RUNS + 4 * SCAN_NT;      // int32[2 * 32]: first lag with a slice, and how many have it
+  static constexpr int EQUAL = SLICED ? RANGE + 4 * 64 : SUMM + (BMRUNS ? 6 * CE * WPL : 8 * SCAN_NT);  // double[18][18]
   static constexpr int NTAB = PURE ? 0 : 1;             // the score tables (general kernel)
   static constexpr int GC = EQUAL + NTAB * 8 * SXC_NCLASS * SXC_NCLASS;  // double[18]
   static constexpr int SCORE = GC + NTAB * 8 * SXC_NCLASS;              // uchar[18][18]
@@ -143,7 +159,7 @@ struct ScanSmem {
   static constexpr int BYTES = MISC + 64 + 4 * CE;
 };
 
-enum { SM_QN = 0, SM_KEPT = 1, SM_RUNS = 2, SM_NCAND = 3, SM_LT = 4, SM_LQ = 5, SM_NRB = 7, SM_NPOS = 16 };
+enum { SM_QN = 0, SM_KEPT = 1, SM_RUNS = 2, SM_NCAND = 3, SM_LT = 4, SM_LQ = 5, SM_NRB = 7, SM_UNSORTED = 8, SM_NPOS = 16 };
 
 // Base code: class id (0..16) of a codec letter, or 128 | byte for a byte whose codec
 // row is zero.  Two bases are identical bytes iff their codes are equal.
@@ -204,12 +220,6 @@ SXC_HD inline uint64_t load32(const uint32_t* pk, int p) {  // 32 bases starting
   return (lo >> b) | ((uint64_t)pk[w + 2] << (64 - b));
 }
 
-SXC_HD inline uint64_t match_block(const uint32_t* tpk, const uint32_t* qpk, int ti, int qj, int k) {
-  if (k < 0) return 0;
-  const uint64_t x = load32(tpk, ti + 32 * k) ^ load32(qpk, qj + 32 * k);
-  return ~(x | (x >> 1)) & 0x5555555555555555ull;
-}
-
 SXC_HD inline int popc64(uint64_t v) { return __builtin_popcountll(v); }
 
 // bits [s, s + 32) of hi:lo, 0 <= s < 32 (a funnel shift: one v_alignbit)
@@ -239,6 +249,13 @@ SXC_HD inline void opaque(uint32_t& x) {
   asm("" : "+v"(x));
 #else
   (void)x;
+#endif
+}
+
+// Nothing is moved across this point by the instruction scheduler (no instruction).
+SXC_HD inline void keep_order() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_sched_barrier(0);
 #endif
 }
 
@@ -338,23 +355,7 @@ SXC_HD inline int window_count(uint64_t e0, uint64_t e1, uint64_t e2, int r) {
   return c;
 }
 
-// Counts over a run of pure A/C/G/T bases: identical positions and C/G bases of each
-// side.  The reference's double sums of 0/1 terms equal these counts exactly.
-SXC_HD inline void packed_counts(const uint32_t* tpk, const uint32_t* qpk, int st, int sq, int len, int& match,
-                                 int& gct, int& gcq) {
-  match = gct = gcq = 0;
-  for (int off = 0; off < len; off += 32) {
-    const int m = (len - off < 32) ? len - off : 32;
-    const uint64_t keep = (m == 32) ? ~0ull : ((1ull << (2 * m)) - 1);
-    const uint64_t tv = load32(tpk, st + off), qv = load32(qpk, sq + off);
-    const uint64_t x = tv ^ qv;
-    match += popc64(~(x | (x >> 1)) & 0x5555555555555555ull & keep);
-    gct += popc64((tv ^ (tv >> 1)) & 0x5555555555555555ull & keep);  // codes 1 (C), 2 (G)
-    gcq += popc64((qv ^ (qv >> 1)) & 0x5555555555555555ull & keep);
-  }
-}
-
-// The same counts where bases may be N (bit 2b of the N mask words set): identical A/C/G/T
+// Counts over a run of bases that may be N (bit 2b of the N mask words set): identical A/C/G/T
 // bases, positions with an N on either side, C/G bases and N bases of each side.
 SXC_HD inline void packed_counts_n(const uint32_t* tpk, const uint32_t* qpk, const uint32_t* tnk,
                                    const uint32_t* qnk, int st, int sq, int len, int& match, int& nk, int& gct,
@@ -462,9 +463,8 @@ SXC_HD inline void push_run(Ex& ex, char* sm, int c0, int rank, int ns, int ne) 
   }
 }
 
-// Pure A/C/G/T lags [c0, c1), gsz threads per lag.  Score = 100 * [match], and a window
-// sum > 1889 <=> >= 19 matches.  C(n) = C(n - 1) + m(n) - m(n - 46) with m(< 0) = 0 equals
-// the reference's running `match` (analysis/CrossCorr.cc:700-705).  Each thread takes whole
+// A/C/G/T/N lags [c0, c1), gsz threads per lag.  The window's counts are running sums with
+// m(< 0) = 0, as the reference's `match` (analysis/CrossCorr.cc:700-705).  Each thread takes whole
 // 32-position blocks of one lag, updates every position branch-free and stores the block's
 // flags (window above the threshold, positions >= 46 and < npos) in the epoch's LDS
 // bitmap.  A second pass over the bitmap words, spread over all threads, turns every rising
@@ -498,7 +498,7 @@ SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, in
     const int ti = g.i0, qj = g.i0 + g.shift;
     const int k0 = na >> 5, klast = (nb - 1) >> 5;
     uint16_t* rl = (uint16_t*)(sm + SS::RLIST);
-    if constexpr (SS::HASN) {
+    {
       // the window test 4 M + K >= 76 over M identical A/C/G/T bases (m bits) and K positions
       // with an N (k bits), byte-parallel from the 2-bit groups m(n) + 1 - m(n - 46) and
       // k(n) + 1 - k(n - 46) (window_flags_mk)
@@ -540,49 +540,7 @@ SXC_HD inline void scan_epoch_bitmap(Ex& ex, char* sm, const uint16_t* cands, in
         k2 = k1;
         k1 = kk0;
       }
-      return;
     }
-    uint64_t e2 = match_block(tpk, qpk, ti, qj, k0 - 2);
-    uint64_t e1 = match_block(tpk, qpk, ti, qj, k0 - 1);
-    const int C = window_count(e1, e2, match_block(tpk, qpk, ti, qj, k0 - 3), 31);  // C at 32 k0 - 1
-    uint32_t prev = (na - 1 >= 46 && C >= SXC_MIN_MATCHES) ? 1u : 0u;          // flag at 32 k0 - 1
-    uint32_t ub = byte_perm(0u, (uint32_t)(C + 128 - SXC_MIN_MATCHES), 0u);   // half_flags' u, every byte
-    // flags from n = 46: block 0 keeps none, block 1 its bits from 14, later blocks all
-    uint32_t keep = k0 == 0 ? 0u : (k0 == 1 ? 0xFFFFC000u : ~0u);
-    uint16_t* rlist = (uint16_t*)(sm + SS::RLIST);
-    // The block's 32 bases of each side are words w, w + 1, w + 2 shifted right by the
-    // diagonal's bit offset; word w + 2 of one block is word w of the next.
-    const int tb = (ti & 15) * 2, qb = (qj & 15) * 2;
-    const uint32_t* tw = tpk + (ti >> 4) + 2 * k0;
-    const uint32_t* qw = qpk + (qj >> 4) + 2 * k0;
-    uint32_t t0 = tw[0], q0 = qw[0];
-    uint32_t e1l = (uint32_t)e1, e1h = (uint32_t)(e1 >> 32), e2h = (uint32_t)(e2 >> 32);
-    uint32_t f = 0;
-    for (int k = k0; k <= klast; ++k, tw += 2, qw += 2) {
-      const uint32_t t1 = tw[1], t2 = tw[2], q1 = qw[1], q2 = qw[2];
-      const uint32_t xl = funnel32(t1, t0, tb) ^ funnel32(q1, q0, qb);
-      const uint32_t xh = funnel32(t2, t1, tb) ^ funnel32(q2, q1, qb);
-      t0 = t2;
-      q0 = q2;
-      const uint32_t e0l = ~(xl | (xl >> 1)) & 0x55555555u, e0h = ~(xh | (xh >> 1)) & 0x55555555u;
-      // m(n - 46) for the block: offsets r < 14 come from block k-2, r >= 14 from block k-1
-      const uint32_t ml = funnel32(e1l, e2h, 4), mh = funnel32(e1h, e1l, 4);
-      // 2-bit group r of z holds m(n) + 1 - m(n - 46), in {0, 1, 2}: no carry crosses a
-      // group, so each 32-bit half is one add
-      const uint32_t zl = e0l + (~ml & 0x55555555u);
-      const uint32_t zh = e0h + (~mh & 0x55555555u);
-      f = window_flags(zl, zh, ub) & keep;
-      keep = 0xFFFFC000u | (keep >> 18);
-      row[k] = f;
-      // (the same increment on every lane: one atomic per wave).  A rise past nb in the
-      // lag's last block only adds a list entry whose word (cut below) yields no run.
-      if (f & ~((f << 1) | prev)) rlist[ex.atomic_add_shared(&misc[SM_NRB], 1)] = (uint16_t)(j * WPL + k);
-      prev = f >> 31;
-      e2h = e1h;
-      e1l = e0l;
-      e1h = e0h;
-    }
-    if (nb - 32 * klast < 32) row[klast] = f & ((1u << (nb - 32 * klast)) - 1);  // the lag ends at npos
   });
   ex.sync();
   int* queue = (int*)(sm + SS::QUEUE);
@@ -720,11 +678,84 @@ SXC_HD inline void scan_epoch_segments(Ex& ex, char* sm, const uint16_t* cands, 
   ex.sync();
 }
 
-// Drains queue entries [0, n): mode 0 filters into t_results, mode 1 writes runs.
-// rank_base: the first lag of the epoch the entries come from (compact queue).
+// Two bit planes of 32 bases (bit b: the low and the high bit of base b's 2-bit code).
+struct alignas(8) BasePlanes {
+  uint32_t lo, hi;
+};
+
+// The low half's bits to the even positions, the high half's to the odd ones.
+SXC_HD inline uint32_t interleave16(uint32_t v) {
+  v = byte_perm(v, v, 0x03010200u);
+  uint32_t t = (v ^ (v >> 4)) & 0x00F000F0u;
+  v ^= t ^ (t << 4);
+  t = (v ^ (v >> 2)) & 0x0C0C0C0Cu;
+  v ^= t ^ (t << 2);
+  t = (v ^ (v >> 1)) & 0x22222222u;
+  return v ^ t ^ (t << 1);
+}
+
+SXC_HD inline uint32_t reverse_bits(uint32_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bitreverse32(x);
+#else
+  uint32_t r = 0;
+  for (int b = 0; b < 32; ++b) r |= ((x >> b) & 1u) << (31 - b);
+  return r;
+#endif
+}
+
+// Bases [32 w, 32 w + 32) of a chunk of A/C/G/T letters (zeros from len on), read 16 bytes at a
+// time: chunks start 16-byte aligned and are padded to whole 16 bytes.
+SXC_HD inline BasePlanes planes_of(const unsigned char* seq, int len, int w) {
+  struct alignas(16) Quad {
+    uint32_t v[4];
+  };
+  const Quad* p = (const Quad*)seq + 2 * w;
+  const int left = len - 32 * w;
+  BasePlanes r = {0, 0};
+  if (left <= 0) return r;
+  const Quad z = {{0, 0, 0, 0}};
+  const Quad a = p[0], b = left > 16 ? p[1] : z;
+  // code bits 0 and 1 of letter x are x1 ^ x2 and x2 ^ x3; byte i of word j goes to bit 8 i + j
+  static_for<0, 8>([&](auto J) {
+    constexpr int j = decltype(J)::value;
+    const uint32_t v = j < 4 ? a.v[j & 3] : b.v[j & 3];
+    const uint32_t y = v ^ (v >> 1);
+    r.lo |= ((y >> 1) & 0x01010101u) << j;
+    r.hi |= ((y >> 2) & 0x01010101u) << j;
+  });
+  // bit 8 i + j to bit 4 j + i: the bit's index turned by two places
+  const uint32_t keep = left >= 32 ? ~0u : (1u << left) - 1;
+  r.lo = interleave16(interleave16(r.lo)) & keep;
+  r.hi = interleave16(interleave16(r.hi)) & keep;
+  return r;
+}
+
+// 32 bases from base p >= -64 on (the planes start two words before base 0)
+SXC_HD inline BasePlanes planes_at(const BasePlanes* pl, int p) {
+  const BasePlanes* w = pl + 2 + (p >> 5);
+  const BasePlanes a = w[0], b = w[1];
+  return BasePlanes{funnel32(b.lo, a.lo, p & 31), funnel32(b.hi, a.hi, p & 31)};
+}
+
+// Counts over a run of pure A/C/G/T bases: identical positions and C/G bases of each side.  The
+// reference's double sums of 0/1 terms equal these counts exactly.
+SXC_HD inline void plane_counts(const BasePlanes* tpl, const BasePlanes* qpl, int st, int sq, int len, int& match,
+                                int& gct, int& gcq) {
+  match = gct = gcq = 0;
+  for (int off = 0; off < len; off += 32) {
+    const uint32_t keep = len - off < 32 ? (1u << (len - off)) - 1 : ~0u;
+    const BasePlanes t = planes_at(tpl, st + off), q = planes_at(qpl, sq + off);
+    match += popc64(keep & ~((t.lo ^ q.lo) | (t.hi ^ q.hi)));
+    gct += popc64(keep & (t.lo ^ t.hi));  // codes 1 (C), 2 (G)
+    gcq += popc64(keep & (q.lo ^ q.hi));
+  }
+}
+
+// One run through the tail: mode 0 filters it into t_results, mode 1 writes it.
 template <int NB, class Ex>
-SXC_HD inline void drain(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev& pr, const uint16_t* cands, int ps,
-                         int n, int rank_base) {
+SXC_HD inline void drain_run(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev& pr, const uint16_t* cands, int ps,
+                             int rank, int ns, int ne) {
   using SS = ScanSmem<NB>;
   constexpr int H = SS::N / 2;
   const unsigned char* tc = (const unsigned char*)(sm + SS::TCODE);
@@ -732,8 +763,116 @@ SXC_HD inline void drain(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev
   const double* equal = (const double*)(sm + SS::EQUAL);
   const double* gcv = (const double*)(sm + SS::GC);
   int* misc = (int*)(sm + SS::MISC);
-  const int* queue = (const int*)(sm + SS::QUEUE);
   const int strand = ps % a.strands;
+  const int shift = (int)cands[rank] - H;
+  const int i0 = shift < 0 ? -shift : 0;
+  const int start_t = i0 + ns - SXC_MIN_LEN;
+  const int len = ne - ns + SXC_MIN_LEN;
+  const int start_q = start_t + shift;
+  const uint64_t key = ((uint64_t)(uint32_t)rank << 32) | (uint32_t)ns;
+  if (a.mode == 1) {
+    const int slot = a.split > 1 ? ex.atomic_add_global(&a.counts[ps], 1) : ex.atomic_add_shared(&misc[SM_KEPT], 1);
+    if (slot >= a.cap) return;
+    const size_t at = (size_t)ps * a.cap + slot;
+    a.runs[3 * at] = start_t;
+    a.runs[3 * at + 1] = start_q;
+    a.runs[3 * at + 2] = len;
+    a.keys[at] = key;
+    return;
+  }
+  if (len < a.min_len) return;  // FilterMatches: GetLength() < m_minLen
+  double ident, prob = 0.;
+  if constexpr (SS::HASN) {
+    int cm, nk, ct, ntn, cq, nqn;
+    packed_counts_n((const uint32_t*)(sm + SS::TPK), (const uint32_t*)(sm + SS::QPK),
+                    (const uint32_t*)(sm + SS::TNK), (const uint32_t*)(sm + SS::QNK), start_t, start_q, len, cm,
+                    nk, ct, ntn, cq, nqn);
+    // DNA_Equal of N against any base or N, and N's GC weight, are quarter multiples, so
+    // the reference's running sums equal these products exactly
+    const double matches = (double)cm + a.tab->equal[SXC_CLASS_N][0] * (double)nk;
+    const double gct = (double)ct + a.tab->gc[SXC_CLASS_N] * (double)ntn;
+    const double gcq = (double)cq + a.tab->gc[SXC_CLASS_N] * (double)nqn;
+    if (a.ptable) {
+      prob = table_from_sums(matches, gct, gcq, len, a.ptable, a.table_prob, ident);
+    } else if ((nk == 0 && z_clearly_skipped(cm, ct, cq, len, a.z_skip)) ||
+               !tail_from_sums(matches, gct, gcq, len, a.target_total, a.z_skip, prob, ident)) {
+      return;
+    }
+  } else if constexpr (SS::PURE) {
+    int cm, ct, cq;
+    plane_counts((const BasePlanes*)(sm + SS::TPL), (const BasePlanes*)(sm + SS::QPL), start_t, start_q, len, cm, ct,
+                 cq);
+    if (a.ptable) {
+      prob = table_from_sums((double)cm, (double)ct, (double)cq, len, a.ptable, a.table_prob, ident);
+    } else if (z_clearly_skipped(cm, ct, cq, len, a.z_skip) ||
+               !tail_from_sums((double)cm, (double)ct, (double)cq, len, a.target_total, a.z_skip, prob, ident)) {
+      return;
+    }
+  } else {
+    double matches = 0, gct = 0, gcq = 0;
+    for (int i = 0; i < len; ++i) {
+      const int ca = code_class(tc[start_t + i]), cb = code_class(qc[start_q + i]);
+      matches += equal[ca * SXC_NCLASS + cb];
+      gct += gcv[ca];
+      gcq += gcv[cb];
+    }
+    if (a.ptable) {
+      prob = table_from_sums(matches, gct, gcq, len, a.ptable, a.table_prob, ident);
+    } else if (!tail_from_sums(matches, gct, gcq, len, a.target_total, a.z_skip, prob, ident)) {
+      return;
+    }
+  }
+  // FilterMatches keeps prob >= m_minProb.  The table's decision is exact; the device's
+  // erf/exp may differ from glibc's by a few ulp, so a probability within the keep band
+  // of min_prob is written flagged and decided on the host with glibc.
+  bool near = false;
+  if (a.ptable) {
+    if (prob < a.min_prob) return;
+  } else {
+    if (prob < a.keep_lo) return;
+    near = prob < a.flag_hi;
+  }
+  const int slot = a.split > 1 ? ex.atomic_add_global(&a.counts[ps], 1) : ex.atomic_add_shared(&misc[SM_KEPT], 1);
+  if (slot >= a.cap) return;
+  const int tstart = pr.t_chunk_start + start_t;
+  // RCQuery (analysis/HomologyByXCorrSlave.cc:56-60) on the reverse strand, with the
+  // -q_chunk size (slave) or, for q_chunk == 0, the query chunk's own length (the
+  // standalone aligner, tools/analysis/HomologyByXCorr.cc:226-228, 793-798)
+  const int rc_chunk = a.q_chunk > 0 ? a.q_chunk : a.qchunks[pr.q_chunk].len;
+  const int qstart =
+      strand == 0 ? pr.q_chunk_start + start_q : start_q + pr.q_record_len - pr.q_chunk_start - rc_chunk;
+  sxc_result_dev r;
+  r.query_id = (uint64_t)(int64_t)pr.q_record;
+  r.target_id = (uint64_t)(int64_t)pr.t_record;
+  r.query_size = (uint64_t)(int64_t)pr.q_record_len;
+  r.qstart = (uint64_t)(int64_t)qstart;
+  r.tstart = (uint64_t)(int64_t)tstart;
+  r.len = (uint64_t)(int64_t)len;
+  r.reverse = (uint8_t)(strand == 1);
+  for (int z = 0; z < 7; ++z) r.pad_[z] = 0;
+  if (near) {
+    const uint32_t pi = (uint32_t)(ps / a.strands);  // the pair, for the host's decision
+    r.pad_[0] = SXC_REC_NEAR;
+    r.pad_[1] = (uint8_t)pi;
+    r.pad_[2] = (uint8_t)(pi >> 8);
+    r.pad_[3] = (uint8_t)(pi >> 16);
+    r.pad_[4] = (uint8_t)(pi >> 24);
+    if (a.nflag) ex.atomic_add_global(a.nflag, 1);
+  }
+  r.prob = prob;
+  r.ident = ident;
+  const size_t at = (size_t)ps * a.cap + slot;
+  a.out[at] = r;
+  a.keys[at] = key;
+}
+
+// Drains queue entries [0, n): mode 0 filters into t_results, mode 1 writes runs.
+// rank_base: the first lag of the epoch the entries come from (compact queue).
+template <int NB, class Ex>
+SXC_HD inline void drain(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev& pr, const uint16_t* cands, int ps,
+                         int n, int rank_base) {
+  using SS = ScanSmem<NB>;
+  const int* queue = (const int*)(sm + SS::QUEUE);
   ex.each([&](int tid) {
     for (int k = tid; k < n; k += SCAN_NT) {
       int rank, ns, ne;
@@ -747,107 +886,391 @@ SXC_HD inline void drain(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev
         ns = queue[2 * k + 1] & 0xffff;
         ne = (queue[2 * k + 1] >> 16) & 0xffff;
       }
-      const int shift = (int)cands[rank] - H;
-      const int i0 = shift < 0 ? -shift : 0;
-      const int start_t = i0 + ns - SXC_MIN_LEN;
-      const int len = ne - ns + SXC_MIN_LEN;
-      const int start_q = start_t + shift;
-      const uint64_t key = ((uint64_t)(uint32_t)rank << 32) | (uint32_t)ns;
-      if (a.mode == 1) {
-        const int slot = a.split > 1 ? ex.atomic_add_global(&a.counts[ps], 1) : ex.atomic_add_shared(&misc[SM_KEPT], 1);
-        if (slot >= a.cap) continue;
-        const size_t at = (size_t)ps * a.cap + slot;
-        a.runs[3 * at] = start_t;
-        a.runs[3 * at + 1] = start_q;
-        a.runs[3 * at + 2] = len;
-        a.keys[at] = key;
+      drain_run<NB>(ex, sm, a, pr, cands, ps, rank, ns, ne);
+    }
+  });
+  ex.sync();
+}
+
+// ---- pairs of pure A/C/G/T chunks: 32 blocks of a lag in the bits of a word (scan_sliced)
+
+// Bit i of word j becomes bit j of word i.
+SXC_HD inline void transpose32(uint32_t* x) {
+  static_for<0, 16>([&](auto K) {
+    constexpr int k = decltype(K)::value;
+    const uint32_t p = x[k], q = x[k + 16];
+    x[k] = byte_perm(q, p, 0x05040100u);
+    x[k + 16] = byte_perm(q, p, 0x07060302u);
+    if constexpr (k % 4 == 3) keep_order();
+  });
+  static_for<0, 16>([&](auto K) {
+    constexpr int k = (decltype(K)::value & 7) | ((decltype(K)::value & 8) << 1);
+    const uint32_t p = x[k], q = x[k + 8];
+    x[k] = byte_perm(q, p, 0x06020400u);
+    x[k + 8] = byte_perm(q, p, 0x07030501u);
+    if constexpr (decltype(K)::value % 4 == 3) keep_order();
+  });
+  auto stage = [&](auto S, uint32_t low) {
+    constexpr int s = decltype(S)::value;
+    static_for<0, 16>([&](auto K) {
+      constexpr int k = (decltype(K)::value & (s - 1)) | ((decltype(K)::value & ~(s - 1)) << 1);
+      const uint32_t p = x[k], q = x[k + s];
+      x[k] = bit_select(low, p, q << s);
+      x[k + s] = bit_select(low, p >> s, q);
+      opaque(x[k]);  // (else the masked halves are kept apart for the next stage, and spilled)
+      opaque(x[k + s]);
+      if constexpr (decltype(K)::value % 4 == 3) keep_order();
+    });
+  };
+  stage(std::integral_constant<int, 4>{}, 0x0F0F0F0Fu);
+  stage(std::integral_constant<int, 2>{}, 0x33333333u);
+  stage(std::integral_constant<int, 1>{}, 0x55555555u);
+}
+
+// s + 2 c = x + y + z in every bit position
+SXC_HD inline void add3(uint32_t x, uint32_t y, uint32_t z, uint32_t& s, uint32_t& c) {
+  s = x ^ y ^ z;
+  c = (x & y) | (z & (x | y));
+}
+
+// The sum of x[0 .. 7] in every bit position: digits s[0 .. 3].
+SXC_HD inline void sum8(const uint32_t* x, uint32_t* s) {
+  uint32_t a, A, b, B, c, C, D, e, E, F;
+  add3(x[0], x[1], x[2], a, A);
+  add3(x[3], x[4], x[5], b, B);
+  add3(x[6], x[7], a, c, C);
+  s[0] = b ^ c;
+  D = b & c;
+  add3(A, B, C, e, E);
+  s[1] = e ^ D;
+  F = e & D;
+  s[2] = E ^ F;
+  s[3] = E & F;
+}
+
+// r = x + y over W digits (what does not fit is known to be zero)
+template <int W>
+SXC_HD inline void sum_digits(const uint32_t* x, const uint32_t* y, uint32_t* r) {
+  uint32_t carry = 0;
+  static_for<0, W>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+    uint32_t s, c;
+    add3(x[i], y[i], carry, s, c);
+    r[i] = s;
+    carry = c;
+  });
+}
+
+constexpr int SLICE_LAGS = 512;    // lags staged at a time
+constexpr int SLICE_BLOCKS = 29;   // blocks a slice decides (of the 32 it computes)
+
+// Slice t of a lag: bit b of a word stands for block 29 t + b - 2.  Bits 0 and 1 are the windows'
+// history, bit 2 the flags before the slice; bits 3 to 31 are the blocks the slice decides (block 0
+// has no flags, DoOne's test begins at n = 46).  Returns the blocks holding a position where the
+// flags have been set `gate` times in a row (d2, d4, d8: ~0 where the gate is below 2, 4, 8), and
+// in block 1 also a run that starts at 46; *rises counts the runs that start in the blocks.
+SXC_HD inline uint32_t slice_blocks(const BasePlanes* tpl, const BasePlanes* qpl, const Lag& g, int t, uint32_t d2,
+                                    uint32_t d4, uint32_t d8, int* rises) {
+  // x[i] bit b: position i of block b differs (words of the planes are offset by two blocks)
+  uint32_t x[32];
+  {
+    const int qj = g.i0 + g.shift;
+    const int tb = g.i0 & 31, qb = qj & 31;
+    const BasePlanes* tw = tpl + (g.i0 >> 5) + SLICE_BLOCKS * t;
+    const BasePlanes* qw = qpl + (qj >> 5) + SLICE_BLOCKS * t;
+    BasePlanes t0 = tw[0], q0 = qw[0];
+    static_for<0, 32>([&](auto B) {
+      constexpr int b = decltype(B)::value;
+      const BasePlanes t1 = tw[b + 1], q1 = qw[b + 1];
+      x[b] = (funnel32(t1.lo, t0.lo, tb) ^ funnel32(q1.lo, q0.lo, qb)) |
+             (funnel32(t1.hi, t0.hi, tb) ^ funnel32(q1.hi, q0.hi, qb));
+      t0 = t1;
+      q0 = q1;
+      if constexpr (b % 4 == 3) keep_order();
+    });
+  }
+  transpose32(x);
+  keep_order();
+  // c: differences among the 46 positions before the block, plus 4: all 32 of the block before and
+  // the last 14 of the one before that.  At most 27 differences <=> bit 5 of the sum is clear.
+  uint32_t c[6];
+  {
+    uint32_t p[6] = {}, q[6] = {}, r[6] = {}, last[6] = {}, first[6] = {}, all[6];
+    sum8(x + 18, p);
+    keep_order();
+    const uint32_t rest[8] = {x[26], x[27], x[28], x[29], x[30], x[31], 0u, 0u};
+    sum8(rest, q);
+    sum_digits<4>(p, q, last);  // <= 14
+    keep_order();
+    sum8(x, p);
+    sum8(x + 8, q);
+    sum_digits<5>(p, q, r);
+    keep_order();
+    uint32_t two[6] = {x[16] ^ x[17], x[16] & x[17], 0u, 0u, 0u, 0u};
+    sum_digits<5>(r, two, first);  // <= 18
+    sum_digits<6>(first, last, all);
+    uint32_t carry = 0;
+    static_for<0, 6>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      uint32_t s, cy;
+      add3(all[i] << 1, last[i] << 2, carry, s, cy);
+      c[i] = s;
+      carry = cy;
+    });
+    uint32_t four = c[2];  // + 4
+    c[2] = ~c[2];
+    static_for<3, 6>([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      const uint32_t s = c[i] ^ four;
+      four = c[i] & four;
+      c[i] = s;
+    });
+    keep_order();
+  }
+  // blocks with n = 32 block + i inside the lag: ha up to i = e, hb after it
+  const int last = (g.npos - 1) >> 5, e = (g.npos - 1) & 31;
+  const int nb = last + 3 - SLICE_BLOCKS * t;
+  const uint32_t ha = nb >= 32 ? ~0u : (1u << nb) - 1;
+  const uint32_t hb = nb - 1 >= 32 ? ~0u : (1u << (nb - 1)) - 1;
+  const uint32_t la = t ? ~3u : ~15u, lb = t ? ~3u : ~7u;  // flags from n = 46; bits 0, 1 have no history
+  uint32_t any = 0, wrapped = 0, at46 = 0;
+  uint32_t runs = 0;
+  uint32_t f[40], r2[40], r4[40], r8[40];
+  auto gates = [&](auto I) {
+    constexpr int i = decltype(I)::value;
+    r2[i] = f[i] & ((i >= 1 ? f[i >= 1 ? i - 1 : 0] : 0u) | d2);
+    r4[i] = r2[i] & ((i >= 2 ? r2[i >= 2 ? i - 2 : 0] : 0u) | d4);
+    r8[i] = r4[i] & ((i >= 4 ? r4[i >= 4 ? i - 4 : 0] : 0u) | d8);
+  };
+  static_for<0, 32>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+    // the count moves up where position n differs and n - 46 does not, down for the opposite
+    const uint32_t old = i < 14 ? x[(i + 18) & 31] << 2 : x[(i - 14) & 31] << 1;
+    uint32_t m = x[i] ^ old;
+    static_for<0, 6>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      const uint32_t next = m & (c[j] ^ old);
+      c[j] ^= m;
+      m = next;
+    });
+    f[i] = ~c[5] & (i <= e ? ha : hb) & (i < 14 ? la : lb);
+    gates(I);
+    if constexpr (i >= 1) {
+      runs += __builtin_popcount(f[i] & ~f[i - 1] & ~7u);
+      opaque(runs);  // (one add per count)
+    }
+    if constexpr (i >= 8) any |= r8[i] & ~r8[i - 1];
+    if constexpr (i == 14) at46 = t ? 0u : f[i] & 8u;
+    keep_order();
+  });
+  // the first positions of the next block follow the last of this one
+  static_for<32, 40>([&](auto I) {
+    constexpr int i = decltype(I)::value;
+    f[i] = f[i - 32] >> 1;
+    gates(I);
+    if constexpr (i == 32) runs += __builtin_popcount(f[i] & ~f[i - 1] & ~3u);
+    wrapped |= r8[i] & ~r8[i - 1];
+  });
+  *rises = (int)runs;
+  return (any & ~7u) | ((wrapped & ~3u) << 1) | at46;
+}
+
+// The runs of block k of lag `rank` that were set `gate` times in a row for the first time inside
+// the block, found again position by position, and their tails.
+template <int NB, class Ex>
+SXC_HD inline void slice_runs(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev& pr, const uint16_t* cands,
+                              int ps, int rank, const Lag& g, int k, int gate, int min_run) {
+  using SS = ScanSmem<NB>;
+  const BasePlanes* tpl = (const BasePlanes*)(sm + SS::TPL);
+  const BasePlanes* qpl = (const BasePlanes*)(sm + SS::QPL);
+  auto match = [&](int b) {  // of block b >= -2
+    const BasePlanes t = planes_at(tpl, g.i0 + 32 * b), q = planes_at(qpl, g.i0 + g.shift + 32 * b);
+    return ~((t.lo ^ q.lo) | (t.hi ^ q.hi));
+  };
+  const int s = k - 1;  // k >= 1
+  uint32_t m2 = s < 2 ? 0u : match(s - 2), m1 = s < 1 ? 0u : match(s - 1);
+  const int C = popc64(m1) + popc64(m2 >> 18);  // at 32 s - 1
+  const uint32_t prev = (32 * s - 1 >= 46 && C >= SXC_MIN_MATCHES) ? 1u : 0u;
+  uint32_t ub = byte_perm(0u, (uint32_t)(C + 128 - SXC_MIN_MATCHES), 0u);  // half_flags' u, every byte
+  // flags of the next block, b (DoOne's positions only: 46 <= n < npos)
+  auto next_flags = [&](int b) {
+    const uint32_t m0 = match(b);
+    const uint32_t old = funnel32(m1, m2, 18);  // m(n - 46)
+    // 2-bit group r: m(n) + 1 - m(n - 46)
+    const uint32_t one = ~(m0 ^ old), two = m0 & ~old;
+    uint32_t f = window_flags(interleave16(byte_perm(two, one, 0x05040100u)),
+                              interleave16(byte_perm(two, one, 0x07060302u)), ub);
+    if (b < 2) f &= b == 0 ? 0u : 0xFFFFC000u;
+    if (g.npos - 32 * b < 32) f &= g.npos > 32 * b ? (1u << (g.npos - 32 * b)) - 1 : 0u;
+    m2 = m1;
+    m1 = m0;
+    return f;
+  };
+  const uint32_t f0 = next_flags(s);
+  const uint64_t f = (uint64_t)f0 | ((uint64_t)next_flags(k) << 32);
+  uint64_t rises = f & ~((f << 1) | prev) & (0xFFFFFFFFull << (33 - gate));
+  for (;;) {
+    // the next run that is long enough or still open: found by all lanes before any takes a tail
+    int ns = -1, ne = g.npos;
+    bool open = false;
+    while (ns < 0 && rises) {
+      const int r = __builtin_ctzll(rises);
+      rises &= rises - 1;
+      const uint64_t clear = ~f & (~0ull << r);
+      open = !clear;  // (the last run of the two blocks)
+      if (clear) ne = 32 * s + __builtin_ctzll(clear);
+      // Too short to be kept (keep_min_run).  A run that starts at 46, where DoOne's test begins,
+      // may have been above the threshold before, so the bound does not hold for it.
+      ns = 32 * s + r;
+      if (clear && ne - ns < min_run && ns != 46) ns = -1;
+    }
+    if (ns < 0) return;
+    if (open) {
+      ne = g.npos;
+      for (int b = k + 1; 32 * b < g.npos; ++b) {
+        const uint32_t fb = next_flags(b);
+        if (~fb) {
+          ne = 32 * b + __builtin_ctz(~fb);
+          break;
+        }
+      }
+      if (ne - ns < min_run && ns != 46) return;
+    }
+    drain_run<NB>(ex, sm, a, pr, cands, ps, rank, ns, ne);
+  }
+}
+
+// Pure A/C/G/T lags [lo, hi).  Score = 100 * [match], and a window sum > 1889 <=> >= 19 matches,
+// <=> <= 27 differences.  C(n) = C(n - 1) + m(n) - m(n - 46) with m(< 0) = 0 equals the reference's
+// running `match` (analysis/CrossCorr.cc:700-705).  A thread takes a slice of a lag, 32 blocks of
+// 32 positions, and transposes their difference words, so that one operation moves the 32 blocks'
+// counts by one position each; blocks with a run that may be kept (or any run, where all are
+// wanted) go to a queue, whose entries all threads take through slice_runs.
+// Vector issue bounds it: a slice takes some 1600 instructions (about 190 for the difference
+// words, 260 for the transposition, 130 for the first counts, 30 per position), 55 per block of 32
+// positions against 110 to 120 where a thread took one block at a time and 150 more before its
+// first, and 32 blocks share one start.  Of the 0.51 ms at N = 8192 the slices take 0.28 and the
+// named blocks about 0.2.  One launch, before (a block at a time) and now: 8192 strands at
+// N = 8192 0.80 and 0.51 ms, 24000 at 2048 3.59 and 1.46 ms, 40000 at 512 1.19 and 0.64 ms, 1000
+// at 32768 1.96 and 0.75 ms.
+template <int NB, class Ex>
+SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev& pr, const uint16_t* cands,
+                               int ps, int lo, int hi, int min_run) {
+  using SS = ScanSmem<NB>;
+  constexpr int H = SS::N / 2;
+  constexpr int SLICES = (SS::WPL - 1 + SLICE_BLOCKS - 1) / SLICE_BLOCKS;
+  static_assert(SLICES >= 1 && SLICES <= 32, "slices of a lag");
+  static_assert(32 * SLICE_BLOCKS <= SS::QCAP, "32 slices' blocks fit the queue");
+  int* misc = (int*)(sm + SS::MISC);
+  int* queue = (int*)(sm + SS::QUEUE);
+  uint16_t* lags = (uint16_t*)(sm + SS::LAGS);
+  int* first = (int*)(sm + SS::RANGE);  // of slice t: its first lag
+  int* many = first + 32;               // and how many lags have one
+  int* runs = (int*)(sm + SS::RUNS);
+  const BasePlanes* tpl = (const BasePlanes*)(sm + SS::TPL);
+  const BasePlanes* qpl = (const BasePlanes*)(sm + SS::QPL);
+  const int Lt = misc[SM_LT], Lq = misc[SM_LQ];
+  const int gate = min_run >= 8 ? 8 : min_run >= 4 ? 4 : min_run >= 2 ? 2 : 1;
+  const uint32_t d2 = gate >= 2 ? 0u : ~0u, d4 = gate >= 4 ? 0u : ~0u, d8 = gate >= 8 ? 0u : ~0u;
+  ex.each([&](int tid) { runs[tid] = 0; });
+  for (int c0 = lo; c0 < hi; c0 += SLICE_LAGS) {
+    const int nl = (hi - c0 < SLICE_LAGS) ? hi - c0 : SLICE_LAGS;
+    ex.each([&](int tid) {
+      for (int x = tid; x < nl; x += SCAN_NT) {
+        lags[x] = cands[c0 + x];
+        if (x && cands[c0 + x - 1] >= cands[c0 + x]) misc[SM_UNSORTED] = 1;
+      }
+    });
+    ex.sync();
+    // A lag has a slice t if npos >= P, which holds for an interval of shifts (npos is concave in
+    // the shift); lags given out of order all count as having it and are looked at one by one.
+    ex.each([&](int tid) {
+      if (tid >= SLICES) return;
+      const int P = 32 * (SLICE_BLOCKS * tid + 1) + 1;
+      int x0 = 0, x1 = nl;
+      if (!misc[SM_UNSORTED]) {
+        auto below = [&](int idx) {  // lags before idx
+          int u = 0, v = nl;
+          while (u < v) {
+            const int w = (u + v) >> 1;
+            if ((int)lags[w] < idx) {
+              u = w + 1;
+            } else {
+              v = w;
+            }
+          }
+          return u;
+        };
+        x0 = below(H + P - Lt + 1);
+        x1 = below(H + Lq - P + 1);
+      }
+      if (P > Lq || P > Lt - 1 || x1 < x0) x1 = x0;
+      first[tid] = x0;
+      many[tid] = x1 - x0;
+    });
+    ex.sync();
+    int total = 0;
+    for (int t = 0; t < SLICES; ++t) total += many[t];
+    // Blocks queued before the current slices, kept per thread: every thread must see the same
+    // count.  Slices whose blocks overflow the queue are scanned again, 32 at a time, whose blocks
+    // always fit an empty one; their runs are counted the first time (slices below `counted`).
+    int queued = 0, width = SCAN_NT, counted = 0;
+    for (int base = 0; base < total;) {
+      ex.each([&](int tid) {
+        int id = base + tid;
+        if (tid >= width || id >= total) return;
+        const bool count = id >= counted;
+        int t = 0;
+        while (id >= many[t]) id -= many[t++];
+        id += first[t];
+        const Lag g = lag_geometry(lags[id], H, Lq, Lt);
+        if (g.npos < 32 * (SLICE_BLOCKS * t + 1) + 1) return;
+        int rises;
+        uint32_t any = slice_blocks(tpl, qpl, g, t, d2, d4, d8, &rises);
+        runs[tid] += count ? rises : 0;
+        while (any) {
+          const int b = __builtin_ctz(any);
+          any &= any - 1;
+          const int at = ex.atomic_add_shared(&misc[SM_QN], 1);  // (one atomic per wave)
+          if (at < SS::QCAP) queue[at] = id | (SLICE_BLOCKS * t + b - 2) << 9;
+        }
+      });
+      ex.sync();
+      const int qn = misc[SM_QN];
+      ex.sync();  // every thread has read the count
+      const bool over = qn > SS::QCAP;
+      if (over) {
+        if (counted < base + width) counted = base + width;
+        width = 32;
+      } else {
+        base += width;
+        if (base >= counted) width = SCAN_NT;
+      }
+      if (!over && qn <= SS::QCAP / 2 && base < total) {
+        queued = qn;
         continue;
       }
-      if (len < a.min_len) continue;  // FilterMatches: GetLength() < m_minLen
-      double ident, prob = 0.;
-      if constexpr (SS::HASN) {
-        int cm, nk, ct, ntn, cq, nqn;
-        packed_counts_n((const uint32_t*)(sm + SS::TPK), (const uint32_t*)(sm + SS::QPK),
-                        (const uint32_t*)(sm + SS::TNK), (const uint32_t*)(sm + SS::QNK), start_t, start_q, len, cm,
-                        nk, ct, ntn, cq, nqn);
-        // DNA_Equal of N against any base or N, and N's GC weight, are quarter multiples, so
-        // the reference's running sums equal these products exactly
-        const double matches = (double)cm + a.tab->equal[SXC_CLASS_N][0] * (double)nk;
-        const double gct = (double)ct + a.tab->gc[SXC_CLASS_N] * (double)ntn;
-        const double gcq = (double)cq + a.tab->gc[SXC_CLASS_N] * (double)nqn;
-        if (a.ptable) {
-          prob = table_from_sums(matches, gct, gcq, len, a.ptable, a.table_prob, ident);
-        } else if ((nk == 0 && z_clearly_skipped(cm, ct, cq, len, a.z_skip)) ||
-                   !tail_from_sums(matches, gct, gcq, len, a.target_total, a.z_skip, prob, ident)) {
-          continue;
+      const int n = over ? queued : qn;
+      ex.each([&](int tid) {
+        for (int x = tid; x < n; x += SCAN_NT) {
+          const int id = queue[x] & (SLICE_LAGS - 1), k = queue[x] >> 9;
+          slice_runs<NB>(ex, sm, a, pr, cands, ps, c0 + id, lag_geometry(lags[id], H, Lq, Lt), k, gate, min_run);
         }
-      } else if constexpr (SS::PURE) {
-        int cm, ct, cq;
-        packed_counts((const uint32_t*)(sm + SS::TPK), (const uint32_t*)(sm + SS::QPK), start_t, start_q, len, cm,
-                      ct, cq);
-        if (a.ptable) {
-          prob = table_from_sums((double)cm, (double)ct, (double)cq, len, a.ptable, a.table_prob, ident);
-        } else if (z_clearly_skipped(cm, ct, cq, len, a.z_skip) ||
-                   !tail_from_sums((double)cm, (double)ct, (double)cq, len, a.target_total, a.z_skip, prob, ident)) {
-          continue;
-        }
-      } else {
-        double matches = 0, gct = 0, gcq = 0;
-        for (int i = 0; i < len; ++i) {
-          const int ca = code_class(tc[start_t + i]), cb = code_class(qc[start_q + i]);
-          matches += equal[ca * SXC_NCLASS + cb];
-          gct += gcv[ca];
-          gcq += gcv[cb];
-        }
-        if (a.ptable) {
-          prob = table_from_sums(matches, gct, gcq, len, a.ptable, a.table_prob, ident);
-        } else if (!tail_from_sums(matches, gct, gcq, len, a.target_total, a.z_skip, prob, ident)) {
-          continue;
-        }
-      }
-      // FilterMatches keeps prob >= m_minProb.  The table's decision is exact; the device's
-      // erf/exp may differ from glibc's by a few ulp, so a probability within the keep band
-      // of min_prob is written flagged and decided on the host with glibc.
-      bool near = false;
-      if (a.ptable) {
-        if (prob < a.min_prob) continue;
-      } else {
-        if (prob < a.keep_lo) continue;
-        near = prob < a.flag_hi;
-      }
-      const int slot = a.split > 1 ? ex.atomic_add_global(&a.counts[ps], 1) : ex.atomic_add_shared(&misc[SM_KEPT], 1);
-      if (slot >= a.cap) continue;
-      const int tstart = pr.t_chunk_start + start_t;
-      // RCQuery (analysis/HomologyByXCorrSlave.cc:56-60) on the reverse strand, with the
-      // -q_chunk size (slave) or, for q_chunk == 0, the query chunk's own length (the
-      // standalone aligner, tools/analysis/HomologyByXCorr.cc:226-228, 793-798)
-      const int rc_chunk = a.q_chunk > 0 ? a.q_chunk : a.qchunks[pr.q_chunk].len;
-      const int qstart =
-          strand == 0 ? pr.q_chunk_start + start_q : start_q + pr.q_record_len - pr.q_chunk_start - rc_chunk;
-      sxc_result_dev r;
-      r.query_id = (uint64_t)(int64_t)pr.q_record;
-      r.target_id = (uint64_t)(int64_t)pr.t_record;
-      r.query_size = (uint64_t)(int64_t)pr.q_record_len;
-      r.qstart = (uint64_t)(int64_t)qstart;
-      r.tstart = (uint64_t)(int64_t)tstart;
-      r.len = (uint64_t)(int64_t)len;
-      r.reverse = (uint8_t)(strand == 1);
-      for (int z = 0; z < 7; ++z) r.pad_[z] = 0;
-      if (near) {
-        const uint32_t pi = (uint32_t)(ps / a.strands);  // the pair, for the host's decision
-        r.pad_[0] = SXC_REC_NEAR;
-        r.pad_[1] = (uint8_t)pi;
-        r.pad_[2] = (uint8_t)(pi >> 8);
-        r.pad_[3] = (uint8_t)(pi >> 16);
-        r.pad_[4] = (uint8_t)(pi >> 24);
-        if (a.nflag) ex.atomic_add_global(a.nflag, 1);
-      }
-      r.prob = prob;
-      r.ident = ident;
-      const size_t at = (size_t)ps * a.cap + slot;
-      a.out[at] = r;
-      a.keys[at] = key;
+      });
+      ex.sync();
+      ex.each([&](int tid) {
+        if (tid == 0) misc[SM_QN] = 0;
+      });
+      ex.sync();
+      queued = 0;
     }
+    ex.each([&](int tid) {
+      if (tid == 0) misc[SM_UNSORTED] = 0;
+    });
+    ex.sync();
+  }
+  ex.each([&](int tid) {
+    if (a.stats) ex.atomic_add_shared(&misc[SM_RUNS], runs[tid]);
   });
   ex.sync();
 }
@@ -899,6 +1322,7 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
     if (tid == 0) {
       misc[SM_QN] = 0;
       misc[SM_NRB] = 0;
+      misc[SM_UNSORTED] = 0;
       misc[SM_KEPT] = 0;
       misc[SM_RUNS] = 0;
       misc[SM_NCAND] = a.ncand[ps];
@@ -908,7 +1332,43 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
   });
   ex.sync();
   const int Lt = tch.len, Lq = qch.len;
-  if constexpr (SS::PURE) {
+  if constexpr (SS::SLICED) {
+    // 2-bit codes A=0, C=1, G=2, T=3 from the ASCII letters (read from HBM); complement =
+    // code ^ 3.  Strand 1 (DNAVector::ReverseComplement, analysis/DNAVector.cc:482-521) turns the
+    // query's planes around.
+    BasePlanes* tpl = (BasePlanes*)(sm + SS::TPL);
+    BasePlanes* qpl = (BasePlanes*)(sm + SS::QPL);
+    ex.each([&](int tid) {
+      for (int w = tid; w < SS::PLW; w += SCAN_NT) {
+        const BasePlanes none = {0, 0};
+        const bool in = w >= 2 && w < 2 + N / 32;
+        tpl[w] = in ? planes_of(ts, Lt, w - 2) : none;
+        qpl[w] = in ? planes_of(qs, Lq, w - 2) : none;
+      }
+    });
+    ex.sync();
+    if (strand) {
+      BasePlanes* rpl = (BasePlanes*)(sm + SS::RPL);
+      ex.each([&](int tid) {
+        for (int w = tid; w < N / 32; w += SCAN_NT) {
+          const int p = Lq - 32 - 32 * w;  // first base of the word, reversed
+          BasePlanes r = {0, 0};
+          if (p > -32) {
+            const BasePlanes v = planes_at(qpl, p);
+            const uint32_t keep = p >= 0 ? ~0u : (1u << (32 + p)) - 1;
+            r.lo = ~reverse_bits(v.lo) & keep;
+            r.hi = ~reverse_bits(v.hi) & keep;
+          }
+          rpl[w] = r;
+        }
+      });
+      ex.sync();
+      ex.each([&](int tid) {
+        for (int w = tid; w < N / 32; w += SCAN_NT) qpl[w + 2] = rpl[w];
+      });
+      ex.sync();
+    }
+  } else if constexpr (SS::PURE) {
     // 2-bit codes A=0, C=1, G=2, T=3 from the ASCII letters (read from HBM); complement =
     // code ^ 3
     uint32_t* tpk = (uint32_t*)(sm + SS::TPK);
@@ -973,7 +1433,8 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
   // Queue entries before the current epoch, kept per thread: every thread must see the same
   // count, and the shared counter may already hold the next epoch's pushes of a faster wave.
   int queued = 0;
-  for (int e0 = lo; e0 < hi; e0 += CE) {
+  if constexpr (SS::SLICED) scan_sliced<NB>(ex, sm, a, pr, cands, ps, lo, hi, min_run);
+  for (int e0 = SS::SLICED ? hi : lo; e0 < hi; e0 += CE) {
     const int qstart = queued;
     const int e1 = (e0 + CE < hi) ? e0 + CE : hi;
     if constexpr (SS::BMRUNS) {
