@@ -278,14 +278,21 @@ hipError_t launch_correlate(int geo, const PairArgs& a, int total, hipStream_t s
   return e ? e->correlate(a, total, s) : hipErrorInvalidValue;
 }
 
-// Workgroups per (pair, strand) for n of them.  A strand's lags are taken 8 or 16 at a time, and
-// every workgroup packs both chunks first, so a share pays only while compute units are idle:
-// up to 2048 workgroups in all (8 per CU), more than 4 per strand only below 512.  Measured
-// at N = 8192, us of the pure kernel with 1 / 2 / 4 / 8 / 16 workgroups per strand: 2 strands
-// 109 / - / - / - / 16, 128 strands - / 17 / 18 / 22 / 29, 740 strands 195 / 120 / - / - / -.
-static int scan_split(int n) {
-  const int k = n > 0 ? std::min({2048 / n, std::max(4, 512 / n), 16}) : 1;
-  return std::max(1, k);
+// Workgroups per (pair, strand) for n of them.  Every workgroup packs both chunks first, so a
+// share pays only while compute units are idle.
+// Pure A/C/G/T: a share's slices also come in whole waves.  us with 1 / 2 / 4 / 8 / 16 workgroups
+// per strand at N = 8192: 2 strands 42 / 34 / 34 / 30 / 29, 32 strands 50 / 36 / 33 / 29 / 30, 128
+// strands 50 / 39 / 42 / 39 / 51, 512 strands 68 / 65 / 87 / 97 / 140, 1024 strands 99 / 102 /
+// 135 / 175 / 266 (N = 2048 the same within 10%); at N = 32768, with 4 times the lags and
+// positions: 32 strands 359 / 196 / 146 / 94 / 81, 128 strands 356 / 203 / 203 / 202 / 203, 512
+// strands 501 / 438 / 555 / - / -, 2048 strands 1434 / 1406 / 1965 / - / -.
+// With N or other letters, lags are taken 8 or 16 at a time: up to 2048 workgroups in all (8 per
+// CU), more than 4 per strand only below 512 (128 strands - / 17 / 18 / 22 / 29, 740 strands
+// 195 / 120 / - / - / -, with a kernel of that kind on A/C/G/T pairs).
+static int scan_split(int kind, int nb, int n) {
+  if (n <= 0) return 1;
+  if (kind == 0) return n <= 32 ? 16 : n <= 128 ? 8 : n <= (nb >= 14 ? 2048 : 768) ? 2 : 1;
+  return std::max(1, std::min({2048 / n, std::max(4, 512 / n), 16}));
 }
 
 hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& kinds, bool can_split, hipStream_t s) {
@@ -294,14 +301,14 @@ hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& ki
   // and not by the pair kernel, which one more store made 3% slower at N = 16384).
   if (can_split && a.stats)
     for (int k = 0; k < 3; ++k)
-      if (kinds.pairs[k] > 0 && scan_split(kinds.pairs[k] * a.strands) > 1) {
+      if (kinds.pairs[k] > 0 && scan_split(k, nb, kinds.pairs[k] * a.strands) > 1) {
         hipLaunchKernelGGL(k_clear_runs, dim3((total + 255) / 256), dim3(256), 0, s, a.stats, total);
         break;
       }
   for (int k = 0; k < 3; ++k) {
     if (kinds.pairs[k] <= 0) continue;
     ScanArgs b = a;
-    b.split = can_split ? scan_split(kinds.pairs[k] * a.strands) : 1;
+    b.split = can_split ? scan_split(k, nb, kinds.pairs[k] * a.strands) : 1;
     const hipError_t e = (k == 0 ? launch_scan_pure : k == 1 ? launch_scan_n : launch_scan_general)(nb, b, total * b.split, s);
     if (e != hipSuccess) return e;
   }

@@ -159,7 +159,7 @@ struct ScanSmem {
   static constexpr int BYTES = MISC + 64 + 4 * CE;
 };
 
-enum { SM_QN = 0, SM_KEPT = 1, SM_RUNS = 2, SM_NCAND = 3, SM_LT = 4, SM_LQ = 5, SM_NRB = 7, SM_UNSORTED = 8, SM_NPOS = 16 };
+enum { SM_QN = 0, SM_KEPT = 1, SM_RUNS = 2, SM_NCAND = 3, SM_LT = 4, SM_LQ = 5, SM_NRB = 7, SM_NPOS = 16 };
 
 // Base code: class id (0..16) of a codec letter, or 128 | byte for a byte whose codec
 // row is zero.  Two bases are identical bytes iff their codes are equal.
@@ -1176,34 +1176,28 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
   for (int c0 = lo; c0 < hi; c0 += SLICE_LAGS) {
     const int nl = (hi - c0 < SLICE_LAGS) ? hi - c0 : SLICE_LAGS;
     ex.each([&](int tid) {
-      for (int x = tid; x < nl; x += SCAN_NT) {
-        lags[x] = cands[c0 + x];
-        if (x && cands[c0 + x - 1] >= cands[c0 + x]) misc[SM_UNSORTED] = 1;
-      }
+      for (int x = tid; x < nl; x += SCAN_NT) lags[x] = cands[c0 + x];
     });
     ex.sync();
     // A lag has a slice t if npos >= P, which holds for an interval of shifts (npos is concave in
-    // the shift); lags given out of order all count as having it and are looked at one by one.
+    // the shift), and FindTop's lags ascend.
     ex.each([&](int tid) {
       if (tid >= SLICES) return;
       const int P = 32 * (SLICE_BLOCKS * tid + 1) + 1;
-      int x0 = 0, x1 = nl;
-      if (!misc[SM_UNSORTED]) {
-        auto below = [&](int idx) {  // lags before idx
-          int u = 0, v = nl;
-          while (u < v) {
-            const int w = (u + v) >> 1;
-            if ((int)lags[w] < idx) {
-              u = w + 1;
-            } else {
-              v = w;
-            }
+      auto below = [&](int idx) {  // lags before idx
+        int u = 0, v = nl;
+        while (u < v) {
+          const int w = (u + v) >> 1;
+          if ((int)lags[w] < idx) {
+            u = w + 1;
+          } else {
+            v = w;
           }
-          return u;
-        };
-        x0 = below(H + P - Lt + 1);
-        x1 = below(H + Lq - P + 1);
-      }
+        }
+        return u;
+      };
+      const int x0 = below(H + P - Lt + 1);
+      int x1 = below(H + Lq - P + 1);
       if (P > Lq || P > Lt - 1 || x1 < x0) x1 = x0;
       first[tid] = x0;
       many[tid] = x1 - x0;
@@ -1224,7 +1218,6 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
         while (id >= many[t]) id -= many[t++];
         id += first[t];
         const Lag g = lag_geometry(lags[id], H, Lq, Lt);
-        if (g.npos < 32 * (SLICE_BLOCKS * t + 1) + 1) return;
         int rises;
         uint32_t any = slice_blocks(tpl, qpl, g, t, d2, d4, d8, &rises);
         runs[tid] += count ? rises : 0;
@@ -1264,10 +1257,6 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
       ex.sync();
       queued = 0;
     }
-    ex.each([&](int tid) {
-      if (tid == 0) misc[SM_UNSORTED] = 0;
-    });
-    ex.sync();
   }
   ex.each([&](int tid) {
     if (a.stats) ex.atomic_add_shared(&misc[SM_RUNS], runs[tid]);
@@ -1322,7 +1311,6 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
     if (tid == 0) {
       misc[SM_QN] = 0;
       misc[SM_NRB] = 0;
-      misc[SM_UNSORTED] = 0;
       misc[SM_KEPT] = 0;
       misc[SM_RUNS] = 0;
       misc[SM_NCAND] = a.ncand[ps];
