@@ -6,8 +6,9 @@
 // opens a run while the window sum exceeds 1889.
 // Pairs of pure A/C/G/T chunks (scan_sliced): a thread moves 32 blocks of a lag by one position
 // per operation, one block in each bit of a word, and names the blocks whose runs may be kept;
-// those are scanned again position by position.  Other pairs take their lags in epochs of 8 or
-// 16.  A/C/G/T/N (scan_epoch_bitmap): threads take whole 32-position blocks of a lag, keep the
+// those are scanned again position by position.  Pairs with a few letters other than A/C/G/T/N are
+// scanned the same way, those letters taken as identical in the first pass.  Other pairs take
+// their lags in epochs of 8 or 16.  A/C/G/T/N (scan_epoch_bitmap): threads take whole 32-position blocks of a lag, keep the
 // window's flags in an LDS bitmap, and a second pass turns each rising edge into a run.  The
 // rest (scan_epoch_segments): a lag's diagonal is split into contiguous
 // segments, one per thread; each thread recomputes the window at its segment start,
@@ -111,6 +112,9 @@ struct ScanSmem {
   // no bitmap: bit planes of the bases instead of the packed words, the staged lags, the queue
   // of blocks and a run count per thread.
   static constexpr bool SLICED = PURE && !HASN;
+  // The general kernel scans pairs with few other letters the same way, with a plane of those
+  // letters beside the bases; its area for that lies over the segment scan's.
+  static constexpr bool AMB = !PURE;
   // The segment scans' queue holds every run one lag can produce (npos / 2 + 1, npos <= N / 2);
   // the bitmap scan flushes its queue whenever it would overflow (896 entries keep its LDS
   // plan at N = 8192 within 20 KB, 8 workgroups per CU).
@@ -123,12 +127,13 @@ struct ScanSmem {
   // The kernel with N (BMRUNS) keeps each epoch's flags in a bitmap of WPL words per lag and
   // turns its rising edges into runs afterwards; the general kernel scans contiguous
   // segments per thread and stitches runs across them.  BMRUNS, and the general kernel from
-  // N = 16384, take one epoch at a time (drained after every epoch) in
+  // N = 8192 (5 of its workgroups per CU instead of 4: 200 strands 0.54 ms instead of 0.74; at
+  // N = 2048 0.57 instead of 0.44), take one epoch at a time (drained after every epoch) in
   // 4-byte queue entries {lag - first lag of the epoch (RB bits), ns (NSB = LOG - 1), ne
   // (LOG)}; otherwise 16-lag epochs accumulate in 8-byte entries {lag rank, ns | ne << 16}
   // until the queue is half full.
   static constexpr bool BMRUNS = HASN;
-  static constexpr bool COMPACT = PURE || LOG >= 14;
+  static constexpr bool COMPACT = PURE || LOG >= 13;
   static constexpr int CE = LOG >= 14 ? 8 : 16;         // lags per epoch
   static constexpr int GSZ = SCAN_NT / CE;              // threads per lag in an epoch
   static constexpr int NSB = LOG - 1;                   // ns < N / 2
@@ -143,13 +148,18 @@ struct ScanSmem {
   static constexpr int BITMAP = SUMM;                   // uint32[CE][WPL] (BMRUNS)
   static constexpr int RLIST = BITMAP + 4 * CE * WPL;   // uint16[CE * WPL]: blocks with a rising edge (BMRUNS)
   static constexpr int PLW = N / 32 + 2 + 34;           // plane words: blocks -2 .. of a scan that runs past the end
-  static constexpr int TPL = (SUMM + 7) & ~7;           // uint32[PLW][2]: low and high bits of 32 bases (SLICED)
+  static constexpr int SQCAP = SLICED ? QCAP : 928;     // queue entries of the sliced scan
+  static constexpr int TPL = (QUEUE + 4 * SQCAP + 7) & ~7;  // uint32[PLW][2]: low and high bits of 32 bases (SLICED, AMB)
   static constexpr int QPL = TPL + 8 * PLW;
+  static constexpr int TAM = QPL + 8 * PLW;             // uint32[PLW]: letters other than A/C/G/T (AMB)
+  static constexpr int QAM = TAM + (AMB ? 4 * PLW : 0);
   static constexpr int RPL = QUEUE;                     // uint32[N/32][2]: the query, reversed (before the scan)
-  static constexpr int LAGS = QPL + 8 * PLW;            // uint16[SLICE_LAGS]
+  static constexpr int LAGS = QAM + (AMB ? 4 * PLW : 0);  // uint16[SLICE_LAGS]
   static constexpr int RUNS = LAGS + 2 * 512;           // int32[SCAN_NT]
   static constexpr int RANGE = RUNS + 4 * SCAN_NT;      // int32[2 * 32]: first lag with a slice, and how many have it
-  static constexpr int EQUAL = SLICED ? RANGE + 4 * 64 : SUMM + (BMRUNS ? 6 * CE * WPL : 8 * SCAN_NT);  // double[18][18]
+  static constexpr int SEND = (RANGE + 4 * 64 + 7) & ~7;
+  static constexpr int EEND = (SUMM + (BMRUNS ? 6 * CE * WPL : 8 * SCAN_NT) + 7) & ~7;
+  static constexpr int EQUAL = SLICED ? SEND : BMRUNS || EEND > SEND ? EEND : SEND;  // double[18][18]
   static constexpr int NTAB = PURE ? 0 : 1;             // the score tables (general kernel)
   static constexpr int GC = EQUAL + NTAB * 8 * SXC_NCLASS * SXC_NCLASS;  // double[18]
   static constexpr int SCORE = GC + NTAB * 8 * SXC_NCLASS;              // uchar[18][18]
@@ -159,7 +169,7 @@ struct ScanSmem {
   static constexpr int BYTES = MISC + 64 + 4 * CE;
 };
 
-enum { SM_QN = 0, SM_KEPT = 1, SM_RUNS = 2, SM_NCAND = 3, SM_LT = 4, SM_LQ = 5, SM_NRB = 7, SM_NPOS = 16 };
+enum { SM_QN = 0, SM_KEPT = 1, SM_RUNS = 2, SM_NCAND = 3, SM_LT = 4, SM_LQ = 5, SM_NRB = 7, SM_AMB = 8, SM_NPOS = 16 };
 
 // Base code: class id (0..16) of a codec letter, or 128 | byte for a byte whose codec
 // row is zero.  Two bases are identical bytes iff their codes are equal.
@@ -731,6 +741,33 @@ SXC_HD inline BasePlanes planes_of(const unsigned char* seq, int len, int w) {
   return r;
 }
 
+// The same of base codes (class ids 0 to 3 are A/C/G/T), and the bases that are another letter.
+SXC_HD inline BasePlanes planes_of_codes(const unsigned char* code, int len, int w, uint32_t& other) {
+  const uint32_t* p = (const uint32_t*)code + 8 * w;
+  const int left = len - 32 * w;
+  BasePlanes r = {0, 0};
+  other = 0;
+  if (left <= 0) return r;
+  static_for<0, 8>([&](auto J) {
+    constexpr int j = decltype(J)::value;
+    const uint32_t v = p[j];
+    r.lo |= (v & 0x01010101u) << j;
+    r.hi |= ((v >> 1) & 0x01010101u) << j;
+    other |= (((((v >> 2) & 0x3F3F3F3Fu) + 0x3F3F3F3Fu) >> 6) & 0x01010101u) << j;  // bit 6: not 0
+  });
+  const uint32_t keep = left >= 32 ? ~0u : (1u << left) - 1;
+  r.lo = interleave16(interleave16(r.lo)) & keep;
+  r.hi = interleave16(interleave16(r.hi)) & keep;
+  other = interleave16(interleave16(other)) & keep;
+  return r;
+}
+
+// 32 bits from base p >= -64 on of a plane that starts two words before base 0
+SXC_HD inline uint32_t bits_at(const uint32_t* pl, int p) {
+  const uint32_t* w = pl + 2 + (p >> 5);
+  return funnel32(w[1], w[0], p & 31);
+}
+
 // 32 bases from base p >= -64 on (the planes start two words before base 0)
 SXC_HD inline BasePlanes planes_at(const BasePlanes* pl, int p) {
   const BasePlanes* w = pl + 2 + (p >> 5);
@@ -961,6 +998,12 @@ SXC_HD inline void sum_digits(const uint32_t* x, const uint32_t* y, uint32_t* r)
   });
 }
 
+// General pairs are scanned in slices while at most one word (32 bases) in 8 of the two chunks holds
+// another letter, for whose windows every position is looked up twice.  ms for chunks of 4096 bases
+// with one such letter in every 2000 / 200 / 64 / 32 of the target, sliced and by segments: 200
+// strands 0.25 / 0.44 / 0.80 / 1.02 and 0.54 / 0.54 / 0.53 / 0.53, 4000 strands 1.39 / 2.96 / 5.11 /
+// 6.34 and 5.37 / 5.33 / 5.32 / 5.29; chunks of 16384, 200 strands, 64: 15.8 and 21.1.
+constexpr int SLICE_WORDS = 8;
 constexpr int SLICE_LAGS = 512;    // lags staged at a time
 constexpr int SLICE_BLOCKS = 29;   // blocks a slice decides (of the 32 it computes)
 
@@ -969,10 +1012,17 @@ constexpr int SLICE_BLOCKS = 29;   // blocks a slice decides (of the 32 it compu
 // has no flags, DoOne's test begins at n = 46).  Returns the blocks holding a position where the
 // flags have been set `gate` times in a row (d2, d4, d8: ~0 where the gate is below 2, 4, 8), and
 // in block 1 also a run that starts at 46; *rises counts the runs that start in the blocks.
-SXC_HD inline uint32_t slice_blocks(const BasePlanes* tpl, const BasePlanes* qpl, const Lag& g, int t, uint32_t d2,
-                                    uint32_t d4, uint32_t d8, int* rises) {
+// AMB: a position with another letter (planes tam, qam) counts as identical, which it scores at
+// most.  Flags are then set where they may be, so a run may start later than the flags do: every
+// block where they have been set often enough is named; blocks whose windows hold another
+// letter are left out of *rises and named if any flag is set (with `count`).
+template <bool AMB>
+SXC_HD inline uint32_t slice_blocks(const BasePlanes* tpl, const BasePlanes* qpl, const uint32_t* tam,
+                                    const uint32_t* qam, const Lag& g, int t, uint32_t d2, uint32_t d4, uint32_t d8,
+                                    bool count, int* rises) {
   // x[i] bit b: position i of block b differs (words of the planes are offset by two blocks)
   uint32_t x[32];
+  uint32_t dirty = 0;  // blocks with another letter in their windows
   {
     const int qj = g.i0 + g.shift;
     const int tb = g.i0 & 31, qb = qj & 31;
@@ -986,8 +1036,17 @@ SXC_HD inline uint32_t slice_blocks(const BasePlanes* tpl, const BasePlanes* qpl
              (funnel32(t1.hi, t0.hi, tb) ^ funnel32(q1.hi, q0.hi, qb));
       t0 = t1;
       q0 = q1;
+      if constexpr (AMB) {
+        const int at = SLICE_BLOCKS * t + b;
+        const uint32_t *ta = tam + (g.i0 >> 5) + at, *qa = qam + (qj >> 5) + at;
+        const uint32_t other = funnel32(ta[1], ta[0], tb) | funnel32(qa[1], qa[0], qb);
+        x[b] &= ~other;
+        dirty |= (other ? 1u : 0u) << b;
+      }
       if constexpr (b % 4 == 3) keep_order();
     });
+    if (AMB && t == 0) dirty &= ~3u;  // before the lag
+    dirty |= (dirty << 1) | (dirty << 2);
   }
   transpose32(x);
   keep_order();
@@ -1034,7 +1093,7 @@ SXC_HD inline uint32_t slice_blocks(const BasePlanes* tpl, const BasePlanes* qpl
   const uint32_t hb = nb - 1 >= 32 ? ~0u : (1u << (nb - 1)) - 1;
   const uint32_t la = t ? ~3u : ~15u, lb = t ? ~3u : ~7u;  // flags from n = 46; bits 0, 1 have no history
   uint32_t any = 0, wrapped = 0, at46 = 0;
-  uint32_t runs = 0;
+  uint32_t runs = 0, set = 0;
   uint32_t f[40], r2[40], r4[40], r8[40];
   auto gates = [&](auto I) {
     constexpr int i = decltype(I)::value;
@@ -1056,10 +1115,11 @@ SXC_HD inline uint32_t slice_blocks(const BasePlanes* tpl, const BasePlanes* qpl
     f[i] = ~c[5] & (i <= e ? ha : hb) & (i < 14 ? la : lb);
     gates(I);
     if constexpr (i >= 1) {
-      runs += __builtin_popcount(f[i] & ~f[i - 1] & ~7u);
+      runs += __builtin_popcount(f[i] & ~f[i - 1] & ~7u & ~dirty);
       opaque(runs);  // (one add per count)
     }
-    if constexpr (i >= 8) any |= r8[i] & ~r8[i - 1];
+    if constexpr (i >= 8) any |= AMB ? r8[i] : r8[i] & ~r8[i - 1];
+    if constexpr (AMB) set |= f[i];
     if constexpr (i == 14) at46 = t ? 0u : f[i] & 8u;
     keep_order();
   });
@@ -1068,18 +1128,21 @@ SXC_HD inline uint32_t slice_blocks(const BasePlanes* tpl, const BasePlanes* qpl
     constexpr int i = decltype(I)::value;
     f[i] = f[i - 32] >> 1;
     gates(I);
-    if constexpr (i == 32) runs += __builtin_popcount(f[i] & ~f[i - 1] & ~3u);
-    wrapped |= r8[i] & ~r8[i - 1];
+    if constexpr (i == 32) runs += __builtin_popcount(f[i] & ~f[i - 1] & ~3u & ~(dirty >> 1));
+    wrapped |= AMB ? r8[i] : r8[i] & ~r8[i - 1];
   });
   *rises = (int)runs;
-  return (any & ~7u) | ((wrapped & ~3u) << 1) | at46;
+  any = (any & ~7u) | ((wrapped & ~3u) << 1) | at46;
+  if constexpr (AMB) any |= count ? set & dirty & ~7u : 0u;
+  return any;
 }
 
 // The runs of block k of lag `rank` that were set `gate` times in a row for the first time inside
-// the block, found again position by position, and their tails.
+// the block, found again position by position, and their tails.  AMB: returns the runs that start
+// in the block if its windows hold another letter (see slice_blocks).
 template <int NB, class Ex>
-SXC_HD inline void slice_runs(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev& pr, const uint16_t* cands,
-                              int ps, int rank, const Lag& g, int k, int gate, int min_run) {
+SXC_HD inline int slice_runs(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair_dev& pr, const uint16_t* cands,
+                             int ps, int rank, const Lag& g, int k, int gate, int min_run) {
   using SS = ScanSmem<NB>;
   const BasePlanes* tpl = (const BasePlanes*)(sm + SS::TPL);
   const BasePlanes* qpl = (const BasePlanes*)(sm + SS::QPL);
@@ -1088,27 +1151,66 @@ SXC_HD inline void slice_runs(Ex& ex, char* sm, const ScanArgs& a, const sxc_pai
     return ~((t.lo ^ q.lo) | (t.hi ^ q.hi));
   };
   const int s = k - 1;  // k >= 1
+  // another letter in block b (AMB)
+  auto other = [&](int b) {
+    if constexpr (!SS::AMB) return 0u;
+    return b < 0 ? 0u : bits_at((const uint32_t*)(sm + SS::TAM), g.i0 + 32 * b) |
+                            bits_at((const uint32_t*)(sm + SS::QAM), g.i0 + g.shift + 32 * b);
+  };
   uint32_t m2 = s < 2 ? 0u : match(s - 2), m1 = s < 1 ? 0u : match(s - 1);
-  const int C = popc64(m1) + popc64(m2 >> 18);  // at 32 s - 1
-  const uint32_t prev = (32 * s - 1 >= 46 && C >= SXC_MIN_MATCHES) ? 1u : 0u;
-  uint32_t ub = byte_perm(0u, (uint32_t)(C + 128 - SXC_MIN_MATCHES), 0u);  // half_flags' u, every byte
+  uint32_t o2 = other(s - 2), o1 = other(s - 1);
+  // score of position n by the tables (AMB), and of the window before block b
+  auto score_at = [&](int n) {
+    return code_score((const unsigned char*)(sm + SS::SCORE), (unsigned char)sm[SS::TCODE + g.i0 + n],
+                      (unsigned char)sm[SS::QCODE + g.i0 + g.shift + n]);
+  };
+  auto window_before = [&](int b) {
+    if (!SS::AMB || !(o1 | o2)) return 100 * (popc64(m1) + popc64(m2 >> 18));
+    int W = 0;
+    for (int n = 32 * b < 46 ? 0 : 32 * b - 46; n < 32 * b; ++n) W += score_at(n);
+    return W;
+  };
+  const uint32_t prev = (32 * s - 1 >= 46 && window_before(s) > SXC_WIN_THRESHOLD) ? 1u : 0u;
+  bool dirty = false;  // of the block next_flags has seen last,
+  int carried = -1;    // and its last window's score, if so
   // flags of the next block, b (DoOne's positions only: 46 <= n < npos)
   auto next_flags = [&](int b) {
-    const uint32_t m0 = match(b);
-    const uint32_t old = funnel32(m1, m2, 18);  // m(n - 46)
-    // 2-bit group r: m(n) + 1 - m(n - 46)
-    const uint32_t one = ~(m0 ^ old), two = m0 & ~old;
-    uint32_t f = window_flags(interleave16(byte_perm(two, one, 0x05040100u)),
-                              interleave16(byte_perm(two, one, 0x07060302u)), ub);
-    if (b < 2) f &= b == 0 ? 0u : 0xFFFFC000u;
-    if (g.npos - 32 * b < 32) f &= g.npos > 32 * b ? (1u << (g.npos - 32 * b)) - 1 : 0u;
+    const uint32_t m0 = match(b), o0 = other(b);
+    uint32_t f = 0;
+    dirty = (o0 | o1 | o2) != 0;
+    if (!dirty) {
+      carried = -1;
+      const uint32_t old = funnel32(m1, m2, 18);  // m(n - 46)
+      // 2-bit group r: m(n) + 1 - m(n - 46)
+      const uint32_t one = ~(m0 ^ old), two = m0 & ~old;
+      const int C = popc64(m1) + popc64(m2 >> 18);
+      uint32_t ub = byte_perm(0u, (uint32_t)(C + 128 - SXC_MIN_MATCHES), 0u);  // half_flags' u, every byte
+      f = window_flags(interleave16(byte_perm(two, one, 0x05040100u)),
+                       interleave16(byte_perm(two, one, 0x07060302u)), ub);
+      if (b < 2) f &= b == 0 ? 0u : 0xFFFFC000u;
+      if (g.npos - 32 * b < 32) f &= g.npos > 32 * b ? (1u << (g.npos - 32 * b)) - 1 : 0u;
+    } else {
+      int W = carried >= 0 ? carried : window_before(b);
+      for (int n = 32 * b; n < 32 * b + 32 && n < g.npos; ++n) {
+        W += score_at(n);
+        if (n >= 46) {
+          W -= score_at(n - 46);
+          f |= (W > SXC_WIN_THRESHOLD ? 1u : 0u) << (n & 31);
+        }
+      }
+      carried = W;
+    }
     m2 = m1;
     m1 = m0;
+    o2 = o1;
+    o1 = o0;
     return f;
   };
   const uint32_t f0 = next_flags(s);
   const uint64_t f = (uint64_t)f0 | ((uint64_t)next_flags(k) << 32);
-  uint64_t rises = f & ~((f << 1) | prev) & (0xFFFFFFFFull << (33 - gate));
+  uint64_t rises = f & ~((f << 1) | prev);
+  const int starts = SS::AMB && dirty ? popc64(rises >> 32) : 0;
+  rises &= 0xFFFFFFFFull << (33 - gate);
   for (;;) {
     // the next run that is long enough or still open: found by all lanes before any takes a tail
     int ns = -1, ne = g.npos;
@@ -1124,7 +1226,7 @@ SXC_HD inline void slice_runs(Ex& ex, char* sm, const ScanArgs& a, const sxc_pai
       ns = 32 * s + r;
       if (clear && ne - ns < min_run && ns != 46) ns = -1;
     }
-    if (ns < 0) return;
+    if (ns < 0) return starts;
     if (open) {
       ne = g.npos;
       for (int b = k + 1; 32 * b < g.npos; ++b) {
@@ -1134,7 +1236,7 @@ SXC_HD inline void slice_runs(Ex& ex, char* sm, const ScanArgs& a, const sxc_pai
           break;
         }
       }
-      if (ne - ns < min_run && ns != 46) return;
+      if (ne - ns < min_run && ns != 46) return starts;
     }
     drain_run<NB>(ex, sm, a, pr, cands, ps, rank, ns, ne);
   }
@@ -1160,7 +1262,8 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
   constexpr int H = SS::N / 2;
   constexpr int SLICES = (SS::WPL - 1 + SLICE_BLOCKS - 1) / SLICE_BLOCKS;
   static_assert(SLICES >= 1 && SLICES <= 32, "slices of a lag");
-  static_assert(32 * SLICE_BLOCKS <= SS::QCAP, "32 slices' blocks fit the queue");
+  constexpr int QCAP = SS::SQCAP;
+  static_assert(32 * SLICE_BLOCKS <= QCAP, "32 slices' blocks fit the queue");
   int* misc = (int*)(sm + SS::MISC);
   int* queue = (int*)(sm + SS::QUEUE);
   uint16_t* lags = (uint16_t*)(sm + SS::LAGS);
@@ -1169,6 +1272,8 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
   int* runs = (int*)(sm + SS::RUNS);
   const BasePlanes* tpl = (const BasePlanes*)(sm + SS::TPL);
   const BasePlanes* qpl = (const BasePlanes*)(sm + SS::QPL);
+  const uint32_t* tam = (const uint32_t*)(sm + SS::TAM);
+  const uint32_t* qam = (const uint32_t*)(sm + SS::QAM);
   const int Lt = misc[SM_LT], Lq = misc[SM_LQ];
   const int gate = min_run >= 8 ? 8 : min_run >= 4 ? 4 : min_run >= 2 ? 2 : 1;
   const uint32_t d2 = gate >= 2 ? 0u : ~0u, d4 = gate >= 4 ? 0u : ~0u, d8 = gate >= 8 ? 0u : ~0u;
@@ -1219,19 +1324,19 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
         id += first[t];
         const Lag g = lag_geometry(lags[id], H, Lq, Lt);
         int rises;
-        uint32_t any = slice_blocks(tpl, qpl, g, t, d2, d4, d8, &rises);
+        uint32_t any = slice_blocks<SS::AMB>(tpl, qpl, tam, qam, g, t, d2, d4, d8, a.stats != nullptr, &rises);
         runs[tid] += count ? rises : 0;
         while (any) {
           const int b = __builtin_ctz(any);
           any &= any - 1;
           const int at = ex.atomic_add_shared(&misc[SM_QN], 1);  // (one atomic per wave)
-          if (at < SS::QCAP) queue[at] = id | (SLICE_BLOCKS * t + b - 2) << 9;
+          if (at < QCAP) queue[at] = id | (SLICE_BLOCKS * t + b - 2) << 9;
         }
       });
       ex.sync();
       const int qn = misc[SM_QN];
       ex.sync();  // every thread has read the count
-      const bool over = qn > SS::QCAP;
+      const bool over = qn > QCAP;
       if (over) {
         if (counted < base + width) counted = base + width;
         width = 32;
@@ -1239,7 +1344,7 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
         base += width;
         if (base >= counted) width = SCAN_NT;
       }
-      if (!over && qn <= SS::QCAP / 2 && base < total) {
+      if (!over && qn <= QCAP / 2 && base < total) {
         queued = qn;
         continue;
       }
@@ -1247,7 +1352,8 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
       ex.each([&](int tid) {
         for (int x = tid; x < n; x += SCAN_NT) {
           const int id = queue[x] & (SLICE_LAGS - 1), k = queue[x] >> 9;
-          slice_runs<NB>(ex, sm, a, pr, cands, ps, c0 + id, lag_geometry(lags[id], H, Lq, Lt), k, gate, min_run);
+          runs[tid] +=
+              slice_runs<NB>(ex, sm, a, pr, cands, ps, c0 + id, lag_geometry(lags[id], H, Lq, Lt), k, gate, min_run);
         }
       });
       ex.sync();
@@ -1311,6 +1417,7 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
     if (tid == 0) {
       misc[SM_QN] = 0;
       misc[SM_NRB] = 0;
+      misc[SM_AMB] = 0;
       misc[SM_KEPT] = 0;
       misc[SM_RUNS] = 0;
       misc[SM_NCAND] = a.ncand[ps];
@@ -1411,6 +1518,28 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
       }
     });
     ex.sync();
+    ex.each([&](int tid) {
+      BasePlanes* tpl = (BasePlanes*)(sm + SS::TPL);
+      BasePlanes* qpl = (BasePlanes*)(sm + SS::QPL);
+      uint32_t* tam = (uint32_t*)(sm + SS::TAM);
+      uint32_t* qam = (uint32_t*)(sm + SS::QAM);
+      int n = 0;
+      for (int w = tid; w < SS::PLW; w += SCAN_NT) {
+        BasePlanes t = {0, 0}, q = {0, 0};
+        uint32_t to = 0, qo = 0;
+        if (w >= 2 && w < 2 + N / 32) {
+          t = planes_of_codes(tc, Lt, w - 2, to);
+          q = planes_of_codes(qc, Lq, w - 2, qo);
+        }
+        tpl[w] = t;
+        qpl[w] = q;
+        tam[w] = to;
+        qam[w] = qo;
+        n += (to != 0) + (qo != 0);
+      }
+      if (n) ex.atomic_add_shared(&misc[SM_AMB], n);
+    });
+    ex.sync();
   }
   const uint16_t* cands = gcands;
   const int ncand = misc[SM_NCAND];
@@ -1421,8 +1550,11 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
   // Queue entries before the current epoch, kept per thread: every thread must see the same
   // count, and the shared counter may already hold the next epoch's pushes of a faster wave.
   int queued = 0;
-  if constexpr (SS::SLICED) scan_sliced<NB>(ex, sm, a, pr, cands, ps, lo, hi, min_run);
-  for (int e0 = SS::SLICED ? hi : lo; e0 < hi; e0 += CE) {
+  bool sliced = SS::SLICED;
+  if constexpr (SS::AMB) sliced = 32 * SLICE_WORDS * misc[SM_AMB] <= Lt + Lq;
+  if constexpr (SS::SLICED || SS::AMB)
+    if (sliced) scan_sliced<NB>(ex, sm, a, pr, cands, ps, lo, hi, min_run);
+  for (int e0 = sliced ? hi : lo; e0 < hi; e0 += CE) {
     const int qstart = queued;
     const int e1 = (e0 + CE < hi) ? e0 + CE : hi;
     if constexpr (SS::BMRUNS) {

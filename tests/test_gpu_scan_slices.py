@@ -1,0 +1,130 @@
+"""The scan and its launches on the GPU against the oracle, at the sizes where a rule changes over:
+slice and window ends, kinds of pair mixed in a batch, the shares a strand's lags are split into
+(to 32, 128 and 768 strands), a workgroup per channel (to 128 strands), the record counts' scan
+(1024 at a time), run ordering and probabilities around their tiles.
+Bar: coordinates, lengths, strands, identities bit-exact; prob within 1e-11 relative (the device's
+erf/exp; keep decisions near min_prob are made on the host)."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import dense_run_pair
+from scan_cases import LENGTHS, LETTERS, related
+
+pytestmark = pytest.mark.gpu
+
+EXACT = ["query_id", "target_id", "query_size", "qstart", "tstart", "len", "reverse", "ident"]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from satsuma2_amd.api import Context
+
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def chunk_pairs(shapes):
+    from satsuma2_amd.api import ChunkPair
+
+    out = []
+    for k, (lt, lq, letters) in enumerate(shapes):
+        t, q = related(lt, lq, letters, 17 * k + 1, reverse=k % 3 == 0)
+        out.append(ChunkPair(t, q, t_record=k, q_record=k, q_record_len=len(q), fast=int(k % 5 == 4)))
+    return out
+
+
+def check(ctx, pairs, t_chunk, target_total=1e6, resident=True):
+    from satsuma2_amd.api import HomologyByXCorr, ResidentBatch, SlaveParams
+
+    prm = SlaveParams(t_chunk=t_chunk, q_chunk=t_chunk, target_total=target_total)
+    ref = oracle.align_batch([dict(tseq=p.tseq, qseq=p.qseq, t_record=p.t_record, q_record=p.q_record,
+                                   q_record_len=p.q_record_len, fast=p.fast) for p in pairs],
+                             oracle.make_params(N=2 * t_chunk, q_chunk=t_chunk, target_total=target_total), threads=16,
+                             cap_per_pair=2048)
+    ref = np.concatenate(ref)
+    results = [HomologyByXCorr(ctx, prm).align_batch(pairs)]
+    if resident:
+        b = ResidentBatch(ctx, pairs, prm)
+        b.run()
+        results.append(b.results())
+        b.close()
+    for got in results:
+        assert len(got) == len(ref)
+        for f in EXACT:
+            assert np.array_equal(got[f], ref[f]), f
+        assert np.all(np.abs(got["prob"] - ref["prob"]) <= 1e-11 * np.abs(ref["prob"]))
+    return ref
+
+
+@pytest.mark.parametrize("letters", LETTERS)
+@pytest.mark.parametrize("t_chunk", [1024, 2048, 4096])
+def test_lengths(ctx, letters, t_chunk):
+    """Diagonals around the ends of windows, words and slices (t_chunk 4096: up to 5 slices)."""
+    ends = [n for n in LENGTHS] + [n + 928 * k for n in (960, 961, 962) for k in (1, 2, 3) if n + 928 * k <= t_chunk]
+    shapes = [(n, (n, t_chunk, t_chunk - 31)[k % 3], letters) for k, n in enumerate(ends) if n <= t_chunk]
+    assert len(check(ctx, chunk_pairs(shapes), t_chunk)) > 0
+
+
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 128, 384, 385, 512, 513, 1025])
+def test_batch_sizes(ctx, n):
+    """Launch rules by the number of pairs, kinds mixed; two strands each."""
+    kinds = ["acgt", "acgt", "n_gap", "few", "acgt", "dense", "words", "zero"]
+    shapes = [(256 - k % 7, 256 - k % 11, kinds[k % len(kinds)]) for k in range(n)]
+    check(ctx, chunk_pairs(shapes), 256)
+
+
+@pytest.mark.parametrize("t_chunk", [256, 512, 1024, 2048, 4096, 8192, 16384])
+@pytest.mark.parametrize("letters", ["acgt", "few"])
+def test_few_pairs_of_every_length(ctx, t_chunk, letters):
+    """A workgroup per channel and 16 shares per strand, odd chunk lengths, every N."""
+    shapes = [(t_chunk, t_chunk, letters), (t_chunk - 1, t_chunk // 2 + 3, letters), (t_chunk // 3, t_chunk, letters)]
+    assert len(check(ctx, chunk_pairs(shapes), t_chunk)) > 0
+
+
+@pytest.mark.parametrize("target_total", [1.0, 30.0, 1e3])
+def test_small_targets(ctx, target_total):
+    """Every gate: kept runs of less than 8, 4 and 2 positions above the threshold."""
+    shapes = [(700, 1000, k) for k in ("acgt", "few", "n_gap", "dense")]
+    assert len(check(ctx, chunk_pairs(shapes), 1024, target_total)) > 0
+
+
+@pytest.mark.parametrize("letter", [b"", b"N", b"R"])
+def test_run_counts(ctx, letter):
+    """A resident batch's count of runs, and more blocks than the queue holds."""
+    from satsuma2_amd.api import ChunkPair, ResidentBatch, SlaveParams
+
+    t = dense_run_pair()
+    t = t[:700] + letter + t[700 + len(letter):]
+    b = ResidentBatch(ctx, [ChunkPair(t, t, q_record_len=len(t))], SlaveParams(target_total=100.0))
+    b.run()
+    lags, runs = b.stats()
+    b.close()
+    want = [0, 0]
+    for qs in (t, oracle.reverse_complement(t)):
+        xc = oracle.xcorr(oracle.encode(t, 8192), oracle.encode(qs, 8192))
+        want[0] += len(oracle.findtop(xc, 1.8))
+        want[1] += len(oracle.matchup(qs, t, xc, 1.8))
+    assert [lags, runs] == want
+
+
+@pytest.mark.parametrize("letters", ["acgt", "n_gap", "few"])
+def test_matchup_runs_and_probabilities(ctx, letters):
+    """MatchUp's runs in order (tiles of 256), their probabilities (64 at a time, 16 bases each step)."""
+    for n in (80, 1023, 4096):
+        t, q = related(n, n, letters, n)
+        xc = oracle.xcorr(oracle.encode(t, 2 * 4096), oracle.encode(q, 2 * 4096))
+        ref = oracle.matchup(q, t, xc, 1.8)
+        got = ctx.matchup(q, t, xc, 1.8)
+        got = np.stack([got[f] for f in got.dtype.names], 1) if got.dtype.names else got
+        assert np.array_equal(got, ref)
+    rng = np.random.default_rng(5)
+    for k in (1, 63, 64, 65, 1025):
+        length = rng.choice([1, 15, 16, 17, 46, 300], k)
+        runs = np.stack([rng.integers(0, len(t) - 300, k), rng.integers(0, len(q) - 300, k), length], 1).astype(np.int32)
+        prob, ident = ctx.match_probability(t, q, runs, 1e6)
+        for (st, sq, n), p, i in zip(runs, prob, ident):
+            want = oracle.match_probability(t, q, int(st), int(sq), int(n), 1e6)
+            assert p == want or abs(p - want) <= 1e-11 * abs(want) or (np.isnan(p) and np.isnan(want))
+            assert i == oracle.print_match_ident(q, t, int(st), int(sq), int(n))
