@@ -116,8 +116,8 @@ struct ScanSmem {
   // letters beside the bases; its area for that lies over the segment scan's.
   static constexpr bool AMB = !PURE;
   // The segment scans' queue holds every run one lag can produce (npos / 2 + 1, npos <= N / 2);
-  // the bitmap scan flushes its queue whenever it would overflow (896 entries keep its LDS
-  // plan at N = 8192 within 20 KB, 8 workgroups per CU).
+  // the bitmap scan and the sliced scan flush theirs whenever it would overflow (the sliced scan's
+  // also holds the query's planes while they are turned around).
   static constexpr int QCAP = (SLICED ? (N / 16 < 1024 ? 1024 : N / 16) : PURE ? 896 : N / 4 + 64);
   static constexpr int PKW = SLICED ? 0 : N / 16 + 4;   // 2-bit packed words (+3 words of read-ahead)
   static constexpr int TCODE = 0;                       // uchar[N] (general kernel)
@@ -1251,8 +1251,8 @@ SXC_HD inline int slice_runs(Ex& ex, char* sm, const ScanArgs& a, const sxc_pair
 // Vector issue bounds it: a slice takes some 1600 instructions (about 190 for the difference
 // words, 260 for the transposition, 130 for the first counts, 30 per position), 55 per block of 32
 // positions against 110 to 120 where a thread took one block at a time and 150 more before its
-// first, and 32 blocks share one start.  Of the 0.51 ms at N = 8192 the slices take 0.28 and the
-// named blocks about 0.2.  One launch, before (a block at a time) and now: 8192 strands at
+// first, and 32 blocks share one start.  306 M instructions for 8192 strands at N = 8192 take
+// 0.507 ms, all of the chip's issue rate: the slices 0.28, the named blocks about 0.2.  One launch, before (a block at a time) and now: 8192 strands at
 // N = 8192 0.80 and 0.51 ms, 24000 at 2048 3.59 and 1.46 ms, 40000 at 512 1.19 and 0.64 ms, 1000
 // at 32768 1.96 and 0.75 ms.
 template <int NB, class Ex>

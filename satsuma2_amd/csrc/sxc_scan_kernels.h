@@ -10,7 +10,7 @@ namespace sxc {
 struct NoRegs {};
 
 // Waves per SIMD the register budget is set for.  The sliced scan (pure A/C/G/T) keeps 32 words of
-// a slice and their counts in registers: 6 waves (80 registers, none spilled) take 0.507 ms for 8192
+// a slice and their counts in registers: 6 waves (80 registers, 6 spilled) take 0.507 ms for 8192
 // strands at N = 8192 and 1.47 for 24000 at 2048, 5 waves 0.529 and 1.53, 8 (26 spilled) 0.515 and
 // 1.40.  The general scan's LDS plan admits 5 workgroups at N = 8192.  The A/C/G/T/N scan gets as many of its 4-wave workgroups per CU as its LDS plan admits,
 // up to 8 waves (the spills the budget costs are cheaper than the latency the waves hide).
