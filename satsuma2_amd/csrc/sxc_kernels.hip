@@ -286,13 +286,17 @@ hipError_t launch_correlate(int geo, const PairArgs& a, int total, hipStream_t s
 // 135 / 175 / 266 (N = 2048 the same within 10%); at N = 32768, with 4 times the lags and
 // positions: 32 strands 359 / 196 / 146 / 94 / 81, 128 strands 356 / 203 / 203 / 202 / 203, 512
 // strands 501 / 438 / 555 / - / -, 2048 strands 1434 / 1406 / 1965 / - / -.
-// With N or other letters, lags are taken 8 or 16 at a time: up to 2048 workgroups in all (8 per
-// CU), more than 4 per strand only below 512 (128 strands - / 17 / 18 / 22 / 29, 740 strands
-// 195 / 120 / - / - / -, with a kernel of that kind on A/C/G/T pairs).
+// With N, lags are taken 8 or 16 at a time: up to 2048 workgroups in all (8 per CU), more than 4 per
+// strand only to 128 strands (1 / 2 / 4 / 8 at N = 8192: 96 strands 156 / 95 / 76 / 64, 256 strands 163 /
+// 113 / 103 / 117, 400 strands 183 / 141 / 154 / 162, 800 strands 251 / 224 / 242 / 282; at N = 2048 400
+// strands 312 / 208 / 180 / 170).  With other letters (5 workgroups per CU) the same to 320 strands,
+// 2 above them: 2 / 4 per strand, one such letter and one in 16 bases, 200 strands 179 / 192 and 731 / 519,
+// 320 strands 193 / 258 and 785 / 943, 512 strands 213 / 307 and 776 / 1062; at N = 2048, one in 16, 320
+// strands 611 / 484, 400 strands 647 / 752.
 static int scan_split(int kind, int nb, int n) {
   if (n <= 0) return 1;
   if (kind == 0) return n <= 32 ? 16 : n <= 128 ? 8 : n <= (nb >= 14 ? 2048 : 768) ? 2 : 1;
-  return std::max(1, std::min({2048 / n, std::max(4, 512 / n), 16}));
+  return std::max(1, std::min({2048 / n, std::max(kind == 2 && n > 320 ? 2 : 4, 512 / n), 16}));
 }
 
 hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& kinds, bool can_split, hipStream_t s) {
