@@ -210,11 +210,16 @@ def _pairs_table(pairs: Sequence[ChunkPair]):
         tab[f + "seq"] = np.frombuffer((C.c_char_p * n)(*seqs), np.uint64)
         tab[f + "len"] = np.fromiter(map(len, seqs), np.int32, n)
     ints = np.array(list(chain.from_iterable(map(attrgetter(*_PAIR_INTS), pairs)))).reshape(n, len(_PAIR_INTS))
-    if ints.dtype.kind not in "iub":
-        raise TypeError("a chunk pair's positions, records and flags are integers")
-    for k, f in enumerate(_PAIR_INTS):
-        tab[f] = ints[:, k]
-    tab["q_record_len"] = np.where(tab["q_record_len"] >= 0, tab["q_record_len"], tab["qlen"])
+    if ints.dtype.kind in "iub":
+        cols = dict(zip(_PAIR_INTS, ints.T))
+    else:  # no common integer type (a record array's uint64 beside an int, more than 64 bits): converted one by one
+        cols = {f: [getattr(p, f) for p in pairs] for f in _PAIR_INTS}
+    # (a negative length before it is cut to 32 bits means the chunk's own)
+    qrl = cols["q_record_len"]
+    cols["q_record_len"] = ([v if v >= 0 else len(q) for v, q in zip(qrl, keep[1])] if isinstance(qrl, list) else
+                            np.where(qrl >= 0, qrl, tab["qlen"]))
+    for f, v in cols.items():
+        tab[f] = np.frombuffer((C.c_int32 * n)(*v), np.int32) if isinstance(v, list) else v
     return (Pair * n).from_buffer(tab), keep
 
 

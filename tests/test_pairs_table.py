@@ -32,3 +32,17 @@ def test_refused(field, value):
         setattr(pairs[n // 2], field, value)
         with pytest.raises((TypeError, C.ArgumentError, ValueError)):
             api._pairs_array(pairs)
+
+
+@pytest.mark.parametrize("value", [np.uint64(7), np.int64(5), True, 1 << 31, (1 << 31) + 5, (1 << 32) + 3, 1 << 63, 1 << 64,
+                                   -(1 << 63) - 1, -5, np.array(4)])
+@pytest.mark.parametrize("field", ["t_record", "q_record_len", "fast"])
+def test_integers_of_any_type(field, value):
+    """Record arrays hold uint64; what one pair is packed to, many are."""
+    pairs = rows(40)
+    setattr(pairs[11], field, value)
+    arr, _ = api._pairs_array(pairs)
+    for k in (0, 11, 39):
+        one, _ = api._pairs_array(pairs[k:k + 1])
+        for f, _ in api.Pair._fields_:
+            assert getattr(arr[k], f) == getattr(one[0], f), (k, f)
