@@ -63,6 +63,10 @@ float elapsed(hipEvent_t a, hipEvent_t b) {
   return ms;
 }
 
+int pair_kind(const sxc::HostBatch& hb, const sxc_pair_dev& p) {
+  return sxc::scan_kind(hb.tchunks[(size_t)p.t_chunk].flags, hb.qchunks[(size_t)p.q_chunk].flags);
+}
+
 // Upload a packed batch (inputs become resident in HBM).
 // The sub-batch's own stream, events and pinned control words (created on first use, on
 // the context's device).
@@ -98,6 +102,13 @@ int batch_upload(sxc_ctx* ctx, sxc_batch_dev& b) {
     HIPCHK(hipMemcpyAsync(b.qch.p, hb.qchunks.data(), hb.qchunks.size() * sizeof(sxc_chunk), hipMemcpyHostToDevice, s));
   if (!hb.pairs.empty())
     HIPCHK(hipMemcpyAsync(b.pairs.p, hb.pairs.data(), hb.pairs.size() * sizeof(sxc_pair_dev), hipMemcpyHostToDevice, s));
+  std::vector<int32_t> list;
+  if (b.kinds.mixed()) {
+    list.resize(hb.pairs.size());
+    b.kinds.list([&](int32_t k) { return pair_kind(hb, hb.pairs[(size_t)k]); }, list.data());
+    HIPCHK(b.list.ensure(list.size() * sizeof(int32_t)));
+    HIPCHK(hipMemcpyAsync(b.list.p, list.data(), list.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
+  }
   std::vector<int32_t> idx(hb.tchunks.size());
   for (size_t i = 0; i < idx.size(); ++i) idx[i] = (int32_t)i;
   if (!idx.empty()) HIPCHK(hipMemcpyAsync(b.which.p, idx.data(), idx.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
@@ -114,7 +125,7 @@ int batch_upload(sxc_ctx* ctx, sxc_batch_dev& b) {
     HIPCHK(hipMemcpyAsync(b.segs.p, hb.segs.data(), hb.segs.size() * sizeof(sxc_tail_seg_dev), hipMemcpyHostToDevice, s));
     HIPCHK(hipMemcpyAsync(b.ttail.p, hb.ttail.data(), hb.ttail.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
   }
-  HIPCHK(hipStreamSynchronize(s));  // idx is a host temporary
+  HIPCHK(hipStreamSynchronize(s));  // list and idx are host temporaries
   return SXC_OK;
 }
 
@@ -203,6 +214,7 @@ int launch_pairs(sxc_ctx* ctx, sxc_batch_dev& b, bool fresh) {
     a.ptable = b.ptable;
     a.table_prob = b.prm.table_prob;
   }
+  a.list = b.kinds.mixed() ? b.list.as<int32_t>() : nullptr;
   HIPCHK(sxc::launch_scan(b.nb, a, total, b.kinds, fresh, b.s));
   return SXC_OK;
 }
@@ -279,7 +291,8 @@ uint64_t graph_signature(const sxc_ctx* ctx, const sxc_batch_dev& b) {
   auto mix = [&](uint64_t v) { h = (h ^ v) * 1099511628211ull; };
   for (const DevBuf* d : {&b.seq, &b.tch, &b.qch, &b.pairs, &b.spectra, &b.which, &b.slots, &b.keys, &b.counts,
                           &b.offsets, &b.total, &b.maxc, &b.final_, &b.stats, &b.cands, &b.ncand, &b.sch, &b.sstr,
-                          &b.tails, &b.segs, &b.ttail, &b.src_sig, &b.ent, &b.nflag, &b.parts})
+                          &b.tails, &b.segs, &b.ttail, &b.src_sig, &b.ent, &b.nflag, &b.parts,
+                          &b.list})
     mix((uint64_t)(uintptr_t)d->p);
   mix((uint64_t)(uintptr_t)b.ptable);
   mix((uint64_t)(uintptr_t)b.h_ctl);
@@ -456,8 +469,7 @@ int batch_prepare(sxc_batch_dev& b, const sxc_pair* pairs, int32_t n, const sxc_
   std::string e = sxc::pack_batch(pairs, n, prm->N, b.hb, t_tail, q_tail);
   if (!e.empty()) return fail(SXC_ERR_ARG, e);
   b.kinds = sxc::ScanKinds();
-  for (const sxc_pair_dev& p : b.hb.pairs)
-    ++b.kinds.pairs[sxc::scan_kind(b.hb.tchunks[(size_t)p.t_chunk].flags, b.hb.qchunks[(size_t)p.q_chunk].flags)];
+  for (const sxc_pair_dev& p : b.hb.pairs) ++b.kinds.pairs[pair_kind(b.hb, p)];
   b.prm = *prm;
   b.nb = nb;
   b.slot_cap = 64;  // records per (pair, strand) a run first makes room for; grows on overflow

@@ -65,6 +65,7 @@ struct sxc_batch_dev {
   DevBuf nflag;  // records the last scan flagged near min_prob (the counts kernel reads and clears it)
   sxc::HostBatch hb;
   sxc::ScanKinds kinds;  // of hb.pairs
+  DevBuf list;           // hb.pairs by kind (ScanKinds::list) where kinds are mixed
   sxc_params prm{};
   int nb = 0;
   int slot_cap = 64;
@@ -92,7 +93,8 @@ struct sxc_batch_dev {
     if (s) (void)hipStreamSynchronize(s);
     if (gexec) (void)hipGraphExecDestroy(gexec), gexec = nullptr;
     for (DevBuf* b : {&seq, &tch, &qch, &pairs, &spectra, &which, &slots, &keys, &counts, &offsets, &total, &maxc,
-                      &final_, &stats, &cands, &ncand, &sch, &sstr, &tails, &segs, &ttail, &src_sig, &ent, &nflag, &parts})
+                      &final_, &stats, &cands, &ncand, &sch, &sstr, &tails, &segs, &ttail, &src_sig, &ent, &nflag, &parts,
+                      &list})
       b->release();
     for (hipEvent_t& e : ev)
       if (e) (void)hipEventDestroy(e), e = nullptr;

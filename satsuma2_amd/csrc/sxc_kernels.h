@@ -12,17 +12,9 @@ namespace sxc {
 hipError_t launch_correlate(int geo, const PairArgs& a, int total, hipStream_t s);
 // Compiled geometries of length 2^nb (distinct stage-A width / round depth), default first.
 int fft_geometries(int nb, int* out, int cap);
-// The kinds of chunk pairs the scan has a kernel of its own for, and how many of a launch's
-// pairs are of each.
-enum { SCAN_PURE = 0, SCAN_N = 1, SCAN_GENERAL = 2 };
-inline int scan_kind(int32_t tflags, int32_t qflags) {
-  return (tflags & qflags & 2) ? SCAN_PURE : (tflags & qflags & 4) ? SCAN_N : SCAN_GENERAL;
-}
-struct ScanKinds {
-  int32_t pairs[3] = {0, 0, 0};
-};
-// Scans the accepted lags of `total` (pair, strand)s.  can_split: counts are zero, so that a
-// launch too small to fill the device may share a strand's lags between several workgroups.
+// Scans the accepted lags of `total` (pair, strand)s, kind by kind; a.list as ScanKinds::list filled
+// it where more than one kind occurs.  can_split: counts are zero, so that a launch too small to
+// fill the device may share a strand's lags between several workgroups.
 hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& kinds, bool can_split, hipStream_t s);
 hipError_t launch_scan_pure(int nb, const ScanArgs& a, int grid, hipStream_t s);
 hipError_t launch_scan_n(int nb, const ScanArgs& a, int grid, hipStream_t s);

@@ -300,9 +300,10 @@ static int scan_split(int kind, int nb, int n) {
 }
 
 hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& kinds, bool can_split, hipStream_t s) {
-  // one launch per kind that occurs, over the same grid; a workgroup exits at once on another
-  // kind's pair.  Shares of a strand add their run counts, so those start at zero (cleared here
-  // and not by the pair kernel, which one more store made 3% slower at N = 16384).
+  // One launch per kind that occurs.  Shares of a strand add their run counts, so those start at
+  // zero (cleared here and not by the pair kernel, which one more store made 3% slower at N = 16384).
+  if (kinds.all() * a.strands != total || (kinds.mixed() && !a.list)) return hipErrorInvalidValue;
+  int first = 0;
   if (can_split && a.stats)
     for (int k = 0; k < 3; ++k)
       if (kinds.pairs[k] > 0 && scan_split(k, nb, kinds.pairs[k] * a.strands) > 1) {
@@ -312,8 +313,13 @@ hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& ki
   for (int k = 0; k < 3; ++k) {
     if (kinds.pairs[k] <= 0) continue;
     ScanArgs b = a;
-    b.split = can_split ? scan_split(k, nb, kinds.pairs[k] * a.strands) : 1;
-    const hipError_t e = (k == 0 ? launch_scan_pure : k == 1 ? launch_scan_n : launch_scan_general)(nb, b, total * b.split, s);
+    const int n = kinds.pairs[k] * a.strands;
+    b.split = can_split ? scan_split(k, nb, n) : 1;
+    b.list = a.list ? a.list + first : nullptr;
+    first += kinds.pairs[k];
+    // a launch of 2^32 threads or more is not refused: its last workgroups are missing
+    if ((int64_t)n * b.split * SCAN_NT >= (int64_t)1 << 32) return hipErrorInvalidValue;
+    const hipError_t e = (k == 0 ? launch_scan_pure : k == 1 ? launch_scan_n : launch_scan_general)(nb, b, n * b.split, s);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -71,6 +71,29 @@ struct ScanArgs {
   // on counts[ps], which must be zero at launch (the pair kernel clears it), and stats
   // runs are added atomically.
   int32_t split;
+  const int32_t* list;       // optional: the pairs to scan (null: pair 0 on)
+};
+
+// The kinds of chunk pairs the scan has a kernel of its own for, and how many of a launch's
+// pairs are of each.
+enum { SCAN_PURE = 0, SCAN_N = 1, SCAN_GENERAL = 2 };
+SXC_HD inline int scan_kind(int32_t tflags, int32_t qflags) {
+  return (tflags & qflags & 2) ? SCAN_PURE : (tflags & qflags & 4) ? SCAN_N : SCAN_GENERAL;
+}
+struct ScanKinds {
+  int32_t pairs[3] = {0, 0, 0};
+  bool mixed() const { return (pairs[0] > 0) + (pairs[1] > 0) + (pairs[2] > 0) > 1; }
+  int32_t all() const { return pairs[0] + pairs[1] + pairs[2]; }
+  // Of a mixed launch, the pairs grouped by kind: a kind's launch covers its own pairs only.  (Over
+  // all pairs, with the others' workgroups leaving at once, the shares of a rare kind's strands
+  // multiplied the whole grid: one pure pair among 100000 with N at N = 512 took 3.2 M workgroups,
+  // 9.27 ms against 7.54, and one among 524297 lost its records, as a grid of 2^32 threads or more
+  // wraps.  One pair with N among 4096 of 4096 bp: 0.615 and 0.598 ms.)
+  template <class KindOf>
+  void list(KindOf&& kind_of, int32_t* out) const {
+    int32_t at[3] = {0, pairs[0], pairs[0] + pairs[1]};
+    for (int32_t k = 0; k < all(); ++k) out[at[kind_of(k)]++] = k;
+  }
 };
 
 // Host: the keep decision's parameters for min_prob and the target size -- the float
@@ -100,8 +123,7 @@ static_assert(25 * SXC_MIN_QUARTERS > SXC_WIN_THRESHOLD && 25 * (SXC_MIN_QUARTER
 // NB: log2 N in bits 0-4; bit 5 selects the kernel for pairs whose two chunks are pure
 // A/C/G/T (SLICED); bit 6 the one for pairs of A/C/G/T/N chunks with an N (HASN), whose LDS plan
 // holds the packed bases, the N masks, the run queue and the counters (the accepted lags are read
-// from global memory).  The general kernel takes every other pair.  Each exits at once on the
-// others' pairs.
+// from global memory).  The general kernel takes every other pair.
 template <int NB>
 struct ScanSmem {
   static constexpr int LOG = NB & 31;
@@ -1375,14 +1397,15 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
   using SS = ScanSmem<NB>;
   constexpr int N = SS::N;
   const int split = a.split > 1 ? a.split : 1;
-  const int ps = blk / split, part = blk % split;
-  const sxc_pair_dev pr = a.pairs[ps / a.strands];
-  const int strand = ps % a.strands;
+  const int at = blk / split, part = blk % split;
+  const int pair = a.list ? a.list[at / a.strands] : at / a.strands;
+  const int strand = at % a.strands;
+  const int ps = pair * a.strands + strand;
+  const sxc_pair_dev pr = a.pairs[pair];
   const sxc_chunk tch = a.tchunks[pr.t_chunk];
   const sxc_chunk qch = a.qchunks[pr.q_chunk];
-  const bool fast = (tch.flags & 2) && (qch.flags & 2);   // both pure A/C/G/T
-  const bool acgtn = (tch.flags & 4) && (qch.flags & 4);  // both A/C/G/T/N
-  if (fast != (SS::PURE && !SS::HASN) || (!fast && acgtn) != SS::HASN) return;  // another kernel's pair
+  // each kernel takes its own kind only, whatever it is launched over
+  if (scan_kind(tch.flags, qch.flags) != (SS::SLICED ? SCAN_PURE : SS::HASN ? SCAN_N : SCAN_GENERAL)) return;
   const sxc_tables* tab = a.tab;
   unsigned char* tc = (unsigned char*)(sm + SS::TCODE);
   unsigned char* qc = (unsigned char*)(sm + SS::QCODE);

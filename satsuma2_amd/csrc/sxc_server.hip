@@ -138,6 +138,10 @@ int64_t block_pairs(const sxc_block& b) {
   return (int64_t)(b.target_to - b.target_from + 1) * (int64_t)(b.query_to - b.query_from + 1);
 }
 
+int pair_kind(const sxc_server* sv, const sxc_pair_dev& p) {
+  return sxc::scan_kind(sv->h_tch[(size_t)p.t_chunk].flags, sv->h_qch[(size_t)p.q_chunk].flags);
+}
+
 int slot_alloc(sxc_server* sv, Slot& sl) {
   const int P = sv->P, N = sv->prm.N;
   const size_t total = (size_t)2 * P;
@@ -145,7 +149,8 @@ int slot_alloc(sxc_server* sv, Slot& sl) {
   HIPCHK(hipEventCreate(&sl.ev_start));
   HIPCHK(hipEventCreate(&sl.ev_count));
   HIPCHK(hipEventCreate(&sl.ev_pack));
-  HIPCHK(sl.pairs.ensure((size_t)P * sizeof(sxc_pair_dev)));
+  const size_t pairs = (size_t)P * (sizeof(sxc_pair_dev) + sizeof(int32_t));  // and their list by kind
+  HIPCHK(sl.pairs.ensure(pairs));
   HIPCHK(sl.cands.ensure(total * N * sizeof(uint16_t)));
   HIPCHK(sl.ncand.ensure(total * sizeof(int32_t)));
   HIPCHK(sl.outs.ensure(total * kDefaultCap * sizeof(sxc_result_dev)));
@@ -156,7 +161,7 @@ int slot_alloc(sxc_server* sv, Slot& sl) {
   HIPCHK(sl.maxc.ensure(sizeof(int32_t)));
   HIPCHK(sl.final_.ensure(total * kDefaultCap * sizeof(sxc_result_dev)));
   sl.out_cap = (int64_t)total * kDefaultCap;
-  HIPCHK(hipHostMalloc((void**)&sl.h_pairs, (size_t)P * sizeof(sxc_pair_dev), hipHostMallocDefault));
+  HIPCHK(hipHostMalloc((void**)&sl.h_pairs, pairs, hipHostMallocDefault));
   HIPCHK(hipHostMalloc((void**)&sl.h_offsets, (total + 1) * sizeof(int64_t), hipHostMallocDefault));
   HIPCHK(hipHostMalloc((void**)&sl.h_maxc, sizeof(int32_t), hipHostMallocDefault));
   sl.h_final_cap = (int64_t)total * kDefaultCap;
@@ -181,7 +186,7 @@ void slot_free(Slot& sl) {
 // Device bytes one slot holds at the default record capacity.
 int64_t slot_bytes_for(int P, int N, int cap) {
   const int64_t total = 2 * (int64_t)P;
-  return (int64_t)P * sizeof(sxc_pair_dev) + total * N * 2 + total * 4 + total * cap * (72 + 8 + 72) + total * 12 + 64;
+  return (int64_t)P * (sizeof(sxc_pair_dev) + sizeof(int32_t)) + total * N * 2 + total * 4 + total * cap * (72 + 8 + 72) + total * 12 + 64;
 }
 
 // fresh: the pair kernel has just cleared the counts, so small launches may split a (pair,
@@ -217,6 +222,7 @@ int launch_scan_slot(sxc_server* sv, Slot& sl, bool fresh, bool order) {
   a.stats = nullptr;
   a.ptable = sv->ptable;
   a.table_prob = sv->prm.table_prob;
+  a.list = sl.kinds.mixed() ? (const int32_t*)(sl.pairs.as<sxc_pair_dev>() + sl.npairs) : nullptr;
   HIPCHK(sxc::launch_scan(sv->nb, a, 2 * sl.npairs, sl.kinds, fresh, sl.s));
   const int total = 2 * sl.npairs;
   HIPCHK(sxc::launch_count_offsets(sl.counts.as<int32_t>(), total, sl.cap, sl.offsets.as<int64_t>(),
@@ -265,7 +271,7 @@ int slot_fill(sxc_server* sv, Slot& sl) {
       d.q_record_len = qm.record_len;
       d.fast = b.fast ? 1 : 0;
       d.q_tail = -1;
-      ++sl.kinds.pairs[sxc::scan_kind(sv->h_tch[(size_t)ti].flags, sv->h_qch[(size_t)qi].flags)];
+      ++sl.kinds.pairs[pair_kind(sv, d)];
       ++pc.count;
       ++r->dispatched;
       // align_target order: query chunks outer, target chunks inner
@@ -282,7 +288,13 @@ int slot_fill(sxc_server* sv, Slot& sl) {
   }
   if (sl.npairs == 0) return SXC_OK;
   HIPCHK(hipEventRecord(sl.ev_start, sl.s));
-  HIPCHK(hipMemcpyAsync(sl.pairs.p, sl.h_pairs, (size_t)sl.npairs * sizeof(sxc_pair_dev), hipMemcpyHostToDevice, sl.s));
+  // the pairs and, behind them, their list by kind
+  size_t bytes = (size_t)sl.npairs * sizeof(sxc_pair_dev);
+  if (sl.kinds.mixed()) {
+    sl.kinds.list([&](int32_t k) { return pair_kind(sv, sl.h_pairs[k]); }, (int32_t*)(sl.h_pairs + sl.npairs));
+    bytes += (size_t)sl.npairs * sizeof(int32_t);
+  }
+  HIPCHK(hipMemcpyAsync(sl.pairs.p, sl.h_pairs, bytes, hipMemcpyHostToDevice, sl.s));
   sxc::PairArgs a{};
   a.tab = sv->ctx->d_tab;
   a.osc = sv->ctx->d_osc;

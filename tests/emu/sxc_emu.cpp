@@ -214,15 +214,26 @@ int run_batch(const sxc::HostBatch& hb, const sxc_params& prm, std::vector<sxc_r
     if (stats)
       for (int ps = 0; ps < total; ++ps) stats[2 * ps + 1] = 0;
   }
-  for (int blk = total * split - 1; blk >= 0; --blk) {
-    // the three kernels, as launched on the device (each skips the others' pairs)
-    EmuExec<int> ex(sxc::SCAN_NT);
-    memset(ssm_pure.data(), 0xCD, ssm_pure.size());
-    sxc::scan_body<NB | 32>(ex, ssm_pure.data(), sc, blk);
-    memset(ssm_n.data(), 0xCD, ssm_n.size());
-    sxc::scan_body<NB | 64>(ex, ssm_n.data(), sc, blk);
-    memset(ssm.data(), 0xCD, ssm.size());
-    sxc::scan_body<NB>(ex, ssm.data(), sc, blk);
+  // the three kernels, as launched on the device: each over its own pairs
+  auto kind_of = [&](int k) {
+    return sxc::scan_kind(hb.tchunks[hb.pairs[k].t_chunk].flags, hb.qchunks[hb.pairs[k].q_chunk].flags);
+  };
+  sxc::ScanKinds kinds;
+  for (int k = 0; k < (int)hb.pairs.size(); ++k) ++kinds.pairs[kind_of(k)];
+  std::vector<int32_t> list(hb.pairs.size());
+  kinds.list(kind_of, list.data());
+  const int32_t* first = list.data();
+  for (int kind = 0; kind < 3; ++kind) {
+    sc.list = kinds.mixed() ? first : nullptr;
+    first += kinds.pairs[kind];
+    for (int blk = kinds.pairs[kind] * prm.strands * split - 1; blk >= 0; --blk) {
+      EmuExec<int> ex(sxc::SCAN_NT);
+      std::vector<char>& mem = kind == 0 ? ssm_pure : kind == 1 ? ssm_n : ssm;
+      memset(mem.data(), 0xCD, mem.size());
+      if (kind == 0) sxc::scan_body<NB | 32>(ex, mem.data(), sc, blk);
+      if (kind == 1) sxc::scan_body<NB | 64>(ex, mem.data(), sc, blk);
+      if (kind == 2) sxc::scan_body<NB>(ex, mem.data(), sc, blk);
+    }
   }
   res.clear();
   const sxc::ResolveCtx rc{hb.seq.data(), hb.tchunks.data(), hb.qchunks.data(), hb.pairs.data(),

@@ -128,3 +128,64 @@ def test_matchup_runs_and_probabilities(ctx, letters):
             want = oracle.match_probability(t, q, int(st), int(sq), int(n), 1e6)
             assert p == want or abs(p - want) <= 1e-11 * abs(want) or (np.isnan(p) and np.isnan(want))
             assert i == oracle.print_match_ident(q, t, int(st), int(sq), int(n))
+
+
+@pytest.mark.parametrize("odd", [b"N", b"R", b""])
+def test_one_pair_of_a_rare_kind_in_a_large_batch(ctx, odd):
+    """More than 2^19 pairs, one of another kind: that pair's strands are shared between 16
+    workgroups each, and 2^20 strands times 16 workgroups of 256 threads are more than a launch takes.
+    (odd empty: one pure pair, all others with an N.)"""
+    from satsuma2_amd.api import ChunkPair, HomologyByXCorr, SlaveParams
+
+    n, at = (1 << 19) + 9, 77777
+    t, q = related(256, 256, "acgt", 3)
+    other = t[:100] + (odd or b"N") + t[101:]
+    seqs = {False: t if odd else other, True: other if odd else t}
+    prm = SlaveParams(t_chunk=256, q_chunk=256, target_total=1e6)
+    want = {}
+    for rare, s in seqs.items():
+        want[rare] = np.concatenate(oracle.align_batch([dict(tseq=s, qseq=q, q_record_len=256)],
+                                                       oracle.make_params(N=512, q_chunk=256, target_total=1e6)))
+        assert len(want[rare]) > 0
+    pairs = [ChunkPair(seqs[k == at], q, q_record=k) for k in range(n)]
+    print(f"[rare kind] {n} pairs, one with {odd or b'A/C/G/T only'}", flush=True)
+    got = HomologyByXCorr(ctx, prm).align_batch(pairs)
+    m, r = len(want[False]), len(want[True])
+    assert len(got) == m * (n - 1) + r
+    parts = np.concatenate([got[:m * at], got[m * at + r:]]).reshape(n - 1, m)
+    ids = np.array([k for k in range(n) if k != at], np.uint64)
+    for f in EXACT:
+        ref = want[False][f][None, :] if f != "query_id" else ids[:, None]
+        assert np.all(parts[f] == ref), f
+        assert np.array_equal(got[m * at:m * at + r][f], want[True][f] if f != "query_id" else np.full(r, at, np.uint64)), f
+
+
+def test_server_launches_of_mixed_kinds(ctx):
+    """A serving launch holds its pairs and, behind them, their list by kind: requests with every kind
+    of pair, one kind alone, full launches and a last one of a single pair."""
+    from satsuma2_amd.api import Chunk, Server, SlaveParams
+    from test_gpu_server import assert_records
+
+    kinds = ["acgt", "n_gap", "few", "acgt", "dense", "words"]
+    T, Q = [], []
+    for k in range(24):
+        t, q = related(1024 - k % 5, 1024, kinds[k % 6], 40 + k, reverse=k % 3 == 0)
+        T.append((t, 700 * k, 0, 20000))
+        Q.append((q[:500] + b"N" * 9 + q[509:] if k % 8 == 3 else q, 900 * k, k % 2, 30000))
+    prm = SlaveParams(t_chunk=1024, q_chunk=1024, target_total=20000.0)
+    srv = Server(ctx, prm, [Chunk(*c) for c in T], [Chunk(*c) for c in Q], max_pairs_per_launch=96, max_slots=2)
+
+    def want(blocks):
+        pairs = [dict(tseq=T[ti][0], qseq=Q[qi][0], t_chunk_start=T[ti][1], q_chunk_start=Q[qi][1], t_record=0,
+                      q_record=Q[qi][2], q_record_len=30000, fast=f)
+                 for tf, tt, qf, qt, f in blocks for qi in range(qf, qt + 1) for ti in range(tf, tt + 1)]
+        return np.concatenate(oracle.align_batch(pairs, oracle.make_params(N=2048, q_chunk=1024, target_total=20000.0),
+                                                 threads=16))
+
+    requests = [[(k, k, k, k, 0)] for k in range(6)] + [[(0, 23, 0, 3, 0)], [(0, 23, 4, 8, 1), (5, 5, 5, 5, 0)], [(0, 0, 0, 2, 0)]]
+    tickets = [srv.submit(r) for r in requests]
+    refs = [want(r) for r in requests]
+    assert sum(map(len, refs)) > 24
+    for r, ticket, ref in zip(requests, tickets, refs):
+        assert_records(srv.results(ticket), ref, r)
+    srv.close()
