@@ -104,8 +104,8 @@ int batch_upload(sxc_ctx* ctx, sxc_batch_dev& b) {
     HIPCHK(hipMemcpyAsync(b.pairs.p, hb.pairs.data(), hb.pairs.size() * sizeof(sxc_pair_dev), hipMemcpyHostToDevice, s));
   std::vector<int32_t> list;
   if (b.kinds.mixed()) {
-    list.resize(hb.pairs.size());
-    b.kinds.list([&](int32_t k) { return pair_kind(hb, hb.pairs[(size_t)k]); }, list.data());
+    list.resize(hb.pairs.size() * (size_t)b.prm.strands);
+    b.kinds.list([&](int32_t k) { return pair_kind(hb, hb.pairs[(size_t)k]); }, b.prm.strands, list.data());
     HIPCHK(b.list.ensure(list.size() * sizeof(int32_t)));
     HIPCHK(hipMemcpyAsync(b.list.p, list.data(), list.size() * sizeof(int32_t), hipMemcpyHostToDevice, s));
   }

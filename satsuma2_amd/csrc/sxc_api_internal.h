@@ -65,7 +65,7 @@ struct sxc_batch_dev {
   DevBuf nflag;  // records the last scan flagged near min_prob (the counts kernel reads and clears it)
   sxc::HostBatch hb;
   sxc::ScanKinds kinds;  // of hb.pairs
-  DevBuf list;           // hb.pairs by kind (ScanKinds::list) where kinds are mixed
+  DevBuf list;           // their (pair, strand)s by kind (ScanKinds::list) where kinds are mixed
   sxc_params prm{};
   int nb = 0;
   int slot_cap = 64;

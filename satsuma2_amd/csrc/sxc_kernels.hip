@@ -316,7 +316,7 @@ hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& ki
     const int n = kinds.pairs[k] * a.strands;
     b.split = can_split ? scan_split(k, nb, n) : 1;
     b.list = a.list ? a.list + first : nullptr;
-    first += kinds.pairs[k];
+    first += n;
     // a launch of 2^32 threads or more is not refused: its last workgroups are missing
     if ((int64_t)n * b.split * SCAN_NT >= (int64_t)1 << 32) return hipErrorInvalidValue;
     const hipError_t e = (k == 0 ? launch_scan_pure : k == 1 ? launch_scan_n : launch_scan_general)(nb, b, n * b.split, s);

@@ -71,7 +71,7 @@ struct ScanArgs {
   // on counts[ps], which must be zero at launch (the pair kernel clears it), and stats
   // runs are added atomically.
   int32_t split;
-  const int32_t* list;       // optional: the pairs to scan (null: pair 0 on)
+  const int32_t* list;       // optional: the (pair, strand)s to scan (null: 0 on)
 };
 
 // The kinds of chunk pairs the scan has a kernel of its own for, and how many of a launch's
@@ -84,15 +84,18 @@ struct ScanKinds {
   int32_t pairs[3] = {0, 0, 0};
   bool mixed() const { return (pairs[0] > 0) + (pairs[1] > 0) + (pairs[2] > 0) > 1; }
   int32_t all() const { return pairs[0] + pairs[1] + pairs[2]; }
-  // Of a mixed launch, the pairs grouped by kind: a kind's launch covers its own pairs only.  (Over
+  // Of a mixed launch, the (pair, strand)s grouped by kind: a kind's launch covers its own only.  (Over
   // all pairs, with the others' workgroups leaving at once, the shares of a rare kind's strands
   // multiplied the whole grid: one pure pair among 100000 with N at N = 512 took 3.2 M workgroups,
   // 9.27 ms against 7.54, and one among 524297 lost its records, as a grid of 2^32 threads or more
   // wraps.  One pair with N among 4096 of 4096 bp: 0.615 and 0.598 ms.)
   template <class KindOf>
-  void list(KindOf&& kind_of, int32_t* out) const {
-    int32_t at[3] = {0, pairs[0], pairs[0] + pairs[1]};
-    for (int32_t k = 0; k < all(); ++k) out[at[kind_of(k)]++] = k;
+  void list(KindOf&& kind_of, int strands, int32_t* out) const {
+    int32_t at[3] = {0, strands * pairs[0], strands * (pairs[0] + pairs[1])};
+    for (int32_t k = 0; k < all(); ++k) {
+      int32_t& to = at[kind_of(k)];
+      for (int s = 0; s < strands; ++s) out[to++] = strands * k + s;
+    }
   }
 };
 
@@ -1397,11 +1400,9 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
   using SS = ScanSmem<NB>;
   constexpr int N = SS::N;
   const int split = a.split > 1 ? a.split : 1;
-  const int at = blk / split, part = blk % split;
-  const int pair = a.list ? a.list[at / a.strands] : at / a.strands;
-  const int strand = at % a.strands;
-  const int ps = pair * a.strands + strand;
-  const sxc_pair_dev pr = a.pairs[pair];
+  const int ps = a.list ? a.list[blk / split] : blk / split, part = blk % split;
+  const sxc_pair_dev pr = a.pairs[ps / a.strands];
+  const int strand = ps % a.strands;
   const sxc_chunk tch = a.tchunks[pr.t_chunk];
   const sxc_chunk qch = a.qchunks[pr.q_chunk];
   // each kernel takes its own kind only, whatever it is launched over

@@ -149,7 +149,7 @@ int slot_alloc(sxc_server* sv, Slot& sl) {
   HIPCHK(hipEventCreate(&sl.ev_start));
   HIPCHK(hipEventCreate(&sl.ev_count));
   HIPCHK(hipEventCreate(&sl.ev_pack));
-  const size_t pairs = (size_t)P * (sizeof(sxc_pair_dev) + sizeof(int32_t));  // and their list by kind
+  const size_t pairs = (size_t)P * (sizeof(sxc_pair_dev) + 2 * sizeof(int32_t));  // and their strands by kind
   HIPCHK(sl.pairs.ensure(pairs));
   HIPCHK(sl.cands.ensure(total * N * sizeof(uint16_t)));
   HIPCHK(sl.ncand.ensure(total * sizeof(int32_t)));
@@ -186,7 +186,7 @@ void slot_free(Slot& sl) {
 // Device bytes one slot holds at the default record capacity.
 int64_t slot_bytes_for(int P, int N, int cap) {
   const int64_t total = 2 * (int64_t)P;
-  return (int64_t)P * (sizeof(sxc_pair_dev) + sizeof(int32_t)) + total * N * 2 + total * 4 + total * cap * (72 + 8 + 72) + total * 12 + 64;
+  return (int64_t)P * (sizeof(sxc_pair_dev) + 2 * sizeof(int32_t)) + total * N * 2 + total * 4 + total * cap * (72 + 8 + 72) + total * 12 + 64;
 }
 
 // fresh: the pair kernel has just cleared the counts, so small launches may split a (pair,
@@ -288,11 +288,11 @@ int slot_fill(sxc_server* sv, Slot& sl) {
   }
   if (sl.npairs == 0) return SXC_OK;
   HIPCHK(hipEventRecord(sl.ev_start, sl.s));
-  // the pairs and, behind them, their list by kind
+  // the pairs and, behind them, their strands by kind
   size_t bytes = (size_t)sl.npairs * sizeof(sxc_pair_dev);
   if (sl.kinds.mixed()) {
-    sl.kinds.list([&](int32_t k) { return pair_kind(sv, sl.h_pairs[k]); }, (int32_t*)(sl.h_pairs + sl.npairs));
-    bytes += (size_t)sl.npairs * sizeof(int32_t);
+    sl.kinds.list([&](int32_t k) { return pair_kind(sv, sl.h_pairs[k]); }, 2, (int32_t*)(sl.h_pairs + sl.npairs));
+    bytes += (size_t)sl.npairs * 2 * sizeof(int32_t);
   }
   HIPCHK(hipMemcpyAsync(sl.pairs.p, sl.h_pairs, bytes, hipMemcpyHostToDevice, sl.s));
   sxc::PairArgs a{};

@@ -220,12 +220,12 @@ int run_batch(const sxc::HostBatch& hb, const sxc_params& prm, std::vector<sxc_r
   };
   sxc::ScanKinds kinds;
   for (int k = 0; k < (int)hb.pairs.size(); ++k) ++kinds.pairs[kind_of(k)];
-  std::vector<int32_t> list(hb.pairs.size());
-  kinds.list(kind_of, list.data());
+  std::vector<int32_t> list(total);
+  kinds.list(kind_of, prm.strands, list.data());
   const int32_t* first = list.data();
   for (int kind = 0; kind < 3; ++kind) {
     sc.list = kinds.mixed() ? first : nullptr;
-    first += kinds.pairs[kind];
+    first += kinds.pairs[kind] * prm.strands;
     for (int blk = kinds.pairs[kind] * prm.strands * split - 1; blk >= 0; --blk) {
       EmuExec<int> ex(sxc::SCAN_NT);
       std::vector<char>& mem = kind == 0 ? ssm_pure : kind == 1 ? ssm_n : ssm;
