@@ -10,6 +10,7 @@
 #include "sxc_kernels.h"
 #include "sxc_pipeline.h"
 #include "sxc_scan.h"
+#include "sxc_scan_kernels.h"
 
 namespace sxc {
 
@@ -287,16 +288,51 @@ hipError_t launch_correlate(int geo, const PairArgs& a, int total, hipStream_t s
 // positions: 32 strands 359 / 196 / 146 / 94 / 81, 128 strands 356 / 203 / 203 / 202 / 203, 512
 // strands 501 / 438 / 555 / - / -, 2048 strands 1434 / 1406 / 1965 / - / -.
 // With N, lags are taken 8 or 16 at a time: up to 2048 workgroups in all (8 per CU), more than 4 per
-// strand only to 128 strands (1 / 2 / 4 / 8 at N = 8192: 96 strands 156 / 95 / 76 / 64, 256 strands 163 /
+// strand only to 102 strands (1 / 2 / 4 / 8 at N = 8192: 96 strands 156 / 95 / 76 / 64, 256 strands 163 /
 // 113 / 103 / 117, 400 strands 183 / 141 / 154 / 162, 800 strands 251 / 224 / 242 / 282; at N = 2048 400
-// strands 312 / 208 / 180 / 170).  With other letters (5 workgroups per CU) the same to 320 strands,
-// 2 above them: 2 / 4 per strand, one such letter and one in 16 bases, 200 strands 179 / 192 and 731 / 519,
-// 320 strands 193 / 258 and 785 / 943, 512 strands 213 / 307 and 776 / 1062; at N = 2048, one in 16, 320
-// strands 611 / 484, 400 strands 647 / 752.
+// strands 312 / 208 / 180 / 170).  With other letters the same to 320 strands, 2 above them.
+// Then no more than pays by the rounds of workgroups that fit the device (scan_resident), as a share
+// costs its packing and the middle shares hold the longer diagonals: with other letters at every N,
+// with N at 32768 where fewer than 8 of them fit a CU and one per strand is resident at once.  us with
+// 1 / 2 / 3 / 4 shares, one other letter in the target and one in 16 bases: N = 512, 800 strands 120 / 200 /
+// 200 / 292 and 171 / 183 / 169 / 197; N = 2048, 800 strands 352 / 368 / 326 / 459 and 1242 / 1152 / 1100 /
+// 1222; N = 8192, 256 strands 302 / 256 / 233 / 270 and 1307 / 817 / 727 / 657, 320 strands 324 / 269 /
+// 256 / 398 and 1340 / 837 / 761 / 1048, 640 strands 347 / 460 / 346 / 605 and 1381 / 1413 / 1371 / 1555;
+// N = 16384, 160 strands 623 / 507 / 443 / 744 and 4486 / 2491 / 2378 / 3350; N = 32768, 128 strands 2092 /
+// 1471 / 1755 / 2376 and 15393 / 8154 / 11801 / 11592, 256 strands 2092 / 2907 / 3011 / 4739 and 15389 /
+// 16005 / 19767 / 22960, 320 strands 4065 / 4220 / 3431 / 5939 and 30355 / 23276 / 23561 / 28650; with N at
+// 32768, 160 strands 1550 / 1102 / 872 / 1198, 512 strands 1933 / 2118 / 2399 / 2866.
+static int resident_scans(int kind, int nb) {  // workgroups that fit 256 CUs
+#define CALL(X) return 256 * (kind == SCAN_N ? scan_resident<(X) | 64>() : scan_resident<X>())
+  switch (nb) {
+    case 12: CALL(12);
+    case 13: CALL(13);
+    case 14: CALL(14);
+    case 15: CALL(15);
+    default: CALL(11);  // (the most waves already)
+  }
+#undef CALL
+}
+
+// At most `most` shares of n strands: the fewest whose rounds on `resident` places, per share, are
+// within 10% of the least.
+static int shares_by_rounds(int n, int resident, int most) {
+  if ((int64_t)n * most <= resident) return most;
+  auto rounds = [&](int k) { return ((int64_t)n * k + resident - 1) / resident; };
+  int best = 1;
+  for (int k = 2; k <= most; ++k)
+    if (rounds(k) * best < rounds(best) * k) best = k;
+  for (int k = 1; k < best; ++k)
+    if (10 * rounds(k) * best <= 11 * rounds(best) * k) return k;
+  return best;
+}
+
 static int scan_split(int kind, int nb, int n) {
   if (n <= 0) return 1;
-  if (kind == 0) return n <= 32 ? 16 : n <= 128 ? 8 : n <= (nb >= 14 ? 2048 : 768) ? 2 : 1;
-  return std::max(1, std::min({2048 / n, std::max(kind == 2 && n > 320 ? 2 : 4, 512 / n), 16}));
+  if (kind == SCAN_PURE) return n <= 32 ? 16 : n <= 128 ? 8 : n <= (nb >= 14 ? 2048 : 768) ? 2 : 1;
+  const int most = std::max(1, std::min({2048 / n, std::max(kind == SCAN_GENERAL && n > 320 ? 2 : 4, 512 / n), 16}));
+  const int resident = resident_scans(kind, nb);
+  return kind == SCAN_GENERAL || (nb == 15 && n <= resident) ? shares_by_rounds(n, resident, most) : most;
 }
 
 hipError_t launch_scan(int nb, const ScanArgs& a, int total, const ScanKinds& kinds, bool can_split, hipStream_t s) {

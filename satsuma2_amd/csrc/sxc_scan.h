@@ -152,7 +152,7 @@ struct ScanSmem {
   // The kernel with N (BMRUNS) keeps each epoch's flags in a bitmap of WPL words per lag and
   // turns its rising edges into runs afterwards; the general kernel scans contiguous
   // segments per thread and stitches runs across them.  BMRUNS, and the general kernel from
-  // N = 8192 (5 of its workgroups per CU instead of 4: 200 strands 0.54 ms instead of 0.74; at
+  // N = 8192 (4 of its workgroups per CU instead of 3: 200 strands 0.54 ms instead of 0.74; at
   // N = 2048 0.57 instead of 0.44), take one epoch at a time (drained after every epoch) in
   // 4-byte queue entries {lag - first lag of the epoch (RB bits), ns (NSB = LOG - 1), ne
   // (LOG)}; otherwise 16-lag epochs accumulate in 8-byte entries {lag rank, ns | ne << 16}

@@ -12,7 +12,10 @@ struct NoRegs {};
 // Waves per SIMD the register budget is set for.  The sliced scan (pure A/C/G/T) keeps 32 words of
 // a slice and their counts in registers: 6 waves (80 registers, 6 spilled) take 0.507 ms for 8192
 // strands at N = 8192 and 1.47 for 24000 at 2048, 5 waves 0.529 and 1.53, 8 (26 spilled) 0.515 and
-// 1.40.  The general scan's LDS plan admits 5 workgroups at N = 8192.  The A/C/G/T/N scan gets as many of its 4-wave workgroups per CU as its LDS plan admits,
+// 1.40.  The general scan is compiled for 5 waves also where its LDS plan admits fewer workgroups (4 at
+// N = 8192, 2 at 16384): it then has the same registers (106, none spilled), but compiled for as many as fit
+// it took 276 instead of 224 us for 128 strands with one other letter at N = 8192 and 559 instead of 446
+// at 16384.  The A/C/G/T/N scan gets as many of its 4-wave workgroups per CU as its LDS plan admits,
 // up to 8 waves (the spills the budget costs are cheaper than the latency the waves hide).
 template <int NB>
 constexpr int scan_waves() {
@@ -25,6 +28,15 @@ constexpr int scan_waves() {
     return wg < 1 ? 1 : (wg > 8 ? 8 : wg);
   }
 }
+
+// Workgroups that a CU holds at once.
+template <int NB>
+constexpr int scan_resident() {
+  constexpr int wg = 163840 / ScanSmem<NB>::BYTES;
+  return wg < scan_waves<NB>() ? wg : scan_waves<NB>();
+}
+static_assert(scan_resident<12>() == 5 && scan_resident<13>() == 4 && scan_resident<14>() == 2, "");
+static_assert(scan_resident<15>() == 1 && scan_resident<15 | 64>() == 2, "");
 
 template <int NB>
 __global__ __launch_bounds__(SCAN_NT) __attribute__((amdgpu_waves_per_eu(scan_waves<NB>()))) void k_scan(ScanArgs a) {

@@ -189,3 +189,25 @@ def test_server_launches_of_mixed_kinds(ctx):
     for r, ticket, ref in zip(requests, tickets, refs):
         assert_records(srv.results(ticket), ref, r)
     srv.close()
+
+
+@pytest.mark.parametrize("letters", ["n_gap", "few", "dense"])
+@pytest.mark.parametrize("t_chunk,n", [(2048, 320), (2048, 321), (4096, 128), (4096, 171), (4096, 256), (8192, 64), (8192, 86),
+                                       (8192, 128), (16384, 16), (16384, 32), (16384, 64), (16384, 86), (16384, 129)])
+def test_shares_of_resident_workgroups(ctx, t_chunk, n, letters):
+    """Numbers of strands around those where as many shares as before no longer fit the device at once."""
+    shapes = [(t_chunk - k % 3, (t_chunk, t_chunk // 3)[k % 2], letters) for k in range(4)]
+    four = chunk_pairs(shapes)
+    ref = oracle.align_batch([dict(tseq=p.tseq, qseq=p.qseq, q_record_len=len(p.qseq)) for p in four],
+                             oracle.make_params(N=2 * t_chunk, q_chunk=t_chunk, target_total=1e6), threads=4,
+                             cap_per_pair=2048)
+    from satsuma2_amd.api import ChunkPair, HomologyByXCorr, SlaveParams
+
+    pairs = [ChunkPair(four[k % 4].tseq, four[k % 4].qseq, q_record=k) for k in range(n)]
+    got = HomologyByXCorr(ctx, SlaveParams(t_chunk=t_chunk, q_chunk=t_chunk, target_total=1e6)).align_batch(pairs)
+    assert np.array_equal(got["query_id"], np.repeat(np.arange(n), [len(ref[k % 4]) for k in range(n)]))
+    want = np.concatenate([ref[k % 4] for k in range(n)])
+    assert len(want) > 0
+    for f in EXACT[1:]:
+        assert np.array_equal(got[f], want[f]), f
+    assert np.all(np.abs(got["prob"] - want["prob"]) <= 1e-11 * np.abs(want["prob"]))
