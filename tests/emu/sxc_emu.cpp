@@ -118,11 +118,19 @@ int run_batch(const sxc::HostBatch& hb, const sxc_params& prm, std::vector<sxc_r
                    (int)which.size(), spectra.data(), dst.data(), nullptr,
                    tails ? hb.ttail.data() : nullptr, tails ? hb.tails.data() : nullptr,
                    tails ? hb.segs.data() : nullptr, tails ? src_sig.data() : nullptr, 0};
-  for (int k = 0; k < sa.n; ++k) {
-    EmuExec<sxc::Regs<GEO>> ex(G::NT);
-    memset(sm.data(), 0xCD, sm.size());
-    sxc::spectra_body<GEO>(ex, sm.data(), sa, k);
-  }
+  // SXC_EMU_PARTS=1: a workgroup per channel, as launches of few strands or chunks run (default
+  // geometries only)
+  const bool by_channel = GEO == NB && getenv("SXC_EMU_PARTS");
+  for (int k = 0; k < sa.n; ++k)
+    for (int ch = 0; ch < (by_channel ? 4 : 1); ++ch) {
+      EmuExec<sxc::Regs<GEO>> ex(G::NT);
+      memset(sm.data(), 0xCD, sm.size());
+      if (by_channel) {
+        sxc::spectra_body<GEO>(ex, sm.data(), sa, k, 3 - ch, 4 - ch);
+      } else {
+        sxc::spectra_body<GEO>(ex, sm.data(), sa, k);
+      }
+    }
   const int total = (int)hb.pairs.size() * prm.strands;
   std::vector<sxc_result_dev> slots((size_t)total * cap);
   std::vector<uint64_t> keys((size_t)total * cap);
@@ -169,8 +177,25 @@ int run_batch(const sxc::HostBatch& hb, const sxc_params& prm, std::vector<sxc_r
       }
     pa.qspectra = qspec.data();
   }
+  std::vector<float> parts(by_channel ? (size_t)total * 4 * G::N : 0);
   for (int ps = 0; ps < total; ++ps) {
     EmuExec<sxc::Regs<GEO>> ex(G::NT);
+    if constexpr (GEO == NB) {
+      if (by_channel) {
+        pa.parts = parts.data();
+        for (int ch = 3; ch >= 0; --ch) {
+          memset(sm.data(), 0xCD, sm.size());
+          sxc::correlate_body<GEO, true>(ex, sm.data(), pa, ps, ch, ch + 1);
+        }
+        memset(sm.data(), 0xCD, sm.size());
+        sxc::sum_peaks_body<GEO>(ex, sm.data(), pa, ps);
+        const float* p = parts.data() + (size_t)ps * 4 * G::N;
+        if (xc_out)
+          for (int i = 0; i < G::N; ++i)
+            xc_out[(size_t)ps * G::N + i] = (((0.f + p[i]) + p[G::N + i]) + p[2 * G::N + i]) + p[3 * G::N + i];
+        continue;
+      }
+    }
     memset(sm.data(), 0xCD, sm.size());
     sxc::correlate_body<GEO>(ex, sm.data(), pa, ps);
   }
