@@ -262,8 +262,13 @@ void sxc_server_destroy(sxc_server* srv);
  * geometry of the pair kernel and of the target-spectra kernel for each length in
  * [N_lo, N_hi] on a synthetic batch (chunks of N/2 bases, both strands), checks that all
  * geometries accept identical lags, and makes the fastest the context's choice for later
- * batches and servers.  out receives one entry per (length, geometry).  The reference has
- * one CPU FFT and no counterpart; sxc_set_geometry applies a saved choice without timing. */
+ * batches and servers.  The choice holds for launches of more than 128 (pair, strand)s (the
+ * pair kernel) or target chunks (the spectra kernel).  Smaller ones, which it was not timed
+ * for, take a workgroup per channel in the default geometry, except in sxc_align_pair_static
+ * and in a server whose budget has no room for that.  out receives one entry per (length,
+ * geometry).  The reference has one CPU FFT and no counterpart; sxc_set_geometry applies a
+ * saved choice without timing, within
+ * the same limits. */
 typedef struct {
   int32_t stage_a;          /* positions per thread in stage A (16 or 32) */
   int32_t round_levels;     /* butterfly levels per LDS round, at most (2 or 3) */
