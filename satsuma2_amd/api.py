@@ -73,9 +73,9 @@ class Context:
     # ---- FFT kernel geometry (autotuner)
     def autotune(self, N_lo: int = 8192, N_hi: int = 0) -> list:
         """Times every compiled FFT geometry of the pair and target-spectra kernels for each
-        length in [N_lo, N_hi] (sxc_autotune) and keeps the fastest for launches of more than 128
-        strands (or target chunks); returns one dict per (length, geometry): N, pairs, geo (a Geometry tuple), correlate_ms, spectra_ms,
-        chosen_correlate, chosen_spectra."""
+        length in [N_lo, N_hi] (sxc_autotune) and keeps the fastest for launches of more than
+        128 strands (or target chunks); returns one dict per (length, geometry): N, pairs, geo
+        (a Geometry tuple), correlate_ms, spectra_ms, chosen_correlate, chosen_spectra."""
         N_hi = N_hi or N_lo
         cap = 128
         out = (_lib.TuneEntry * cap)()

@@ -143,3 +143,49 @@ def test_look_back_limit(ctx):
         for jump in (64, 65):
             got, _ = kmatch(ctx, query, target, 11, 11, jump, 1)
             assert got.tobytes() == expected(query, target, 11, 11, jump)[0].tobytes(), (gap, jump)
+
+
+def one_bucket(n, bits, seed):
+    """n records of 31 bases whose k-mers fall into bucket 0 of 2^bits (sxc_kmatch_unique.h: mix)."""
+    rng = np.random.default_rng(seed)
+    f = rng.integers(0, 1 << 62, n << (bits + 1), dtype=np.uint64)
+    rc = np.zeros_like(f)
+    for i in range(31):
+        rc = (rc << np.uint64(2)) | (np.uint64(3) - ((f >> np.uint64(2 * i)) & np.uint64(3)))
+    h = np.minimum(f, rc) * np.uint64(0x9E3779B97F4A7C15)
+    f = f[((h ^ (h >> np.uint64(32))) & np.uint64((1 << bits) - 1)) == 0][:n]
+    assert len(f) == n
+    code = np.stack([(f >> np.uint64(2 * (30 - i))) & np.uint64(3) for i in range(31)], 1).astype(np.uint8)
+    return [bytes(r) for r in np.frombuffer(b"ACGT", np.uint8)[code]]
+
+
+@pytest.mark.parametrize("name", ["one wave", "several workgroups", "full", "just over"])
+def test_more_kmers_than_a_bucket_holds(ctx, name):
+    """More than 1024 different k-mers in one bucket: the general path decides, after the device path has
+    run in part.  Records, order and counts as ever, and the next run on the context is its own."""
+    from satsuma2_amd.kmatch import kmatch
+
+    rng = np.random.default_rng(len(name))
+    if name == "one wave":  # 1500 table slots: 4 buckets
+        r = one_bucket(1250, 2, 1)
+        query, target = r[:750], r[500:]
+    elif name == "several workgroups":  # 20000 slots: 64 buckets, one of more than 16384 entries
+        r = one_bucket(3000, 6, 2)
+        query = r[:1800] + [r[int(i)] for i in rng.integers(0, 700, 8200)]
+        target = r[1000:] + [r[int(i)] for i in rng.integers(1500, 2400, 8000)]
+    else:  # 1024 k-mers fill the table, 1025 do not fit
+        r = one_bucket(1024 if name == "full" else 1025, 2, 3)
+        query, target = r[:700], r[300:]
+    target = [t.translate(COMP)[::-1] if k % 3 == 0 else t for k, t in enumerate(target)]
+    print(f"[kmatch] {name}: {len(query)} and {len(target)} records", flush=True)
+    got, st = kmatch(ctx, query, target, 31, 31, 30, 1)
+    want, nq, nt, joined = expected(query, target, 31, 31, 30)
+    assert len(want) > 100
+    assert (st["query_kept"], st["target_kept"], st["joined"], st["blocks"]) == (nq, nt, joined, len(want))
+    assert got.tobytes() == want.tobytes()
+    assert (st["sweep_ms"] > 0) == (name != "full")  # chained on the host: the general path
+    q, t = genomes("records")
+    got, st = kmatch(ctx, q, t, 21, 40, 20, 1)
+    want, nq, nt, joined = expected(q, t, 21, 40, 20)
+    assert (st["query_kept"], st["target_kept"], st["joined"]) == (nq, nt, joined)
+    assert got.tobytes() == want.tobytes()
