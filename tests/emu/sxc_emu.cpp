@@ -348,6 +348,13 @@ void emu_keep_band(double min_prob, double target_size, double* lo, double* hi) 
   sxc::keep_band(min_prob, target_size, lo, hi);
 }
 
+// The shortest flagged stretch a kept run can have, by kind of pair (sxc::set_keep).
+void emu_min_run(double min_prob, double target_size, int32_t* out) {
+  sxc::ScanArgs a{};
+  sxc::set_keep(a, min_prob, target_size);
+  for (int k = 0; k < 3; ++k) out[k] = a.min_run[k];
+}
+
 // FFT of one signal through stage A + rounds (spectra_body with a given signal).
 int emu_fft_forward(const float* in, float* out, int N) {
   const Tables& T = tables();

@@ -42,3 +42,24 @@ def related(lt: int, lq: int, letters: str, seed: int, reverse=False):
         at = (lq - n) // 3
         q[at:at + n] = piece
     return other_letters(t.tobytes(), letters, rng), bytes(q.tobytes())
+
+
+# (target total, gate of pure pairs, gate of pairs with few other letters): the shortest stretch a kept run
+# can have (keep_min_run) is looked for 1, 2, 4 or 8 positions at a time
+GATES = [(1e3, 1, 1), (3e4, 2, 1), (5e4, 2, 1), (1e5, 4, 2), (2e5, 4, 2), (1e6, 4, 4), (4e6, 8, 4), (1e7, 8, 4), (1e9, 8, 8)]
+
+
+def short_runs(n: int, letters: str, seed: int):
+    """(target, query) whose kept runs are short: the target all G/C, the query all A/T but for stretches of
+    24 to 40 positions where they agree, on as many A/T as G/C, so that little is expected by chance."""
+    rng = np.random.default_rng(seed)
+    t = rng.choice(list(b"GC"), n).astype(np.uint8)
+    q = rng.choice(list(b"AT"), n).astype(np.uint8)
+    shift, at = int(rng.integers(5, 40)), 60 + seed % 32
+    while at + 110 < n - shift:
+        m = int(rng.integers(24, 41))
+        hit = at + rng.permutation(m)[:m - int(rng.integers(0, 4))]
+        t[hit] = rng.permutation(np.resize(rng.permutation(list(b"ACGT")), len(hit)))
+        q[hit + shift] = t[hit]
+        at += m + int(rng.integers(50, 70))
+    return other_letters(t.tobytes(), letters, rng), bytes(q.tobytes())

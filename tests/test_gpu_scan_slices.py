@@ -9,7 +9,7 @@ import pytest
 
 import oracle
 from conftest import dense_run_pair
-from scan_cases import LENGTHS, LETTERS, related
+from scan_cases import GATES, LENGTHS, LETTERS, related, short_runs
 
 pytestmark = pytest.mark.gpu
 
@@ -211,3 +211,14 @@ def test_shares_of_resident_workgroups(ctx, t_chunk, n, letters):
     for f in EXACT[1:]:
         assert np.array_equal(got[f], want[f]), f
     assert np.all(np.abs(got["prob"] - want["prob"]) <= 1e-11 * np.abs(want["prob"]))
+
+
+@pytest.mark.parametrize("letters", ["acgt", "few", "words", "n_gap"])
+@pytest.mark.parametrize("target_total", [g[0] for g in GATES])
+def test_every_gate(ctx, target_total, letters):
+    """Target sizes whose shortest kept run asks for each gate (tests/test_scan_slices.py says which)."""
+    from satsuma2_amd.api import ChunkPair
+
+    pairs = [ChunkPair(*(short_runs(500, letters, k) if k < 64 else related(900, 1000, letters, k, reverse=k % 2 == 1)),
+                       t_record=k, q_record=k, q_record_len=500) for k in range(68)]
+    assert len(check(ctx, pairs, 1024, target_total)) >= (3 if target_total > 1e8 else 40)

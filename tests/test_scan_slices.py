@@ -10,7 +10,7 @@ import pytest
 import hostbuild
 import oracle
 from conftest import dense_run_pair
-from scan_cases import LENGTHS, LETTERS, related
+from scan_cases import GATES, LENGTHS, LETTERS, related, short_runs
 from test_emu import COLS, emu_batch
 
 
@@ -57,3 +57,18 @@ def test_more_blocks_than_the_queue(emu, letter):
     t = dense_run_pair(length=2048)
     t = t[:700] + letter + t[700 + len(letter):]
     assert len(check(emu, [dict(tseq=t, qseq=t, t_record=0, q_record=0)], 4096, 10.0)) > 0
+
+
+@pytest.mark.parametrize("letters", ["acgt", "few", "words"])
+@pytest.mark.parametrize("target_total,pure,general", GATES)
+def test_every_gate(emu, target_total, pure, general, letters):
+    """Gates 1, 2, 4 and 8, each by a target size whose shortest kept run asks for it; the runs start at
+    every position of a block."""
+    least = (C.c_int32 * 3)()
+    emu.emu_min_run(C.c_double(0.99), C.c_double(target_total), least)
+    assert [max(g for g in (1, 2, 4, 8) if g <= n) for n in (least[0], least[2])] == [pure, general]
+    pairs = []
+    for k in range(35):
+        t, q = short_runs(500, letters, k) if k < 32 else related(900, 1000, letters, k, reverse=k == 33)
+        pairs.append(dict(tseq=t, qseq=q, t_record=k, q_record=k))
+    assert len(check(emu, pairs, 2048, target_total)) >= (3 if target_total > 1e8 else 25)
