@@ -33,9 +33,8 @@ constexpr uint32_t kNone = 0xffffffffu;     // no entry of this k-mer on a side
 constexpr uint32_t kMulti = 0xfffffffeu;    // more than one
 constexpr uint32_t kNeg = 0x80000000u;      // the reverse complement was the smaller
 // A bijection of the 64-bit words (a product, its upper half folded into the lower): the low bits
-// spread the k-mers over the buckets, the top bits over a bucket's table.  The radix sort is
-// given low bits: asked to sort 64-bit keys by bits that end at 64, the library's sort does not
-// return.
+// spread the k-mers over the buckets, the top bits over a bucket's table.  (The radix sort is given
+// low bits, as no call ends at bit 64: see sort_pairs.)
 constexpr uint64_t kMul = 0x9E3779B97F4A7C15ull;
 constexpr uint64_t inverse(uint64_t a) {
   uint64_t x = a;  // correct to 3 bits, doubled by each step
