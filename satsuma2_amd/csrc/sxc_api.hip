@@ -138,7 +138,7 @@ int batch_alloc(sxc_ctx* ctx, sxc_batch_dev& b) {
   HIPCHK(b.slots.ensure((size_t)total * b.slot_cap * sizeof(sxc_result_dev)));
   HIPCHK(b.keys.ensure((size_t)total * b.slot_cap * sizeof(uint64_t)));
   HIPCHK(b.counts.ensure((size_t)total * sizeof(int32_t)));
-  HIPCHK(b.stats.ensure((size_t)total * 2 * sizeof(int32_t)));
+  if (b.want_stats) HIPCHK(b.stats.ensure((size_t)total * 2 * sizeof(int32_t)));
   HIPCHK(b.offsets.ensure((size_t)total * sizeof(int64_t)));
   HIPCHK(b.total.ensure(2 * sizeof(int64_t)));
   if (total <= sxc::CHANNEL_SPLIT) HIPCHK(b.parts.ensure((size_t)total * 4 * b.prm.N * sizeof(float)));

@@ -280,8 +280,7 @@ struct Buffers {
 // Pairs sorted by key bits [0, end).  Asked once for bits [63, 64) of 100 such keys, the library's sort
 // had not returned after 60 s; the cause is not known, so no call goes to it with an end of 64.
 template <class V>
-hipError_t sort_pairs(void* tmp, size_t& bytes, const uint64_t* k0, uint64_t* k1, const V* v0, V* v1, size_t n, int end,
-                      hipStream_t s) {
+hipError_t sort_pairs(void* tmp, size_t& bytes, uint64_t* k0, uint64_t* k1, V* v0, V* v1, size_t n, int end, hipStream_t s) {
   if (end < 1 || end > 63) return hipErrorInvalidValue;
   return rocprim::radix_sort_pairs(tmp, bytes, k0, k1, v0, v1, n, 0, end, s);
 }

@@ -184,7 +184,7 @@ __global__ void k_unique_unfilled(uint64_t* keys, uint32_t* vals, int64_t slots_
   ctl->n = n;
 }
 
-// First entry of every bucket; the buckets above kHeavy are listed.
+// First entry of every bucket.
 __global__ __launch_bounds__(256) void k_bounds(const uint64_t* keys, uint32_t n, uint32_t buckets, uint32_t* start) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i > n) return;
@@ -193,6 +193,7 @@ __global__ __launch_bounds__(256) void k_bounds(const uint64_t* keys, uint32_t n
   for (uint32_t b = b0; b <= b1; ++b) start[b] = i;
 }
 
+// The buckets above kHeavy.
 __global__ __launch_bounds__(256) void k_heavy_list(const uint32_t* start, uint32_t buckets, uint32_t* list, Ctl* ctl) {
   const uint32_t b = blockIdx.x * 256u + threadIdx.x;
   if (b < buckets && start[b + 1] - start[b] > kHeavy) list[atomicAdd(&ctl->heavy, 1u)] = b;

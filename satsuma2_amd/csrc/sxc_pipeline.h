@@ -158,7 +158,7 @@ SXC_HD inline const float* twiddle_table(const char* sm, const sxc_tables* tab) 
 // The class cache's entry for positions past the chunk's end: their signal is e * 0 = 0.
 constexpr unsigned CLASS_PAST = SXC_NCLASS;
 
-enum { MISC_L = 0, MISC_THIRDS = 1, MISC_NCAND = 2, MISC_KEPT = 3, MISC_Q4 = 4 /* 4 ints */, MISC_RUNS = 8 };
+enum { MISC_L = 0, MISC_THIRDS = 1, MISC_NCAND = 2, MISC_KEPT = 3, MISC_Q4 = 4 /* 4 ints */ };
 
 template <int NB>
 struct Regs {
@@ -511,7 +511,13 @@ SXC_HD inline void forward_channel(Ex& ex, char* sm, const sxc_tables* tab, cons
     if (g >= G::GROUPS) return;
     const Regs<NB>& rg = ex.template reg<Regs<NB>>(g);
     float v[G::SA];
-    if (CACHED && !given && !tail.n) {
+    if constexpr (!CACHED) {
+      static_for<0, G::SA>([&](auto I) {
+        constexpr int r = decltype(I)::value;
+        const int p = stageA_pos<NB>(g, r);
+        v[r] = given ? given[p] : encode_at<NB>(sm, qs, p, ch, tail);
+      });
+    } else if (!given && !tail.n) {
       // Slot r of group g is position stageA_hi(r) + bitrev(g), its class in the cache, its window
       // weight one read at a constant offset, and odd slots lie past N/2, where most chunks have
       // ended.  Testing every position against the chunk's end, in both halves, and looking the
@@ -524,12 +530,10 @@ SXC_HD inline void forward_channel(Ex& ex, char* sm, const sxc_tables* tab, cons
       const double* diff = (const double*)(sm + SM::CODEC) + ch;
       auto slots = [&](auto HALF) {
         static_for<0, G::SA / 4>([&](auto W) {
-          uint32_t w = 0;
-          if constexpr (CACHED) w = fresh(rg.cls[decltype(W)::value]);
+          const uint32_t w = fresh(rg.cls[decltype(W)::value]);
           static_for<0, 2>([&](auto B) {
             constexpr int r = 4 * decltype(W)::value + 2 * decltype(B)::value + decltype(HALF)::value;
-            const int p = stageA_hi<NB>(r) + low;
-            const unsigned c = CACHED ? (w >> (8 * (r % 4))) & 255u : p < qs.L ? qs[p] : CLASS_PAST;
+            const unsigned c = (w >> (8 * (r % 4))) & 255u;
             const double e = (double)ent[stageA_hi<NB>(r) >> WSH];
             v[r] = (float)(e * diff[4 * c]);
           });
@@ -541,7 +545,7 @@ SXC_HD inline void forward_channel(Ex& ex, char* sm, const sxc_tables* tab, cons
       } else {
         static_for<0, G::SA / 2>([&](auto I) { v[2 * decltype(I)::value + 1] = 0.f; });
       }
-    } else if constexpr (CACHED) {
+    } else {
       static_for<0, G::SA / 4>([&](auto W) {
         const uint32_t w = fresh(rg.cls[decltype(W)::value]);
         static_for<0, 4>([&](auto B) {
@@ -549,12 +553,6 @@ SXC_HD inline void forward_channel(Ex& ex, char* sm, const sxc_tables* tab, cons
           const int p = stageA_pos<NB>(g, r);
           v[r] = given ? given[p] : encode_class<NB>(sm, qs.L, (w >> (8 * (r % 4))) & 255u, p, ch, tail);
         });
-      });
-    } else {
-      static_for<0, G::SA>([&](auto I) {
-        constexpr int r = decltype(I)::value;
-        const int p = stageA_pos<NB>(g, r);
-        v[r] = given ? given[p] : encode_at<NB>(sm, qs, p, ch, tail);
       });
     }
     stageA_forward<G::SA>(v, tw);

@@ -214,33 +214,6 @@ SXC_HD inline int code_score(const unsigned char* score, unsigned ca, unsigned c
 
 SXC_HD inline int code_class(unsigned c) { return c < 128 ? (int)c : SXC_CLASS_ZERO; }
 
-// GetMatchProbabilityEx on base codes; `ident` is also PrintMatch's identity (the same
-// DNA_Equal sum in the same order).
-SXC_HD inline double code_tail(const unsigned char* tc, const unsigned char* qc, const double* equal,
-                               const double* gcv, int start_t, int start_q, int len, double target_size,
-                               double& ident) {
-  double matches = 0, gct = 0, gcq = 0;
-  for (int i = 0; i < len; ++i) {
-    const int ca = code_class(tc[start_t + i]), cb = code_class(qc[start_q + i]);
-    matches += equal[ca * SXC_NCLASS + cb];
-    gct += gcv[ca];
-    gcq += gcv[cb];
-  }
-  ident = matches / (double)len;
-  const double gc_target = gct / (double)len;
-  // GCAdjustExpect, Sigma, CDF (analysis/AlignProbability.cc:11-40)
-  const double at_target = 1. - gc_target;
-  double r = gcq * gc_target;
-  r += ((double)len - gcq) * at_target;
-  const double p = r / (double)len / 2.;
-  const double s = sqrt(p * (1. - p) * (double)len);
-  const double m = p * (double)len;
-  const double x = (double)len * ident;
-  const double cdf = 0.5 * (1. + erf((m - x) / s / 1.414213562));
-  const double expect = cdf * target_size;
-  return exp(-expect);
-}
-
 // ---- bit-parallel window counts for pure A/C/G/T diagonals
 //
 // Bases are packed 2 bits each, 16 per 32-bit word.  32 bases of the target and of the

@@ -43,7 +43,7 @@ constexpr size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Byte offsets of the regions inside `scratch` for FFT length N, S strands.
 struct Layout {
-  size_t tseq, qseq, tch, qch, pair, which, ent, spectra, cands, ncand, counts, stats, offsets, total, maxc, nflag,
+  size_t tseq, qseq, tch, qch, pair, which, ent, spectra, cands, ncand, counts, offsets, total, maxc, nflag,
       slots, keys, final_, end;
   Layout(int N, int S) {
     size_t at = 0;
@@ -63,7 +63,6 @@ struct Layout {
     cands = take((size_t)S * N * sizeof(uint16_t));
     ncand = take((size_t)S * sizeof(int32_t));
     counts = take((size_t)S * sizeof(int32_t));
-    stats = take((size_t)2 * S * sizeof(int32_t));
     offsets = take((size_t)S * sizeof(int64_t));
     total = take(2 * sizeof(int64_t));
     maxc = take(sizeof(int32_t));
