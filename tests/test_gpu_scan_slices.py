@@ -222,3 +222,35 @@ def test_every_gate(ctx, target_total, letters):
     pairs = [ChunkPair(*(short_runs(500, letters, k) if k < 64 else related(900, 1000, letters, k, reverse=k % 2 == 1)),
                        t_record=k, q_record=k, q_record_len=500) for k in range(68)]
     assert len(check(ctx, pairs, 1024, target_total)) >= (3 if target_total > 1e8 else 40)
+
+
+@pytest.mark.parametrize("strands", [1, 2])
+@pytest.mark.parametrize("t_chunk", [0, 512])
+def test_mixed_kinds_by_strands_and_lengths(ctx, strands, t_chunk):
+    """The list of a mixed batch's strands, forward only too, and one list per length class (t_chunk 0)."""
+    from satsuma2_amd.api import ChunkPair, HomologyByXCorr, ResidentBatch, SlaveParams
+
+    kinds, pairs = ["acgt", "few", "n_gap", "dense", "acgt"], []
+    for k in range(90):
+        n = (500, 300, 900)[k % 3] if t_chunk == 0 else 512 - k % 9
+        t, q = related(n, n - k % 4, kinds[(k * k) % 5], 300 + k, reverse=k % 4 == 1)
+        pairs.append(ChunkPair(t, q, t_record=k, q_record=k, q_record_len=len(q)))
+    want = []
+    for p in pairs:
+        N = 2 * t_chunk or max(512, 1 << (len(p.tseq) + len(p.qseq) - 1).bit_length())
+        want += oracle.align_batch([dict(tseq=p.tseq, qseq=p.qseq, t_record=p.t_record, q_record=p.q_record,
+                                         q_record_len=p.q_record_len)],
+                                   oracle.make_params(N=N, strands=strands, q_chunk=512, target_total=1e6))
+    want = np.concatenate(want)
+    assert len(want) > 20
+    prm = SlaveParams(t_chunk=t_chunk, q_chunk=512, strands=strands, target_total=1e6)
+    b = ResidentBatch(ctx, pairs, prm)
+    got = [HomologyByXCorr(ctx, prm).align_batch(pairs)]
+    for _ in range(3):  # eager, captured, replayed
+        b.run()
+        got.append(b.results())
+    b.close()
+    for g in got:
+        assert len(g) == len(want)
+        for f in EXACT:
+            assert np.array_equal(g[f], want[f]), f
