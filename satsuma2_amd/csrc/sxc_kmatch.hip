@@ -298,11 +298,10 @@ int upload(const Side& side, unsigned char* d, std::vector<std::string>& stage, 
       continue;
     }
     const int64_t at = side.off[k];
-    std::string run;
-    for (; k < side.seq.size() && (int64_t)side.lengths[k] < kLong && (int64_t)run.size() < kStage; ++k) {
-      run.resize((size_t)(side.off[k] - at), 'N');
-      run.append(side.seq[k], (size_t)side.lengths[k]);
-    }
+    size_t e = k;
+    while (e < side.seq.size() && (int64_t)side.lengths[e] < kLong && side.off[e] - at < kStage) ++e;
+    std::string run((size_t)(side.off[e - 1] + (int64_t)side.lengths[e - 1] - at), 'N');
+    for (; k < e; ++k) memcpy(&run[(size_t)(side.off[k] - at)], side.seq[k], (size_t)side.lengths[k]);
     stage.push_back(std::move(run));
     KCHK(hipMemcpyAsync(d + at, stage.back().data(), stage.back().size(), hipMemcpyHostToDevice, s));
   }
