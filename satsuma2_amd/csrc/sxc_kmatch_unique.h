@@ -32,8 +32,10 @@ constexpr int64_t kStride = 10000000000LL;  // KMATCH_POSITION_CHR_CNST (KMatch.
 constexpr uint32_t kNone = 0xffffffffu;     // no entry of this k-mer on a side
 constexpr uint32_t kMulti = 0xfffffffeu;    // more than one
 constexpr uint32_t kNeg = 0x80000000u;      // the reverse complement was the smaller
-// A bijection of the 64-bit words (a product, its upper half folded into the lower): the low bits
-// spread the k-mers over the buckets, the top bits over a bucket's table.  (The radix sort is given
+// A bijection of the 64-bit words (a product, its upper half folded into the lower, twice): the low bits
+// spread the k-mers over the buckets, the top bits over a bucket's table.  (Once leaves bits 52 and up out
+// of the low 20: the first five bases of 31, whose 1024 variants before one 26-mer, as before the
+// homopolymer runs of two 200-Mbp genomes, then shared a bucket and filled its table.)  (The radix sort is given
 // low bits, as no call ends at bit 64: see sort_pairs.)
 constexpr uint64_t kMul = 0x9E3779B97F4A7C15ull;
 constexpr uint64_t inverse(uint64_t a) {
@@ -43,8 +45,9 @@ constexpr uint64_t inverse(uint64_t a) {
 }
 constexpr uint64_t kInv = inverse(kMul);
 static_assert(kMul * kInv == 1, "");
-__host__ __device__ constexpr uint64_t mix(uint64_t kmer) { return (kmer * kMul) ^ ((kmer * kMul) >> 32); }
-__host__ __device__ constexpr uint64_t unmix(uint64_t h) { return (h ^ (h >> 32)) * kInv; }
+__host__ __device__ constexpr uint64_t fold(uint64_t x) { return x ^ (x >> 32); }  // its own inverse
+__host__ __device__ constexpr uint64_t mix(uint64_t kmer) { return fold(fold(kmer * kMul) * kMul); }
+__host__ __device__ constexpr uint64_t unmix(uint64_t h) { return fold(fold(h) * kInv) * kInv; }
 static_assert(unmix(mix(0x123456789abcdefull)) == 0x123456789abcdefull, "");
 constexpr uint64_t kFree = mix(1ull << 63);  // the image of 2^63, which no k-mer is (K <= 31)
 

@@ -152,8 +152,11 @@ def one_bucket(n, bits, seed):
     rc = np.zeros_like(f)
     for i in range(31):
         rc = (rc << np.uint64(2)) | (np.uint64(3) - ((f >> np.uint64(2 * i)) & np.uint64(3)))
-    h = np.minimum(f, rc) * np.uint64(0x9E3779B97F4A7C15)
-    f = f[((h ^ (h >> np.uint64(32))) & np.uint64((1 << bits) - 1)) == 0][:n]
+    h = np.minimum(f, rc)
+    for _ in range(2):
+        h = h * np.uint64(0x9E3779B97F4A7C15)
+        h ^= h >> np.uint64(32)
+    f = f[(h & np.uint64((1 << bits) - 1)) == 0][:n]
     assert len(f) == n
     code = np.stack([(f >> np.uint64(2 * (30 - i))) & np.uint64(3) for i in range(31)], 1).astype(np.uint8)
     return [bytes(r) for r in np.frombuffer(b"ACGT", np.uint8)[code]]
@@ -187,5 +190,23 @@ def test_more_kmers_than_a_bucket_holds(ctx, name):
     q, t = genomes("records")
     got, st = kmatch(ctx, q, t, 21, 40, 20, 1)
     want, nq, nt, joined = expected(q, t, 21, 40, 20)
+    assert (st["query_kept"], st["target_kept"], st["joined"]) == (nq, nt, joined)
+    assert got.tobytes() == want.tobytes()
+
+
+@pytest.mark.parametrize("tail", [b"A" * 26, b"AC" * 13, b"AGTACCATTGACATTTAGCAGGCATA"])
+def test_kmers_that_differ_in_their_first_bases(ctx, tail):
+    """All 1024 k-mers of five bases before one 26-mer, as before homopolymer runs, with a few hundred others:
+    they spread over the buckets (the device path decides), from either strand."""
+    from satsuma2_amd.kmatch import kmatch
+
+    rng = np.random.default_rng(8)
+    heads = [bytes(b"ACGT"[(k >> (2 * i)) & 3] for i in range(5)) for k in range(1024)]
+    query = [h + tail for h in heads] + [rnd(rng, 31) for _ in range(200)]
+    target = [h + tail for h in heads[::3]] + query[1000:] + [rnd(rng, 31) for _ in range(100)]
+    target = [t.translate(COMP)[::-1] if k % 2 else t for k, t in enumerate(target)]
+    got, st = kmatch(ctx, query, target, 31, 31, 30, 1)
+    want, nq, nt, joined = expected(query, target, 31, 31, 30)
+    assert len(want) > 100 and st["sweep_ms"] == 0
     assert (st["query_kept"], st["target_kept"], st["joined"]) == (nq, nt, joined)
     assert got.tobytes() == want.tobytes()
