@@ -9,9 +9,9 @@
 // one array, two radix passes (three above 26 M entries) bring equal k-mers into the same bucket
 // of about 200 .. 400 entries, and one wave per bucket counts them in an LDS hash table.  Bound
 // by HBM: 12 bytes per position written once, and read and written once per radix pass.
-// Measured, host bytes in and records out: two 12-Mbp genomes, K = 21, 13.4 -> 2.3 ms (device
-// phase 6.3 -> 2.1 ms, most of it the upload; chaining 1.7 ms on the host before); two 1.2-Mbp
-// genomes 5.2 -> 0.6 ms.
+// Measured, host bytes in and records out, in a loop over the same genomes: two 12-Mbp genomes, K = 21,
+// 13.4 -> 2.3 ms (device phase 6.3 -> 2.1 ms, most of it the upload; chaining 1.7 ms on the host
+// before), with other genomes at each call 21 to 23 -> 3.1 ms; two 1.2-Mbp genomes 5.2 -> 0.6 ms.
 //
 // Chaining (dump_matching_blocks, kmatch/KMatch.cc:196-318).  A joined position extends the open
 // block on its diagonal if that block's end lies at most max_jump before it, and as positions
