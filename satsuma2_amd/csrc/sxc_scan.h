@@ -194,7 +194,8 @@ struct ScanSmem {
   static constexpr int BYTES = MISC + 64 + 4 * CE;
 };
 
-enum { SM_QN = 0, SM_KEPT = 1, SM_RUNS = 2, SM_NCAND = 3, SM_LT = 4, SM_LQ = 5, SM_NRB = 7, SM_AMB = 8, SM_NPOS = 16 };
+enum { SM_QN = 0, SM_KEPT = 1, SM_RUNS = 2, SM_NCAND = 3, SM_LT = 4, SM_LQ = 5, SM_NRB = 7, SM_AMB = 8, SM_BASES = 9 /* 4 ints */,
+       SM_NPOS = 16 };
 
 // Base code: class id (0..16) of a codec letter, or 128 | byte for a byte whose codec
 // row is zero.  Two bases are identical bytes iff their codes are equal.
@@ -996,12 +997,42 @@ SXC_HD inline void sum_digits(const uint32_t* x, const uint32_t* y, uint32_t* r)
   });
 }
 
-// General pairs are scanned in slices while at most one word (32 bases) in 8 of the two chunks holds
-// another letter, for whose windows every position is looked up twice.  ms for chunks of 4096 bases
-// with one such letter in every 2000 / 200 / 64 / 32 of the target, sliced and by segments: 200
-// strands 0.25 / 0.44 / 0.80 / 1.02 and 0.54 / 0.54 / 0.53 / 0.53, 4000 strands 1.39 / 2.96 / 5.11 /
-// 6.34 and 5.37 / 5.33 / 5.32 / 5.29; chunks of 16384, 200 strands, 64: 15.8 and 21.1.
-constexpr int SLICE_WORDS = 8;
+// The scan's gate: flags set that many times in a row name a block.
+SXC_HD inline int scan_gate(int min_run) { return min_run >= 8 ? 8 : min_run >= 4 ? 4 : min_run >= 2 ? 2 : 1; }
+
+// Whether slices pay for a general pair's `lags` (else segments).  What slices save on most blocks they
+// lose on the named ones, found again position by position, by table lookups where the windows hold
+// another letter.  How many are named follows from the gate and from how often a base of one chunk
+// equals one of the other (by their counts).  The limits are where both took the same time, fitted to
+// 1300 measured launches (0 to 6 such letters in 1000, G/C 0.2 to 0.5, N = 512 to 32768, 8 to 4000
+// strands); never with another letter in more than one word (32 bases) in 8.  ms sliced and by segments,
+// gates 1, 4 and 8, one such letter in the target / 2 / 6 in 1000:
+//   512 strands of 16384 bases, G/C 0.41 (equal 0.258): 15.6 7.4 4.8 and 34.8 32.6 32.1 / 24.8 14.5 9.9 and
+//   34.2 32.2 31.7 / 30.9 18.9 14.2 and 33.8 31.7 31.4; 0.35 (0.273): 26.5 11.2 7.0 and 36.9 33.3 32.6 / 42.1
+//   22.6 15.5 and 36.8 33.3 32.6 / 49.9 31.6 22.6 and 37.2 33.8 33.2; 0.25 (0.313): 64.7 33.2 22.3 and 47.8 40.0
+//   36.9 / 100.2 60.2 44.1 and 47.4 39.8 36.8 / 122 78.5 58.1 and 47.8 40.4 37.4;
+//   4000 strands of 2048 bases, whose segments are the fastest: 0.41: 1.19 0.81 0.68 and 1.64 1.45 1.43 / 1.52
+//   1.11 0.89 and 1.63 1.43 1.42; 0.35: 1.79 0.99 0.78 and 1.74 1.51 1.45; 0.25: 3.70 2.30 1.70 and 2.26 1.91 1.72.
+// A share of few blocks leaves most threads of a slice idle: 8 strands in 16 shares, G/C 0.41, gate 1, us:
+// 256 bases (about 80 blocks) 104 and 38, 512 (330) 133 and 68, 2048 (420) 179 and 119, 1024 (1300) 142 and 156,
+// 4096 (2300) 209 and 322.
+SXC_HD inline bool slices_pay(const int* misc, int log_n, int gate, int split, int lags) {
+  const float lt = (float)misc[SM_LT], lq = (float)misc[SM_LQ];
+  const float wt = (float)(misc[SM_AMB] & 0xffff), wq = (float)(misc[SM_AMB] >> 16);
+  if (8.f * 32.f * (wt + wq) > lt + lq) return false;
+  const int shorter = misc[SM_LT] < misc[SM_LQ] ? misc[SM_LT] : misc[SM_LQ];
+  if (split > 1 && lags * (shorter >> 5) < (log_n == 12 ? 1400 : 800)) return false;
+  float equal = 0.f;
+  for (int k = 0; k < 4; ++k) {
+    const unsigned t = (unsigned)misc[SM_BASES + k / 2], q = (unsigned)misc[SM_BASES + 2 + k / 2];
+    equal += (float)((k & 1) ? t >> 16 : t & 0xffffu) * (float)((k & 1) ? q >> 16 : q & 0xffffu);
+  }
+  // the share of blocks with another letter in their windows, which span three words
+  const float dirty = fminf(96.f * (wt / lt + wq / lq), 0.6f);
+  const float limit = gate == 8 ? 0.320f : gate == 4 ? 0.315f : gate == 2 ? 0.295f : 0.283f;
+  const float slope = (log_n <= 11 ? 0.01f : log_n == 12 ? 0.035f : 0.04f) * (gate >= 4 ? 1.8f : gate == 2 ? 1.3f : 1.f);
+  return equal <= (limit - slope * dirty - (log_n == 12 ? 0.018f : 0.f)) * lt * lq;
+}
 constexpr int SLICE_LAGS = 512;    // lags staged at a time
 constexpr int SLICE_BLOCKS = 29;   // blocks a slice decides (of the 32 it computes)
 
@@ -1273,7 +1304,7 @@ SXC_HD inline void scan_sliced(Ex& ex, char* sm, const ScanArgs& a, const sxc_pa
   const uint32_t* tam = (const uint32_t*)(sm + SS::TAM);
   const uint32_t* qam = (const uint32_t*)(sm + SS::QAM);
   const int Lt = misc[SM_LT], Lq = misc[SM_LQ];
-  const int gate = min_run >= 8 ? 8 : min_run >= 4 ? 4 : min_run >= 2 ? 2 : 1;
+  const int gate = scan_gate(min_run);
   const uint32_t d2 = gate >= 2 ? 0u : ~0u, d4 = gate >= 4 ? 0u : ~0u, d8 = gate >= 8 ? 0u : ~0u;
   ex.each([&](int tid) { runs[tid] = 0; });
   for (int c0 = lo; c0 < hi; c0 += SLICE_LAGS) {
@@ -1406,6 +1437,7 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
         score[i] = (&tab->score[0][0])[i];
       }
       for (int i = tid; i < SXC_NCLASS; i += SCAN_NT) gcv[i] = tab->gc[i];
+      if (tid < 5 * 32) ((int*)(sm + SS::RUNS))[tid] = 0;
       for (int i = tid; i < 128; i += SCAN_NT) {
         cls[i] = tab->cls[i];
         rc[i] = tab->rc[i];
@@ -1414,7 +1446,6 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
     if (tid == 0) {
       misc[SM_QN] = 0;
       misc[SM_NRB] = 0;
-      misc[SM_AMB] = 0;
       misc[SM_KEPT] = 0;
       misc[SM_RUNS] = 0;
       misc[SM_NCAND] = a.ncand[ps];
@@ -1520,21 +1551,40 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
       BasePlanes* qpl = (BasePlanes*)(sm + SS::QPL);
       uint32_t* tam = (uint32_t*)(sm + SS::TAM);
       uint32_t* qam = (uint32_t*)(sm + SS::QAM);
-      int n = 0;
+      // per thread, two 16-bit counts each: words with another letter of the target and the query; A, C
+      // and G, T of the target, of the query
+      int sum[5] = {0, 0, 0, 0, 0};
+      auto count = [&](const BasePlanes& b, uint32_t other, int left, int side) {
+        const uint32_t v = ~other & (left >= 32 ? ~0u : left > 0 ? (1u << left) - 1 : 0u);
+        sum[0] += (other != 0) << (16 * side);
+        sum[1 + 2 * side] += __builtin_popcount(v & ~b.lo & ~b.hi) + (__builtin_popcount(v & b.lo & ~b.hi) << 16);
+        sum[2 + 2 * side] += __builtin_popcount(v & ~b.lo & b.hi) + (__builtin_popcount(v & b.lo & b.hi) << 16);
+      };
       for (int w = tid; w < SS::PLW; w += SCAN_NT) {
         BasePlanes t = {0, 0}, q = {0, 0};
         uint32_t to = 0, qo = 0;
         if (w >= 2 && w < 2 + N / 32) {
           t = planes_of_codes(tc, Lt, w - 2, to);
           q = planes_of_codes(qc, Lq, w - 2, qo);
+          count(t, to, Lt - 32 * (w - 2), 0);
+          count(q, qo, Lq - 32 * (w - 2), 1);
         }
         tpl[w] = t;
         qpl[w] = q;
         tam[w] = to;
         qam[w] = qo;
-        n += (to != 0) + (qo != 0);
       }
-      if (n) ex.atomic_add_shared(&misc[SM_AMB], n);
+      // (32 places for each sum: with one, the additions are scans over the lanes, 15 us in all)
+      int* part = (int*)(sm + SS::RUNS);
+      for (int k = 0; k < 5; ++k) ex.atomic_add_shared(&part[32 * k + (tid & 31)], sum[k]);
+    });
+    ex.sync();
+    ex.each([&](int tid) {
+      if (tid >= 5) return;
+      const int* part = (const int*)(sm + SS::RUNS) + 32 * tid;
+      int n = 0;
+      for (int k = 0; k < 32; ++k) n += part[(k + tid) & 31];
+      misc[SM_AMB + tid] = n;
     });
     ex.sync();
   }
@@ -1548,7 +1598,7 @@ SXC_HD inline void scan_body(Ex& ex, char* sm, const ScanArgs& a, int blk) {
   // count, and the shared counter may already hold the next epoch's pushes of a faster wave.
   int queued = 0;
   bool sliced = SS::SLICED;
-  if constexpr (SS::AMB) sliced = 32 * SLICE_WORDS * misc[SM_AMB] <= Lt + Lq;
+  if constexpr (SS::AMB) sliced = slices_pay(misc, SS::LOG, scan_gate(min_run), split, hi - lo);
   if constexpr (SS::SLICED || SS::AMB)
     if (sliced) scan_sliced<NB>(ex, sm, a, pr, cands, ps, lo, hi, min_run);
   for (int e0 = sliced ? hi : lo; e0 < hi; e0 += CE) {

@@ -63,3 +63,18 @@ def short_runs(n: int, letters: str, seed: int):
         q[hit + shift] = t[hit]
         at += m + int(rng.integers(50, 70))
     return other_letters(t.tobytes(), letters, rng), bytes(q.tobytes())
+
+
+def composed(lt: int, lq: int, gc: float, other: float, seed: int):
+    """(target, query) of a G/C content, related, with that share of other letters in both: pairs on either
+    side of the limits up to which slices pay."""
+    rng = np.random.default_rng(seed)
+    p = [(1 - gc) / 2, gc / 2, gc / 2, (1 - gc) / 2]
+    t, q = (rng.choice(list(b"ACGT"), n, p=p).astype(np.uint8) for n in (lt, lq))
+    n = min(lt, lq) // 2
+    q[lq - n:] = np.where(rng.random(n) < 0.15, q[lq - n:], t[:n])
+    for s in (t, q):
+        at = rng.random(len(s)) < other
+        at[len(s) // 3] = True
+        s[at] = rng.choice(list(b"RYKMSW"), int(at.sum()))
+    return t.tobytes(), q.tobytes()

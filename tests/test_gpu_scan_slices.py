@@ -9,7 +9,7 @@ import pytest
 
 import oracle
 from conftest import dense_run_pair
-from scan_cases import GATES, LENGTHS, LETTERS, related, short_runs
+from scan_cases import GATES, LENGTHS, LETTERS, composed, related, short_runs
 
 pytestmark = pytest.mark.gpu
 
@@ -254,3 +254,17 @@ def test_mixed_kinds_by_strands_and_lengths(ctx, strands, t_chunk):
         assert len(g) == len(want)
         for f in EXACT:
             assert np.array_equal(g[f], want[f]), f
+
+
+@pytest.mark.parametrize("target_total", [1e3, 1e6, 1e9])
+@pytest.mark.parametrize("t_chunk,n", [(256, 3), (256, 600), (1024, 3), (1024, 60), (2048, 30), (4096, 3), (4096, 40), (16384, 3)])
+def test_slices_or_segments(ctx, t_chunk, n, target_total):
+    """General pairs on both sides of slices_pay's limits, in launches of few shares and many."""
+    from satsuma2_amd.api import ChunkPair
+
+    pairs = []
+    for k in range(n):
+        gc, other = ((0.15, 0.0), (0.41, 0.0), (0.41, 0.004), (0.3, 0.002), (0.5, 0.02))[k % 5]
+        t, q = composed(t_chunk - k % 4, t_chunk - k % 6, gc, other, 700 + k)
+        pairs.append(ChunkPair(t, q, t_record=k, q_record=k, q_record_len=len(q)))
+    assert len(check(ctx, pairs, t_chunk, target_total)) > 0

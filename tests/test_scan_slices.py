@@ -10,7 +10,7 @@ import pytest
 import hostbuild
 import oracle
 from conftest import dense_run_pair
-from scan_cases import GATES, LENGTHS, LETTERS, related, short_runs
+from scan_cases import GATES, LENGTHS, LETTERS, composed, related, short_runs
 from test_emu import COLS, emu_batch
 
 
@@ -72,3 +72,17 @@ def test_every_gate(emu, target_total, pure, general, letters):
         t, q = short_runs(500, letters, k) if k < 32 else related(900, 1000, letters, k, reverse=k == 33)
         pairs.append(dict(tseq=t, qseq=q, t_record=k, q_record=k))
     assert len(check(emu, pairs, 2048, target_total)) >= (3 if target_total > 1e8 else 25)
+
+
+@pytest.mark.parametrize("split", ["", "16"])
+@pytest.mark.parametrize("target_total", [1e3, 1e5, 1e6, 1e9])
+def test_slices_or_segments(emu, monkeypatch, target_total, split):
+    """General pairs on both sides of slices_pay's limits: composition, other letters, gate, share of lags.
+    Each pair alone and in one batch."""
+    if split:
+        monkeypatch.setenv("SXC_EMU_SPLIT", split)
+    pairs = []
+    for k, (gc, other) in enumerate((g, o) for g in (0.1, 0.25, 0.35, 0.41, 0.5) for o in (0.0, 0.002, 0.005)):
+        t, q = composed(1000 - 7 * k, 1024 - 31 * k, gc, other, 90 + k)
+        pairs.append(dict(tseq=t, qseq=q, t_record=k, q_record=k))
+    assert len(check(emu, pairs, 2048, target_total)) > 0
