@@ -286,10 +286,13 @@ hipError_t sort_pairs(void* tmp, size_t& bytes, uint64_t* k0, uint64_t* k1, V* v
 }
 
 // A genome's buffer into device memory at d.  Long sequences are copied from where they lie,
-// runs of short ones through `stage` (which has to live until the stream is synchronised).
+// runs of short ones, each with the 'N' before it, through `stage` (which has to live until the stream is
+// synchronised).
 int upload(const Side& side, unsigned char* d, std::vector<std::string>& stage, hipStream_t s) {
   constexpr int64_t kLong = 65536, kStage = 1 << 22;
-  KCHK(hipMemsetAsync(d, 'N', (size_t)side.len, s));
+  bool any_long = false;
+  for (uint64_t n : side.lengths) any_long |= (int64_t)n >= kLong;
+  if (any_long) KCHK(hipMemsetAsync(d, 'N', (size_t)side.len, s));
   for (size_t k = 0; k < side.seq.size();) {
     const int64_t n = (int64_t)side.lengths[k];
     if (n >= kLong) {
@@ -297,7 +300,7 @@ int upload(const Side& side, unsigned char* d, std::vector<std::string>& stage, 
       ++k;
       continue;
     }
-    const int64_t at = side.off[k];
+    const int64_t at = side.off[k] - 1;
     size_t e = k;
     while (e < side.seq.size() && (int64_t)side.lengths[e] < kLong && side.off[e] - at < kStage) ++e;
     std::string run((size_t)(side.off[e - 1] + (int64_t)side.lengths[e - 1] - at), 'N');

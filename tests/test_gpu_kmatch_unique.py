@@ -145,6 +145,27 @@ def test_look_back_limit(ctx):
             assert got.tobytes() == expected(query, target, 11, 11, jump)[0].tobytes(), (gap, jump)
 
 
+@pytest.mark.parametrize("jump", [20, 65])
+@pytest.mark.parametrize("order", ["sls", "lsl", "ssl", "lss", "l", "s"])
+def test_long_and_short_records(ctx, order, jump):
+    """Neighbours cut from one sequence: a letter missing between two records gives k-mers across the cut."""
+    from satsuma2_amd.kmatch import kmatch
+
+    rng = np.random.default_rng(11)
+    g = rnd(rng, 140000)
+    query, at = [], 0
+    for c in order:
+        for n in (65536 + 3 * at % 7,) if c == "l" else (40, 31, 700):
+            query.append(g[at:at + n])
+            at += n
+    target = [g[max(0, at - 900):at - 300], g[at - 300:at]] + query[::-1]
+    for q, t in ((query, target), (query, [g[:at]])):
+        got, st = kmatch(ctx, q, t, 15, 15, jump, 1)
+        want, nq, nt, joined = expected(q, t, 15, 15, jump)
+        assert (st["query_kept"], st["target_kept"], st["joined"]) == (nq, nt, joined)
+        assert got.tobytes() == want.tobytes()
+
+
 def one_bucket(n, bits, seed):
     """n records of 31 bases whose k-mers fall into bucket 0 of 2^bits (sxc_kmatch_unique.h: mix)."""
     rng = np.random.default_rng(seed)
